@@ -157,7 +157,8 @@ __host__ __device__ inline uint32_t brick_at(const BrickParams& bp, uint32_t d) 
 // contiguous run of dispatch positions, in pencil order (PENCIL) or in brick index order;
 // >= nbricks for the few padding workgroups.  Pencils cut the mixed force kernel's HBM reads
 // from 2.63 to 2.40 GB per C2 launch and the build's from 0.71 to 0.47 GB; the FP64 force
-// kernel (one workgroup per CU) measured 3 % slower with them, so it keeps index order.
+// kernel, bound by its arithmetic, measured 1-2 % slower with them (2,048,000 atoms 340 -> 347
+// us, 8,388,608 1388 -> 1400 us), so it keeps index order.
 template <bool PENCIL>
 __device__ inline uint32_t brick_of_block(const BrickParams& bp) {
   const uint32_t d = (blockIdx.x % kXcds) * bp.per_xcd + blockIdx.x / kXcds;
@@ -792,6 +793,8 @@ __device__ __forceinline__ void compute_pair_brick_body(const Geom& g, const Bri
   using Tr = ComputePairTraits<F>;
   static_assert(Tr::Batched || Tr::BufferLessCompatible, "the traversal calls the batched or the buffer-less form");
   static_assert(!(EPI == EPI_NEXT && ACCUM), "a fused step starts the force from 0");
+  constexpr bool CHECKED = PairChecked<Tr>::value;
+  static_assert(!CHECKED || (Tr::Batched && Tr::ComputeBufferCompatible), "a second walk starts again from zero sums");
   constexpr bool BUFFERED = Tr::ComputeBufferCompatible;
   constexpr bool ENERGY = Tr::CentralEnergy && EPI != EPI_NEXT;
   extern __shared__ __align__(16) char lds[];
@@ -832,35 +835,50 @@ __device__ __forceinline__ void compute_pair_brick_body(const Geom& g, const Bri
     if (Tr::CentralEnergy) te = A.ep[At.slot];
   }
   const int type_a = Tr::CentralType ? (int)L.pt[At.ia] : 0;
-  for (uint32_t q0 = 0; q0 < nmax; q0 += U) {
-    uint2 wc[W];
+  // walks the lane's list from the batch in wn, calling pairs(batch) on every batch of U entries
+  auto walk = [&](auto&& pairs) {
+    for (uint32_t q0 = 0; q0 < nmax; q0 += U) {
+      uint2 wc[W];
 #pragma unroll
-    for (int w = 0; w < W; w++) wc[w] = wn[w];
-    if (q0 + U < nmax) {
-      const uint2* nxt = lst + (size_t)((q0 + U) >> 2) * T;
+      for (int w = 0; w < W; w++) wc[w] = wn[w];
+      if (q0 + U < nmax) {
+        const uint2* nxt = lst + (size_t)((q0 + U) >> 2) * T;
 #pragma unroll
-      for (int w = 0; w < W; w++) wn[w] = load_list_group(nxt + (size_t)w * T);
+        for (int w = 0; w < W; w++) wn[w] = load_list_group(nxt + (size_t)w * T);
+      }
+      NbhBatch<U> nb;
+      nb.pos = L.px;
+      nb.type = L.pt;
+#pragma unroll
+      for (int w = 0; w < W; w++) {
+        nb.j[4 * w + 0] = wc[w].x & 0xffffu;
+        nb.j[4 * w + 1] = wc[w].x >> 16;
+        nb.j[4 * w + 2] = wc[w].y & 0xffffu;
+        nb.j[4 * w + 3] = wc[w].y >> 16;
+        // 24-bit multiplies of the 16-bit halves (one instruction each with a word select)
+        nb.off[4 * w + 0] = __umul24(wc[w].x & 0xffffu, 24u);
+        nb.off[4 * w + 1] = __umul24(wc[w].x >> 16, 24u);
+        nb.off[4 * w + 2] = __umul24(wc[w].y & 0xffffu, 24u);
+        nb.off[4 * w + 3] = __umul24(wc[w].y >> 16, 24u);
+      }
+      // entries past a lane's count are the sentinel (rejected by the cutoff)
+      pairs(nb);
     }
-    NbhBatch<U> nb;
-    nb.pos = L.px;
-    nb.type = L.pt;
+  };
+  if constexpr (CHECKED) {
+    PairRange rng;
+    walk([&](const NbhBatch<U>& nb) { func.template batch_checked<U, ENERGY>(ra, nb, rng, tx, ty, tz, te); });
+    if (__builtin_expect(__any(func.unchecked_parameters() || rng.outside()), 0)) {
+      tx = ty = tz = te = 0.0;
 #pragma unroll
-    for (int w = 0; w < W; w++) {
-      nb.j[4 * w + 0] = wc[w].x & 0xffffu;
-      nb.j[4 * w + 1] = wc[w].x >> 16;
-      nb.j[4 * w + 2] = wc[w].y & 0xffffu;
-      nb.j[4 * w + 3] = wc[w].y >> 16;
-      // 24-bit multiplies of the 16-bit halves (one instruction each with a word select)
-      nb.off[4 * w + 0] = __umul24(wc[w].x & 0xffffu, 24u);
-      nb.off[4 * w + 1] = __umul24(wc[w].x >> 16, 24u);
-      nb.off[4 * w + 2] = __umul24(wc[w].y & 0xffffu, 24u);
-      nb.off[4 * w + 3] = __umul24(wc[w].y >> 16, 24u);
+      for (int w = 0; w < W; w++) wn[w] = t < T ? load_list_group(lst + (size_t)w * T) : make_uint2(0u, 0u);
+      walk([&](const NbhBatch<U>& nb) { func.template batch<U, ENERGY>(ra, nb, tx, ty, tz, te); });
     }
-    // entries past a lane's count are the sentinel (rejected by the cutoff)
-    if constexpr (Tr::Batched) {
-      func.template batch<U, ENERGY>(ra, nb, tx, ty, tz, te);
-    } else {
-      const NbhCells cells{L.pt, nullptr};
+  } else if constexpr (Tr::Batched) {
+    walk([&](const NbhBatch<U>& nb) { func.template batch<U, ENERGY>(ra, nb, tx, ty, tz, te); });
+  } else {
+    const NbhCells cells{L.pt, nullptr};
+    walk([&](const NbhBatch<U>& nb) {
 #pragma unroll
       for (int u = 0; u < U; u++) {
         const double4 rb = nb(u);
@@ -877,7 +895,7 @@ __device__ __forceinline__ void compute_pair_brick_body(const Geom& g, const Bri
             func(dr, d2, tx, ty, tz, cells, 0, nb.j[u], 1.0);
         }
       }
-    }
+    });
   }
   constexpr bool NEXT = EPI == EPI_NEXT;
   bool over = false;
@@ -932,10 +950,7 @@ __device__ __forceinline__ void compute_pair_brick_body(const Geom& g, const Bri
 }
 
 template <bool MIXED, bool ACCUM, int EPI, int U>
-// waves_per_eu(5) caps registers at 96: measured faster for the FP64 instantiations, neutral
-// for the mixed ones.  The FP64 form's spills (44-52 bytes) all sit in the pair loop's
-// small-argument branch (d2 < 2^-767, the generic root and division), not in its hot path.
-__global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(5))) k_lj_brick(Geom g, BrickParams bp, const double4* __restrict__ r,
+__global__ void __launch_bounds__(1024) k_lj_brick(Geom g, BrickParams bp, const double4* __restrict__ r,
                                                    const uint32_t* __restrict__ cell_off, const uint32_t* __restrict__ cell_n,
                                                    const uint16_t* __restrict__ blist, const uint32_t* __restrict__ bcnt,
                                                    LJConst lj, PState A, double dth, NextStep nx) {
@@ -1449,11 +1464,9 @@ __device__ __forceinline__ void lj_batch_case(const BoxFrame& f, uint32_t b, uin
 // Force of every brick of the listed boxes, all of one precision (one kernel per precision,
 // so the mixed form runs with its own, smaller register budget); the epilogue is per box
 // (uniform per workgroup).  EPI_KICK closes a box's run; EPI_NEXT fuses its next step;
-// EPI_NONE stores the force and energy only.  The
-// register cap of 5 waves per SIMD (the FP64 form otherwise takes 110 VGPRs, 4 waves) measured
-// 3% faster on 256 FP64 boxes; the mixed form fits under it anyway.
+// EPI_NONE stores the force and energy only.
 template <bool MIXED>
-__global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(5))) kb_lj_brick(const BoxFrame* __restrict__ F, const uint32_t* __restrict__ work,
+__global__ void __launch_bounds__(1024) kb_lj_brick(const BoxFrame* __restrict__ F, const uint32_t* __restrict__ work,
                                                     const uint32_t* __restrict__ clock) {
   uint32_t box, b;
   if (!batch_brick(work, box, b)) return;  // whole workgroup

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <cmath>
+
 #include "../../include/xnb_compute_pair.h"
 
 namespace xnb {
@@ -18,6 +20,7 @@ namespace xnb {
 struct LJConst {
   double sigma, eps4, m24eps, rc2;
   float sigma6f, eps4f, m24epsf;  // sigma^6, 4 eps, -24 eps for the mixed form
+  uint32_t any;                   // parameters lj_batch_fp64 does not cover: the generic operations
 };
 
 // FP32 part of the mixed form from x = 1/r^2 (0 outside the cutoff): s6 = sigma^6 x^3, the
@@ -28,22 +31,6 @@ __device__ inline float lj_coef_f32(float x, float sigma6, float m24eps, float& 
   return (s6 * x) * fmaf(s6, 2.0f * m24eps, -m24eps);
 }
 __device__ inline float lj_energy_f32(float s6, float eps4) { return eps4 * fmaf(s6, s6, -s6); }
-
-template <bool ACCUM>
-__device__ inline void store_force(uint32_t s, double tx, double ty, double tz, double te, double* __restrict__ fx,
-                                   double* __restrict__ fy, double* __restrict__ fz, double* __restrict__ ep) {
-  if (ACCUM) {
-    fx[s] += tx;
-    fy[s] += ty;
-    fz[s] += tz;
-    ep[s] += te;
-  } else {
-    fx[s] = 0.0 + tx;
-    fy[s] = 0.0 + ty;
-    fz[s] = 0.0 + tz;
-    ep[s] = 0.0 + te;
-  }
-}
 
 // Wave-wide maximum (every lane of the wave must be active), returned as a wave-uniform (scalar) value so loops bounded by it stay
 // scalar branches
@@ -86,40 +73,44 @@ __device__ inline double recip_normal(double y) {
   return fma(rem, a, a);
 }
 
-// 1 / sqrt(x) as two correctly rounded steps, r = sqrt(x) then 1.0 / r; the normal-range
-// sequences unless some lane of the wave has x below their range (never for physical pair
-// distances), in which case the whole wave takes the library operations.
-__device__ inline double inv_sqrt_rounded(double x) {
-  if (__builtin_expect(__any(x < 0x1p-767), 0)) return 1.0 / sqrt(x);
-  return recip_normal(sqrt_normal(x));
+// RN(1 / RN(sqrt(x))) for x in [2^-767, 2^1000].  The root is sqrt_normal's; its iteration
+// leaves h = 0.5 / sqrt(x) to about 2^-45, so the reciprocal starts from 2 h instead of a
+// v_rcp_f64 estimate: one Newton-Raphson step brings it within 1 ulp of 1 / r and the last
+// fma-corrected step rounds it correctly (Markstein, as above) for every r but one whose
+// significand is all ones.  Those roots come from the two largest significands below a power
+// of 4 only; PairRange sends every x whose low word is 0xfffffffe or 0xffffffff (2 in 2^32) to
+// the generic operations.
+__device__ inline double inv_sqrt_normal(double x) {
+  const double g = __builtin_amdgcn_rsq(x);
+  double s = x * g;
+  double h = g * 0.5;
+  const double r = fma(-h, s, 0.5);
+  s = fma(s, r, s);
+  h = fma(h, r, h);
+  double d = fma(-s, s, x);
+  s = fma(d, h, s);
+  d = fma(-s, s, x);
+  s = fma(d, h, s);
+  double a = h + h;
+  double e = fma(-s, a, 1.0);
+  a = fma(e, a, a);
+  e = fma(-s, a, 1.0);
+  return fma(e, a, a);
 }
 
-// One pair of the plain FP64 form.  Pairs outside 0 < d2 <= rc^2 contribute through a
-// select of 0.0: adding +-0 leaves the running sums bitwise unchanged (they start at +0.0 and
-// round-to-nearest never produces -0 from a sum with a +0 operand), so the result equals the
-// reference's branch.
-template <bool ENERGY = true>
-__device__ inline void lj_pair_fp64(const LJConst& lj, const double4& ra, const double4& rb, double& tx, double& ty, double& tz,
-                                    double& te) {
-  const double dx = rb.x - ra.x;
-  const double dy = rb.y - ra.y;
-  const double dz = rb.z - ra.z;
-  const double d2 = (dx * dx + dy * dy) + dz * dz;
-  const bool in = d2 > 0.0 && d2 <= lj.rc2;
-  const double inv_r = inv_sqrt_rounded(in ? d2 : 1.0);  // 1.0 / sqrt(d2), each correctly rounded
-  const double ratio = lj.sigma * inv_r;
-  const double ratio2 = ratio * ratio;
-  const double ratio6 = ratio2 * ratio2 * ratio2;
-  const double ratio12 = ratio6 * ratio6;
-  const double e = lj.eps4 * (ratio12 - ratio6);
-  double de = (lj.m24eps * (2. * ratio12 - ratio6)) * inv_r;
-  de *= inv_r;  // interaction_weight / r with weight 1.0: the same correctly rounded 1.0/r
-  de = in ? de : 0.0;
-  tx += de * dx;
-  ty += de * dy;
-  tz += de * dz;
-  if (ENERGY) te += in ? e : 0.0;
-}
+// What a lane's d2 values have shown of inv_sqrt_normal's range: the smallest high word (0 for
+// coincident atoms) and the largest low word.  Kept per list, half an instruction a pair for
+// each (v_min3_u32 / v_max3_u32), and looked at once after it, so the pair loop has no branch.
+struct PairRange {
+  uint32_t hi = 0xffffffffu, lo = 0u;
+  __device__ inline void add(double d2) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(d2);
+    hi = min(hi, (uint32_t)(b >> 32));
+    lo = max(lo, (uint32_t)b);
+  }
+  // some d2 below 2^-767, or a low word next to all ones
+  __device__ inline bool outside() const { return hi < 0x10000000u || lo >= 0xfffffffeu; }
+};
 
 // One pair of the mixed form: FP64 displacement and cutoff test, FP32 coefficient
 // de/r = -24 eps (2 s^12 - s^6) / r^2 (lj_coef_f32) from (float)d2 with a hardware
@@ -176,32 +167,29 @@ inline int make_lj_multi(int ntypes, const double* eps, const double* sigma, con
   return 0;
 }
 
-// U pairs of the plain FP64 form at once, summed in u order (the same sums as U calls of
-// lj_pair_fp64): the distance tests first, one wave-uniform range decision for all U roots, then
-// the U independent root / reciprocal chains back to back, which the compiler interleaves.
+// U pairs of the plain FP64 form, summed in u order, for parameters without LJConst::any and
+// d2 within rng.  A pair outside the cutoff takes 2^1000 for the high
+// word of d2: its sixth power of sigma / r underflows to 0, so it adds +-0 to every sum, which
+// leaves them bitwise unchanged (they start at +0.0 and round-to-nearest never produces -0 from
+// a sum with a +0 operand), as the reference's branch does; one select instead of the two of a
+// selected coefficient, and no second test (d2 == 0 shows in rng).  2 s^12 - s^6 is one fma:
+// doubling is exact.  The pair is bound by issuing its VALU instructions: with these, the root
+// chain above and the single range look per list it is about 42 instead of 52 of them, and the
+// kernel takes 56 instead of 96 registers, so two workgroups share a CU (2,048,000 atoms:
+// force launch 404 -> 339 us; 131,072: 41.9 -> 36.7).
 template <int U, bool ENERGY = true>
-__device__ inline void lj_batch_fp64(const LJConst& lj, const double4& ra, const double4 (&rb)[U], double& tx, double& ty,
-                                     double& tz, double& te) {
-  double dx[U], dy[U], dz[U], x[U];
-  bool in[U];
-  bool small = false;
+__device__ inline void lj_batch_fp64(const LJConst& lj, const double4& ra, const double4 (&rb)[U], PairRange& rng, double& tx,
+                                     double& ty, double& tz, double& te) {
+  double dx[U], dy[U], dz[U], inv_r[U];
 #pragma unroll
   for (int u = 0; u < U; u++) {
     dx[u] = rb[u].x - ra.x;
     dy[u] = rb[u].y - ra.y;
     dz[u] = rb[u].z - ra.z;
     const double d2 = (dx[u] * dx[u] + dy[u] * dy[u]) + dz[u] * dz[u];
-    in[u] = d2 > 0.0 && d2 <= lj.rc2;
-    x[u] = in[u] ? d2 : 1.0;
-    small = small || x[u] < 0x1p-767;
-  }
-  double inv_r[U];
-  if (__builtin_expect(__any(small), 0)) {
-#pragma unroll
-    for (int u = 0; u < U; u++) inv_r[u] = 1.0 / sqrt(x[u]);
-  } else {
-#pragma unroll
-    for (int u = 0; u < U; u++) inv_r[u] = recip_normal(sqrt_normal(x[u]));
+    rng.add(d2);
+    const uint32_t hi = d2 <= lj.rc2 ? (uint32_t)__double2hiint(d2) : 0x7e700000u;
+    inv_r[u] = inv_sqrt_normal(__hiloint2double((int)hi, __double2loint(d2)));
   }
 #pragma unroll
   for (int u = 0; u < U; u++) {
@@ -209,17 +197,36 @@ __device__ inline void lj_batch_fp64(const LJConst& lj, const double4& ra, const
     const double ratio2 = ratio * ratio;
     const double ratio6 = ratio2 * ratio2 * ratio2;
     const double ratio12 = ratio6 * ratio6;
-    double de = (lj.m24eps * (2. * ratio12 - ratio6)) * inv_r[u];
-    de *= inv_r[u];
-    de = in[u] ? de : 0.0;
+    double de = (lj.m24eps * fma(2., ratio12, -ratio6)) * inv_r[u];
+    de *= inv_r[u];  // interaction_weight / r with weight 1.0: the same correctly rounded 1.0/r
     tx += de * dx[u];
     ty += de * dy[u];
     tz += de * dz[u];
-    if (ENERGY) {
-      const double e = lj.eps4 * (ratio12 - ratio6);
-      te += in[u] ? e : 0.0;
-    }
+    if (ENERGY) te += lj.eps4 * (ratio12 - ratio6);
   }
+}
+
+// One pair of the plain FP64 form with the generic operations: any d2, any parameters.
+template <bool ENERGY>
+__device__ inline void lj_pair_fp64_any(const LJConst& lj, const double4& ra, const double4& rb, double& tx, double& ty, double& tz,
+                                        double& te) {
+  const double dx = rb.x - ra.x;
+  const double dy = rb.y - ra.y;
+  const double dz = rb.z - ra.z;
+  const double d2 = (dx * dx + dy * dy) + dz * dz;
+  const bool in = d2 > 0.0 && d2 <= lj.rc2;
+  const double inv_r = 1.0 / sqrt(in ? d2 : 1.0);
+  const double ratio = lj.sigma * inv_r;
+  const double ratio2 = ratio * ratio;
+  const double ratio6 = ratio2 * ratio2 * ratio2;
+  const double ratio12 = ratio6 * ratio6;
+  double de = (lj.m24eps * (2. * ratio12 - ratio6)) * inv_r;
+  de *= inv_r;
+  de = in ? de : 0.0;
+  tx += de * dx;
+  ty += de * dy;
+  tz += de * dz;
+  if (ENERGY) te += in ? lj.eps4 * (ratio12 - ratio6) : 0.0;
 }
 
 // ------------------------------------------------------------------ force functors
@@ -227,9 +234,15 @@ __device__ inline void lj_batch_fp64(const LJConst& lj, const double4& ra, const
 // form (lennard_jones.cu:105-124, plus the per-atom energy field) and the batched form the
 // brick traversal uses.  MIXED selects the mixed form (FP32 pair coefficient, FP64
 // displacement, cutoff test and accumulation).
+// FP64 pairs evaluated together: 1, 2 and 4 measured the same at 2,048,000 atoms (338.9, 338.6
+// and 341.8 us a launch) with 53, 56 and 68 registers
+static constexpr int kLjGroup = 2;
 template <bool MIXED>
 struct LennardJonesForceFunctor {
   LJConst p;
+
+  // batch_checked does not cover these parameters
+  __device__ inline bool unchecked_parameters() const { return p.any != 0u; }
 
   __device__ inline void operator()(Vec3d dr, double d2, double& fx, double& fy, double& fz, double& ep, const NbhCells&, size_t,
                                     size_t, double w) const {
@@ -259,9 +272,7 @@ struct LennardJonesForceFunctor {
   }
 
   // U list entries in list order (sentinel padding included); pairs outside 0 < d2 <= rc^2
-  // add +-0.  FP64: pairs by two, each pair's positions read just before its arithmetic and
-  // the scheduler kept from hoisting the next pair's reads (with the force kernel's register
-  // cap: 8.4M-atom FP64 force 1.91 -> 1.78 ms against eight pairs read up front).
+  // add +-0.  FP64: any distances and parameters, with the generic operations.
   template <int U, bool ENERGY>
   __device__ __forceinline__ void batch(const double4& ra, const NbhBatch<U>& nb, double& fx, double& fy, double& fz,
                                         double& ep) const {
@@ -273,13 +284,23 @@ struct LennardJonesForceFunctor {
       for (int u = 0; u < U; u++) lj_pair_mixed<ENERGY>(p, ra, rb[u], fx, fy, fz, ep);
     } else {
 #pragma unroll
-      for (int h = 0; h < U; h += 2) {
-        double4 rb[2];
+      for (int u = 0; u < U; u++) lj_pair_fp64_any<ENERGY>(p, ra, nb(u), fx, fy, fz, ep);
+    }
+  }
+
+  // The same for parameters without LJConst::any, valid if rng stays inside: pairs by kLjGroup,
+  // each group's positions read just before its arithmetic and the scheduler kept from
+  // hoisting the next group's reads, which bounds the registers.
+  template <int U, bool ENERGY>
+  __device__ __forceinline__ void batch_checked(const double4& ra, const NbhBatch<U>& nb, PairRange& rng, double& fx, double& fy,
+                                                double& fz, double& ep) const {
 #pragma unroll
-        for (int u = 0; u < 2; u++) rb[u] = nb(h + u);
-        lj_batch_fp64<2, ENERGY>(p, ra, rb, fx, fy, fz, ep);
-        __builtin_amdgcn_sched_barrier(0);
-      }
+    for (int h = 0; h < U; h += kLjGroup) {
+      double4 rb[kLjGroup];
+#pragma unroll
+      for (int u = 0; u < kLjGroup; u++) rb[u] = nb(h + u);
+      lj_batch_fp64<kLjGroup, ENERGY>(p, ra, rb, rng, fx, fy, fz, ep);
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
 };
@@ -291,6 +312,7 @@ struct ComputePairTraits<LennardJonesForceFunctor<MIXED>> {
   static constexpr bool CentralType = false;
   static constexpr bool CentralEnergy = true;
   static constexpr bool Batched = true;
+  static constexpr bool Checked = !MIXED;
 };
 
 // GravitationalForceFunctor (contribs/pi/gravitational_force.cu:44-82): Newtonian attraction
@@ -335,6 +357,8 @@ inline LJConst make_lj_const(double eps, double sigma, double rcut) {
   c.sigma6f = (float)(sigma * sigma * sigma * sigma * sigma * sigma);
   c.eps4f = (float)(4. * eps);
   c.m24epsf = (float)(-24. * eps);
+  // finite energies, and sigma * 2^-500 far below the fourth root of the smallest double
+  c.any = std::isfinite(c.eps4) && std::isfinite(c.m24eps) && std::fabs(sigma) <= 0x1p100 ? 0u : 1u;
   return c;
 }
 

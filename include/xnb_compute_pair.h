@@ -33,7 +33,14 @@
  * from the staged region, when the functor chooses), makes the cutoff test itself and adds
  * +-0 for a rejected pair (the list padding is a far-away sentinel atom); ENERGY false means
  * the energy is not wanted.  The traversal then calls it once per batch of U entries instead
- * of the per-pair form, so a functor can interleave the long-latency parts of U pairs.
+ * of the per-pair form, so a functor can interleave the long-latency parts of U pairs.  If its
+ * traits also set Checked (which need not be there), the traversal calls
+ *
+ *   batch_checked(ra, nb, rng, fx, fy, fz, ep)   (the template arguments of batch)
+ *
+ * instead, which may assume distances inside PairRange: it notes every d2 in rng (rng.add), and
+ * a wave whose lists held one outside, or any wave when unchecked_parameters() is true, is
+ * walked again from zero sums with batch.
  *
  * The traversals are instantiated inside the library: compute_pair_brick_body (brick lists,
  * exanbody_amd/csrc/xnb_brick.hip) and k_compute_pair_slots (per-slot lists, all cells,
@@ -63,6 +70,16 @@ struct ComputePairTraits {
   static constexpr bool CentralType = false;
   static constexpr bool CentralEnergy = false;
   static constexpr bool Batched = false;
+};
+
+/* ComputePairTraits<F>::Checked, false for traits without it */
+template <class T, class = void>
+struct PairChecked {
+  static constexpr bool value = false;
+};
+template <class T>
+struct PairChecked<T, decltype(void(T::Checked))> {
+  static constexpr bool value = T::Checked;
 };
 
 namespace field {
