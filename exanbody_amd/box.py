@@ -115,8 +115,8 @@ class Box:
     def export(self, ghosts=False):
         n_in, n_g = self.num_particles()
         n = n_in + (n_g if ghosts else 0)
-        out = dict(cell=np.zeros(n, np.uint32), r=np.zeros((n, 3)), v=np.zeros((n, 3)), f=np.zeros((n, 3)),
-                   ep=np.zeros(n), id=np.zeros(n, np.uint64), type=np.zeros(n, np.uint8))
+        out = dict(cell=np.empty(n, np.uint32), r=np.empty((n, 3)), v=np.empty((n, 3)), f=np.empty((n, 3)),
+                   ep=np.empty(n), id=np.empty(n, np.uint64), type=np.empty(n, np.uint8))
         self._check(self.L.xnb_get_particles(self._h, int(ghosts), _ptr(out["cell"]), _ptr(out["r"]), _ptr(out["v"]),
                                              _ptr(out["f"]), _ptr(out["ep"]), _ptr(out["id"]), _ptr(out["type"])),
                     "get_particles")
@@ -159,17 +159,19 @@ class Box:
 
     def streams(self, cells=None):
         """Per-cell CS=1 uint16 streams and the max neighbour count: a list of arrays, one per
-        cell, or a dict {cell: array} for the given cells."""
+        cell (slices of one array, none of them overlapping), or a dict {cell: array} for the
+        given cells."""
         tot, mx = C.c_size_t(), C.c_uint32()
         self._check(self.L.xnb_chunk_neighbors_stream(self._h, None, 0, None, C.byref(tot), C.byref(mx)), "stream size")
         _, _, nc = self.grid_info()
-        buf = np.zeros(max(tot.value, 1), np.uint16)
-        offs = np.zeros(nc + 1, np.uint64)
+        buf = np.empty(max(tot.value, 1), np.uint16)
+        offs = np.empty(nc + 1, np.uint64)
         self._check(self.L.xnb_chunk_neighbors_stream(self._h, _ptr(buf), buf.size, _ptr(offs), C.byref(tot),
                                                       C.byref(mx)), "stream export")
         if cells is not None:
             return {int(c): buf[offs[c]:offs[c + 1]].copy() for c in cells}, mx.value
-        return [buf[offs[c]:offs[c + 1]].copy() for c in range(nc)], mx.value
+        at = offs.tolist()
+        return [buf[a:b] for a, b in zip(at[:-1], at[1:])], mx.value
 
     def zero_particle_force(self, ghost=False):
         self._check(self.L.xnb_zero_particle_force(self._h, int(ghost)), "zero_particle_force")

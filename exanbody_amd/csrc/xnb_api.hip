@@ -16,6 +16,7 @@
 
 #include "../../include/xnb_amd.h"
 #include "xnb_ctx.h"
+#include "xnb_readback.h"
 
 using namespace xnb;
 
@@ -569,9 +570,11 @@ int xnb_create(xnb_ctx** out, const xnb_domain* d, int device) {
   if (hipGetDeviceCount(&ndev) != hipSuccess || ndev <= 0) return fail(nullptr, XNB_E_HIP, "no HIP device");
   if (device < 0 || device >= ndev) return fail(nullptr, XNB_E_ARG, "bad device index");
   xnb_ctx* c = new xnb_ctx();
+  readback_context_created();
   c->device = device;
   c->dom = *d;
   if (hipSetDevice(device) != hipSuccess || hipStreamCreateWithFlags(&c->st, hipStreamNonBlocking) != hipSuccess) {
+    readback_context_destroyed();
     delete c;
     return fail(nullptr, XNB_E_HIP, "stream creation failed");
   }
@@ -629,6 +632,7 @@ int xnb_destroy(xnb_ctx* c) {
   if (c->h_u32) (void)hipHostFree(c->h_u32);
   if (c->h_u64) (void)hipHostFree(c->h_u64);
   if (c->st) (void)hipStreamDestroy(c->st);
+  readback_context_destroyed();
   delete c;
   return XNB_OK;
 }
@@ -685,47 +689,32 @@ int xnb_set_particles_with_fields(xnb_ctx* c, size_t n, const double* r, const d
   const Geom& g = c->g;
   // host binning in input order (domain_periodic_location, domain.h:160-191)
   std::vector<uint32_t> cell(n), count(g.ncells, 0);
-  std::vector<double> wr(3 * n);
   for (size_t p = 0; p < n; p++) {
     double x = r[3 * p], y = r[3 * p + 1], z = r[3 * p + 2];
     int li, lj, lk;
     periodic_location(g, x, y, z, li, lj, lk);
     if (li < 0 || lj < 0 || lk < 0 || li >= g.Di || lj >= g.Dj || lk >= g.Dk)
       return fail(c, XNB_E_OUTSIDE, "particle outside a non-periodic domain");
-    wr[3 * p] = x;
-    wr[3 * p + 1] = y;
-    wr[3 * p + 2] = z;
     cell[p] = cell_index(g, li + g.gl, lj + g.gl, lk + g.gl);
     count[cell[p]]++;
   }
-  std::vector<uint32_t> off(g.ncells + 1, 0);
+  // ghost cells hold no particle yet; their offsets follow the inner slots
+  std::vector<uint32_t> off(g.ncells), cur(g.ncells), order(n);
   uint32_t acc = 0;
+  for (uint32_t q = 0; q < g.ncells; q++) {
+    cur[q] = acc;
+    acc += count[q];
+  }
   for (uint32_t q = 0; q < g.ncells; q++) {
     int i, j, k;
     cell_ijk(g, q, i, j, k);
-    off[q] = acc;
-    if (!is_ghost(g, i, j, k)) acc += count[q];
+    off[q] = is_ghost(g, i, j, k) ? acc : cur[q];
   }
-  for (uint32_t q = 0; q < g.ncells; q++) {  // ghost cells: empty, placed after inner slots
-    int i, j, k;
-    cell_ijk(g, q, i, j, k);
-    if (is_ghost(g, i, j, k)) off[q] = acc;
-  }
-  std::vector<uint32_t> cur(off.begin(), off.end() - 1);
-  std::vector<double4> hr(n);
-  std::vector<double> hv[3];
-  for (int a = 0; a < 3; a++) hv[a].assign(n, 0.0);
-  std::vector<uint64_t> hid(n);
-  std::vector<uint32_t> hsc(n);
+  for (size_t p = 0; p < n; p++) order[cur[cell[p]]++] = (uint32_t)p;
   std::vector<double> hx[kMaxExtraFields];
-  for (int k = 0; k < n_extra; k++) hx[k].resize(n);
-  for (size_t p = 0; p < n; p++) {
-    const uint32_t t = cur[cell[p]]++;
-    hr[t] = make_double4(wr[3 * p], wr[3 * p + 1], wr[3 * p + 2], type ? (double)type[p] : 0.0);
-    for (int a = 0; a < 3; a++) hv[a][t] = v ? v[3 * p + a] : 0.0;
-    hid[t] = id ? id[p] : (uint64_t)p;
-    hsc[t] = cell[p];
-    for (int k = 0; k < n_extra; k++) hx[k][t] = extra[k][p];
+  for (int k = 0; k < n_extra; k++) {
+    hx[k].resize(n);
+    for (size_t t = 0; t < n; t++) hx[k][t] = extra[k][order[t]];
   }
   c->N = (uint32_t)n;
   c->G = 0;
@@ -738,21 +727,10 @@ int xnb_set_particles_with_fields(xnb_ctx* c, size_t n, const double* r, const d
   for (int k = 0; k < n_extra; k++)
     if (n > 0) HIPCHK(c, hipMemcpyAsync(c->xA[k].p, hx[k].data(), n * sizeof(double), hipMemcpyHostToDevice, c->st));
   if (n > 0) {
-    HIPCHK(c, hipMemcpyAsync(c->A.r, hr.data(), n * sizeof(double4), hipMemcpyHostToDevice, c->st));
-    HIPCHK(c, hipMemcpyAsync(c->A.vx, hv[0].data(), n * sizeof(double), hipMemcpyHostToDevice, c->st));
-    HIPCHK(c, hipMemcpyAsync(c->A.vy, hv[1].data(), n * sizeof(double), hipMemcpyHostToDevice, c->st));
-    HIPCHK(c, hipMemcpyAsync(c->A.vz, hv[2].data(), n * sizeof(double), hipMemcpyHostToDevice, c->st));
-    HIPCHK(c, hipMemcpyAsync(c->A.id, hid.data(), n * sizeof(uint64_t), hipMemcpyHostToDevice, c->st));
-    HIPCHK(c, hipMemcpyAsync(c->slot_cell_A.p, hsc.data(), n * sizeof(uint32_t), hipMemcpyHostToDevice, c->st));
+    if ((e = write_particles(c, n, order.data(), cell.data(), r, v, id, type))) return e;
     launch_zero_force((uint32_t)n, c->A, c->st);
   }
-  std::vector<uint32_t> cn(g.ncells);
-  for (uint32_t q = 0; q < g.ncells; q++) {
-    int i, j, k;
-    cell_ijk(g, q, i, j, k);
-    cn[q] = is_ghost(g, i, j, k) ? 0u : count[q];
-  }
-  HIPCHK(c, hipMemcpyAsync(c->cell_n.p, cn.data(), g.ncells * sizeof(uint32_t), hipMemcpyHostToDevice, c->st));
+  HIPCHK(c, hipMemcpyAsync(c->cell_n.p, count.data(), g.ncells * sizeof(uint32_t), hipMemcpyHostToDevice, c->st));
   HIPCHK(c, hipMemcpyAsync(c->cell_off.p, off.data(), g.ncells * sizeof(uint32_t), hipMemcpyHostToDevice, c->st));
   HIPCHK(c, hipStreamSynchronize(c->st));
   c->lists_valid = c->ghosts_valid = c->backup_valid = false;
@@ -970,53 +948,7 @@ int xnb_get_particles(xnb_ctx* c, int include_ghosts, uint32_t* cell, double* r,
                       uint8_t* type) {
   int e;
   if ((e = check_ctx(c))) return e;
-  const size_t tot = (size_t)c->N + c->G;
-  const Geom& g = c->g;
-  std::vector<double4> hr(tot);
-  std::vector<double> hv[3], hf[3], he(tot);
-  std::vector<uint64_t> hid(tot);
-  std::vector<uint32_t> off(g.ncells), cn(g.ncells);
-  for (int a = 0; a < 3; a++) {
-    hv[a].resize(tot);
-    hf[a].resize(tot);
-  }
-  if (tot) {
-    HIPCHK(c, hipMemcpyAsync(hr.data(), c->A.r, tot * sizeof(double4), hipMemcpyDeviceToHost, c->st));
-    double* dv[3] = {c->A.vx, c->A.vy, c->A.vz};
-    double* df[3] = {c->A.fx, c->A.fy, c->A.fz};
-    for (int a = 0; a < 3; a++) {
-      HIPCHK(c, hipMemcpyAsync(hv[a].data(), dv[a], tot * sizeof(double), hipMemcpyDeviceToHost, c->st));
-      HIPCHK(c, hipMemcpyAsync(hf[a].data(), df[a], tot * sizeof(double), hipMemcpyDeviceToHost, c->st));
-    }
-    HIPCHK(c, hipMemcpyAsync(he.data(), c->A.ep, tot * sizeof(double), hipMemcpyDeviceToHost, c->st));
-    HIPCHK(c, hipMemcpyAsync(hid.data(), c->A.id, tot * sizeof(uint64_t), hipMemcpyDeviceToHost, c->st));
-  }
-  HIPCHK(c, hipMemcpyAsync(off.data(), c->cell_off.p, g.ncells * sizeof(uint32_t), hipMemcpyDeviceToHost, c->st));
-  HIPCHK(c, hipMemcpyAsync(cn.data(), c->cell_n.p, g.ncells * sizeof(uint32_t), hipMemcpyDeviceToHost, c->st));
-  HIPCHK(c, hipStreamSynchronize(c->st));
-  size_t k = 0;
-  for (uint32_t q = 0; q < g.ncells; q++) {
-    int i, j, kk;
-    cell_ijk(g, q, i, j, kk);
-    if (!include_ghosts && is_ghost(g, i, j, kk)) continue;
-    for (uint32_t p = 0; p < cn[q]; p++, k++) {
-      const size_t s = (size_t)off[q] + p;
-      if (cell) cell[k] = q;
-      if (r) {
-        r[3 * k] = hr[s].x;
-        r[3 * k + 1] = hr[s].y;
-        r[3 * k + 2] = hr[s].z;
-      }
-      for (int a = 0; a < 3; a++) {
-        if (v) v[3 * k + a] = hv[a][s];
-        if (f) f[3 * k + a] = hf[a][s];
-      }
-      if (ep) ep[k] = he[s];
-      if (id) id[k] = hid[s];
-      if (type) type[k] = (uint8_t)hr[s].w;
-    }
-  }
-  return XNB_OK;
+  return read_particles(c, include_ghosts != 0, cell, r, v, f, ep, id, type);
 }
 
 int xnb_move_particles(xnb_ctx* c) {
@@ -1111,11 +1043,10 @@ int xnb_chunk_neighbors_stream(xnb_ctx* c, uint16_t* out, size_t cap, uint64_t* 
   launch_stream_fill(g, c->list_atoms, c->slot_cell_A.p, c->cell_off.p, c->cell_n.p, c->nbr.p, c->nbr_cnt.p, c->nbr_cap, c->pstart.p,
                      c->plen.p, c->coff.p, ntables, c->list_cfg.random_access, c->stream_buf.p, c->st);
   HIPCHK(c, hipGetLastError());
-  std::vector<uint32_t> co(g.ncells);
-  HIPCHK(c, hipMemcpyAsync(out, c->stream_buf.p, (size_t)tot * sizeof(uint16_t), hipMemcpyDeviceToHost, c->st));
-  HIPCHK(c, hipMemcpyAsync(co.data(), c->coff.p, g.ncells * sizeof(uint32_t), hipMemcpyDeviceToHost, c->st));
-  HIPCHK(c, hipStreamSynchronize(c->st));
+  if ((e = read_bytes(c, c->stream_buf.p, (size_t)tot * sizeof(uint16_t), out))) return e;
   if (cell_offsets) {
+    std::vector<uint32_t> co(g.ncells);
+    if ((e = read_bytes(c, c->coff.p, g.ncells * sizeof(uint32_t), co.data()))) return e;
     for (uint32_t q = 0; q < g.ncells; q++) cell_offsets[q] = co[q];
     cell_offsets[g.ncells] = tot;
   }

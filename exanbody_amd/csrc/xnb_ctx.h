@@ -148,6 +148,7 @@ void bind_states(xnb_ctx* c);
 void swap_buffers(xnb_ctx* c);
 int ensure_capacity(xnb_ctx* c, size_t ncap, size_t keep);
 int check_ctx(xnb_ctx* c);
+int scan(xnb_ctx* c, const uint32_t* in, uint32_t n, uint32_t add, uint32_t* out);
 int op_ghost_all(xnb_ctx* c, bool move_check = false, bool forces = true);
 int op_backup(xnb_ctx* c);
 int op_amr(xnb_ctx* c, double density, bool forces);

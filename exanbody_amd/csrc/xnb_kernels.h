@@ -235,4 +235,40 @@ hipError_t launch_brick_to_slots(const Geom& g, BrickParams bp, const uint32_t* 
                                  const uint32_t* bcnt, uint32_t* nbr, uint32_t* nbr_cnt, uint32_t cap, hipStream_t st);
 void launch_energies(uint32_t N, const PState& A, double* part, uint32_t nparts, double* out, hipStream_t st);
 
+// ---- particles in a caller's layout (xnb_get_particles)
+constexpr uint32_t kPackThreads = 256;
+enum { kPackR = 1, kPackV = 2, kPackF = 4, kPackE = 8, kPackId = 16, kPackCell = 32, kPackType = 64 };
+// Byte offsets of the fields in a block of m particles; each present field takes a multiple of
+// 16 bytes, all of them `bytes`.
+struct PackLayout {
+  uint32_t r, v, f, ep, id, cell, type, bytes;
+};
+inline PackLayout pack_layout(uint32_t m, int fields) {
+  PackLayout L{};
+  auto put = [&](int bit, uint32_t elem, uint32_t& at) {
+    at = L.bytes;
+    if (fields & bit) L.bytes += (m * elem + 15u) & ~15u;
+  };
+  put(kPackR, 24, L.r);
+  put(kPackV, 24, L.v);
+  put(kPackF, 24, L.f);
+  put(kPackE, 8, L.ep);
+  put(kPackId, 8, L.id);
+  put(kPackCell, 4, L.cell);
+  put(kPackType, 1, L.type);
+  return L;
+}
+// Particles first .. first + m - 1 of order (slots; null: every slot in turn) into out, which is
+// device-visible and holds pack_layout(m, fields).bytes.
+void launch_pack_particles(const PState& A, const uint32_t* slot_cell, const uint32_t* order, uint32_t first, uint32_t m, int fields,
+                           char* out, hipStream_t st);
+// Slots first .. first + m - 1 from in: m each of x, y, z, vx, vy, vz, id (8 bytes), cell and
+// type (4 bytes); positions are wrapped into the periodic domain.
+constexpr size_t kUnpackBytes = 64;
+void launch_unpack_particles(const Geom& g, const PState& A, uint32_t* slot_cell, uint32_t first, uint32_t m, const char* in,
+                             hipStream_t st);
+// order[start[cell of s] + index of s in its cell] = s for the slots s < n
+void launch_cell_order(uint32_t n, const uint32_t* slot_cell, const uint32_t* cell_off, const uint32_t* start, uint32_t* order,
+                       hipStream_t st);
+
 }  // namespace xnb

@@ -993,6 +993,81 @@ __global__ void k_stream_fill(Geom g, uint32_t n_atoms, const uint32_t* __restri
   }
 }
 
+// ------------------------------------------------------- particles in a caller's layout
+// cnt x 3 doubles of one workgroup through LDS: lane t's x, y, z become words 3 t .. 3 t + 2 of
+// a contiguous run, stored 16 bytes a lane so that the bus sees whole lines
+__device__ inline void store_xyz(double* tile, double x, double y, double z, double* out, uint32_t cnt) {
+  const uint32_t t = threadIdx.x;
+  tile[3 * t] = x;
+  tile[3 * t + 1] = y;
+  tile[3 * t + 2] = z;
+  __syncthreads();
+  const uint32_t words = 3 * cnt;
+  for (uint32_t w = 2 * t; w < words; w += 2 * kPackThreads) {
+    if (w + 1 < words) *reinterpret_cast<double2*>(out + w) = make_double2(tile[w], tile[w + 1]);
+    else out[w] = tile[w];
+  }
+  __syncthreads();
+}
+
+// Particles first .. first + m - 1 of the output order (order: their slots; null: the slots
+// themselves) in the caller's layout.  Bound by the bus (93 bytes a particle with every field).
+__global__ void __launch_bounds__(kPackThreads) k_pack_particles(PState A, const uint32_t* __restrict__ slot_cell,
+                                                                 const uint32_t* __restrict__ order, uint32_t first, uint32_t m,
+                                                                 int fields, PackLayout L, char* __restrict__ out) {
+  __shared__ __align__(16) double tile[3 * kPackThreads];
+  __shared__ __align__(16) uint8_t types[kPackThreads];
+  const uint32_t t = threadIdx.x, base = blockIdx.x * kPackThreads;
+  const uint32_t cnt = min(kPackThreads, m - base);
+  const bool live = t < cnt;
+  uint32_t s = 0;
+  if (live) s = order ? order[first + base + t] : first + base + t;
+  if (fields & (kPackR | kPackType)) {
+    const double4 p = live ? A.r[s] : make_double4(0., 0., 0., 0.);
+    if (fields & kPackType) types[t] = (uint8_t)p.w;
+    if (fields & kPackR) store_xyz(tile, p.x, p.y, p.z, reinterpret_cast<double*>(out + L.r) + 3 * (size_t)base, cnt);
+    else __syncthreads();
+    if ((fields & kPackType) && 4 * t < cnt)  // the section is padded to 16 bytes
+      reinterpret_cast<uint32_t*>(out + L.type)[base / 4 + t] = reinterpret_cast<const uint32_t*>(types)[t];
+  }
+  if (fields & kPackV)
+    store_xyz(tile, live ? A.vx[s] : 0., live ? A.vy[s] : 0., live ? A.vz[s] : 0., reinterpret_cast<double*>(out + L.v) + 3 * (size_t)base,
+              cnt);
+  if (fields & kPackF)
+    store_xyz(tile, live ? A.fx[s] : 0., live ? A.fy[s] : 0., live ? A.fz[s] : 0., reinterpret_cast<double*>(out + L.f) + 3 * (size_t)base,
+              cnt);
+  if (!live) return;
+  if (fields & kPackE) reinterpret_cast<double*>(out + L.ep)[base + t] = A.ep[s];
+  if (fields & kPackId) reinterpret_cast<uint64_t*>(out + L.id)[base + t] = A.id[s];
+  if (fields & kPackCell) reinterpret_cast<uint32_t*>(out + L.cell)[base + t] = slot_cell[s];
+}
+
+__global__ void __launch_bounds__(256) k_unpack_particles(Geom g, PState A, uint32_t* __restrict__ slot_cell, uint32_t first, uint32_t m,
+                                                           const double* __restrict__ in) {
+  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= m) return;
+  const uint32_t s = first + t;
+  const uint32_t* words = reinterpret_cast<const uint32_t*>(in + 7 * (size_t)m);
+  double x = in[t], y = in[(size_t)m + t], z = in[2 * (size_t)m + t];
+  int li, lj, lk;
+  periodic_location(g, x, y, z, li, lj, lk);
+  A.r[s] = make_double4(x, y, z, (double)words[m + t]);
+  A.vx[s] = in[3 * (size_t)m + t];
+  A.vy[s] = in[4 * (size_t)m + t];
+  A.vz[s] = in[5 * (size_t)m + t];
+  A.id[s] = reinterpret_cast<const uint64_t*>(in)[6 * (size_t)m + t];
+  slot_cell[s] = words[t];
+}
+
+// order[position of slot s among all cells in index order] = s
+__global__ void k_cell_order(uint32_t n, const uint32_t* __restrict__ slot_cell, const uint32_t* __restrict__ cell_off,
+                             const uint32_t* __restrict__ start, uint32_t* __restrict__ order) {
+  const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
+  if (s >= n) return;
+  const uint32_t c = slot_cell[s];
+  order[start[c] + (s - cell_off[c])] = s;
+}
+
 // --------------------------------------------------------------------- energies
 // Deterministic two-pass reduction: fixed per-block shuffle tree, then one block sums the
 // block partials in index order.
@@ -1242,6 +1317,19 @@ void launch_stream_fill(const Geom& g, uint32_t n_atoms, const uint32_t* slot_ce
                         const uint32_t* coff, int ntables, int random_access, uint16_t* out, hipStream_t st) {
   k_stream_fill<<<nblk(n_atoms, 256), 256, 0, st>>>(g, n_atoms, slot_cell, cell_off, cell_n, nbr, nbr_cnt, cap, pstart, plen, coff,
                                                     ntables, random_access, out);
+}
+
+void launch_pack_particles(const PState& A, const uint32_t* slot_cell, const uint32_t* order, uint32_t first, uint32_t m, int fields,
+                           char* out, hipStream_t st) {
+  k_pack_particles<<<nblk(m, kPackThreads), kPackThreads, 0, st>>>(A, slot_cell, order, first, m, fields, pack_layout(m, fields), out);
+}
+void launch_unpack_particles(const Geom& g, const PState& A, uint32_t* slot_cell, uint32_t first, uint32_t m, const char* in,
+                             hipStream_t st) {
+  k_unpack_particles<<<nblk(m, 256), 256, 0, st>>>(g, A, slot_cell, first, m, reinterpret_cast<const double*>(in));
+}
+void launch_cell_order(uint32_t n, const uint32_t* slot_cell, const uint32_t* cell_off, const uint32_t* start, uint32_t* order,
+                       hipStream_t st) {
+  k_cell_order<<<nblk(n, 256), 256, 0, st>>>(n, slot_cell, cell_off, start, order);
 }
 
 void launch_energies(uint32_t N, const PState& A, double* part, uint32_t nparts, double* out, hipStream_t st) {
