@@ -319,28 +319,43 @@ inline uint32_t grow_cap(uint32_t mx) {
   return (mx + mx / 8 + gran - 1) / gran * gran;
 }
 
-// Brick dims, T and Rmax for the current cell occupancy; NOT_APPLICABLE if nothing fits LDS.
-int choose_bricks(xnb_ctx* c, uint32_t cap, BrickParams& out) {
-  // (4,3,2) and (3,3,2) only for batched boxes: under the batch's LDS cap they beat (4,2,2)
-  // (512-box batch: 3.58e9 -> 3.90e9 atom-steps/s), while the two-species slab run alone is
-  // faster on (4,2,2) bricks
-  static const int cand[][3] = {{4, 4, 2}, {4, 3, 2}, {3, 3, 2}, {4, 2, 2}, {2, 2, 2}, {4, 2, 1}, {2, 2, 1}, {2, 1, 1}, {1, 1, 1}};
-  const int ncand = (int)(sizeof(cand) / sizeof(cand[0]));
-  int e;
-  for (int q = -1; q < ncand; q++) {
-    if ((q == 1 || q == 2) && !c->batch_shapes) continue;
+// Boxes of at most this many atoms give every atom four lanes (four atoms' lanes fill two waves
+// per SIMD of the chip; larger boxes have enough waves with one lane an atom, which takes 1.7
+// times fewer instructions).  Force and build launch with one and with four lanes: 6,912 atoms
+// FP64 20.5 and 13.6, 68 and 28 us; 27,431 atoms mixed 15.8 and 15.5, 68 and 38 us; 131,072
+// atoms FP64 36 and 50, 89 and 104 us.
+constexpr uint32_t kQuadAtoms = 32768;
+// Bricks are made smaller until there are this many (three quarters of the CUs): with fewer,
+// idle CUs cost more than the larger staged share of smaller bricks.  60,000-atom slab,
+// force: 112 bricks 70 us, 196 bricks 45 us; 131,072 atoms: 250 bricks 36 us, 500 bricks 41 us.
+constexpr uint32_t kEnoughBricks = 192;
+
+// Brick dims, lanes, T and Rmax for the current cell occupancy; NOT_APPLICABLE if nothing fits LDS.
+int choose_bricks(xnb_ctx* c, uint32_t cap, bool quads, BrickParams& out) {
+  struct Cand {
     int dims[3];
-    if (q < 0) {
-      if (c->brick_dims[0] <= 0) continue;
-      dims[0] = c->brick_dims[0];
-      dims[1] = c->brick_dims[1];
-      dims[2] = c->brick_dims[2];
-    } else {
-      dims[0] = cand[q][0];
-      dims[1] = cand[q][1];
-      dims[2] = cand[q][2];
-    }
-    BrickParams bp = brick_params(c->g, dims[0], dims[1], dims[2]);
+    uint32_t lanes;
+    bool any;  // taken whatever its brick count
+  };
+  // Larger bricks first.  (4,3,2) and (3,3,2) only for batched boxes: under the batch's LDS cap
+  // they beat (4,2,2) (512-box batch: 3.58e9 -> 3.90e9 atom-steps/s), while the two-species slab
+  // run alone is faster on (4,2,2) bricks.  Batched boxes share the chip: no brick count to reach.
+  static const int wide[][3] = {{4, 4, 2}, {4, 3, 2}, {3, 3, 2}, {4, 2, 2}, {2, 2, 2}, {4, 2, 1}, {2, 2, 1}, {2, 1, 1}, {1, 1, 1}};
+  static const int quad[][3] = {{2, 2, 2}, {2, 2, 1}, {2, 1, 1}, {1, 1, 1}};
+  Cand cand[2 + 4 + 9];
+  int ncand = 0;
+  auto add = [&](const int (&d)[3], uint32_t lanes, bool any) { cand[ncand++] = Cand{{d[0], d[1], d[2]}, lanes, any}; };
+  if (c->brick_dims[0] > 0) {
+    if (quads) add(c->brick_dims, kQuad, true);
+    add(c->brick_dims, 1u, true);
+  }
+  if (quads)
+    for (const auto& d : quad) add(d, kQuad, &d == &quad[3]);
+  for (int q = 0; q < 9; q++)
+    if ((q != 1 && q != 2) || c->batch_shapes) add(wide[q], 1u, c->batch_shapes || q == 8);
+  for (int q = 0; q < ncand; q++) {
+    BrickParams bp = brick_params(c->g, cand[q].dims[0], cand[q].dims[1], cand[q].dims[2]);
+    if (!cand[q].any && bp.nbricks < kEnoughBricks) continue;
     HIPCHK(c, hipMemsetAsync(c->u32s.p + 3, 0, 2 * sizeof(uint32_t), c->st));
     launch_brick_stats(c->g, bp, c->cell_n.p, c->u32s.p + 3, c->st);
     HIPCHK(c, hipGetLastError());
@@ -351,7 +366,8 @@ int choose_bricks(xnb_ctx* c, uint32_t cap, BrickParams& out) {
     const uint32_t r_max = (uint32_t)std::ceil(c->h_u32[1] * c->brick_margin);
     uint32_t T = std::max<uint32_t>({nb_max, (uint32_t)bp.nrc, (uint32_t)bp.nbc, 64u});
     T = (T + 63) / 64 * 64;
-    if (T > 1024 || r_max >= 65535u) continue;
+    bp.lanes = cand[q].lanes;
+    if (T * bp.lanes > 1024 || r_max >= 65535u) continue;
     bp.T = T;
     bp.Rmax = std::max<uint32_t>(r_max, 1u);
     bp.cap = cap;
@@ -360,7 +376,6 @@ int choose_bricks(xnb_ctx* c, uint32_t cap, BrickParams& out) {
     out = bp;
     return XNB_OK;
   }
-  (void)e;
   return NOT_APPLICABLE;
 }
 
@@ -368,9 +383,12 @@ int op_nbh_brick(xnb_ctx* c, double nbh_dist, const xnb_chunk_neighbors_config& 
   const double max2 = nbh_dist * nbh_dist;
   int e;
   uint32_t cap = (c->nbr_cap + list_granule() - 1) / list_granule() * list_granule();
+  // four lanes an atom: lists of the prefiltered build, for a box run by itself
+  const bool quads = (c->brick_lanes ? c->brick_lanes == (int)kQuad : c->N <= kQuadAtoms) && !c->batch_shapes && c->nbh_prefilter &&
+                     !cfg.half_symmetric && !cfg.skip_ghosts;
   for (int attempt = 0; attempt < 3; attempt++) {
     BrickParams bp;
-    if ((e = choose_bricks(c, cap, bp))) return e;
+    if ((e = choose_bricks(c, cap, quads, bp))) return e;
     if ((e = dalloc(c, c->blist, (size_t)bp.nbricks * bp.cap * bp.T))) return e;
     if ((e = dalloc(c, c->bcnt, (size_t)bp.nbricks * bp.T))) return e;
     HIPCHK(c, hipMemsetAsync(c->u32s.p + 2, 0, sizeof(uint32_t), c->st));
@@ -597,9 +615,9 @@ int xnb_create(xnb_ctx** out, const xnb_domain* d, int device) {
   int lds = 0;
   if (hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device) == hipSuccess && lds > 0)
     c->lds_limit = (uint32_t)lds;
-  if (const char* v = std::getenv("XNB_BRICKS")) {  // "0" disables the brick path, "i,j,k" fixes brick dims
+  if (const char* v = std::getenv("XNB_BRICKS")) {  // "0" disables the brick path, "i,j,k[,lanes]" fixes brick dims (and lanes per atom)
     if (v[0] == '0' && v[1] == 0) c->use_bricks = false;
-    else std::sscanf(v, "%d,%d,%d", &c->brick_dims[0], &c->brick_dims[1], &c->brick_dims[2]);
+    else std::sscanf(v, "%d,%d,%d,%d", &c->brick_dims[0], &c->brick_dims[1], &c->brick_dims[2], &c->brick_lanes);
   }
   if (const char* v = std::getenv("XNB_FUSE_PUSH")) c->fuse_push = v[0] != '0';
   if (const char* v = std::getenv("XNB_NBH_PREFILTER")) c->nbh_prefilter = v[0] != '0';

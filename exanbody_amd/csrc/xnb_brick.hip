@@ -16,6 +16,7 @@
 // Requires cell_layers == 1 (cell edge >= nbh_dist) and ghost layers >= 1.
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "xnb_kernels.h"
@@ -345,9 +346,9 @@ struct LaneAtom {
   uint32_t slot;  // global slot
 };
 
-__device__ inline LaneAtom lane_atom(const BrickParams& bp, const BrickLds& L) {
+// atom t of the brick
+__device__ inline LaneAtom lane_atom(const BrickParams& bp, const BrickLds& L, uint32_t t) {
   LaneAtom A;
-  const uint32_t t = threadIdx.x;
   A.live = t < L.bpref[bp.nbc];
   if (!A.live) {
     A.rc = 0;
@@ -404,19 +405,22 @@ __global__ void k_brick_stats(Geom g, BrickParams bp, const uint32_t* __restrict
 // positions, so the lists are those of the FP64 test.  With PAIRWISE the chunk test keeps a
 // superset at the atom's largest pair radius and each candidate is decided against its own
 // pair's radius while the mask is expanded.
-template <bool FILTER, bool PAIRWISE = false, bool PREF = false>
+// LANES 4 (prefiltered builds of small boxes): four lanes share an atom.  Each tests its quarter
+// of a row's candidates; their kept counts give each lane the place of its entries in the list.
+template <bool FILTER, bool PAIRWISE = false, bool PREF = false, uint32_t LANES = 1>
 __device__ __forceinline__ void nbh_brick_body(const Geom& g, const BrickParams& bp, uint32_t b, const double4* __restrict__ r,
                                                const uint32_t* __restrict__ cell_off, const uint32_t* __restrict__ cell_n,
                                                double max2, int half_symmetric, int skip_ghosts, uint16_t* __restrict__ blist,
                                                uint32_t* __restrict__ bcnt, uint32_t* __restrict__ max_cnt,
                                                const PairCut* pc = nullptr) {
   static_assert(!PREF || !FILTER, "the FP32 prefilter serves the unfiltered builds");
+  static_assert(LANES == 1 || (LANES == kQuad && PREF), "four lanes an atom only with the prefilter");
   extern __shared__ __align__(16) char lds[];
   const BrickLds L = brick_lds(bp, lds);
   const BrickPos P = brick_pos(g, bp, b);
   if (!brick_setup(g, bp, P, L, r, cell_off, cell_n, PREF ? (PAIRWISE ? kPosF32N : kPosF32) : kPosF64)) return;
-  const LaneAtom A = lane_atom(bp, L);
-  const uint32_t t = threadIdx.x, T = bp.T;
+  const uint32_t t = threadIdx.x / LANES, T = bp.T;
+  const LaneAtom A = lane_atom(bp, L, t);
   uint16_t* out = blist + (size_t)b * bp.cap * T;
   // every lane, live or not, tests against its own LDS atom when past the candidate cell's
   // end (A.ia = 0 for lanes without an atom), so d2 == 0 rejects those candidates
@@ -514,8 +518,9 @@ __device__ __forceinline__ void nbh_brick_body(const Geom& g, const BrickParams&
         const uint32_t rbase = A.live ? L.rpref[rc0] : R;
         const uint32_t rlen = A.live ? L.rpref[rc0 + 3] - rbase : 0u;
         const uint32_t lmax = wave_max_b(rlen);
-        for (uint32_t p0 = 0; p0 < lmax; p0 += 32) {
-          const uint32_t np = min((lmax - p0 + 3) & ~3u, 32u);
+        for (uint32_t row0 = 0; row0 < lmax; row0 += 32 * LANES) {
+          const uint32_t np = min(((lmax - row0 + LANES - 1) / LANES + 3) & ~3u, 32u);
+          const uint32_t p0 = row0 + (threadIdx.x % LANES) * np;  // this lane's candidates of the row
           const uint32_t lb = p0 < rlen ? rbase + p0 : R;
           const float4* pp = L.pf + lb;
           uint32_t mhi = 0, mlo = 0;  // bit 31 - k: candidate k within the chunk radius + H2; surely kept
@@ -565,6 +570,58 @@ __device__ __forceinline__ void nbh_brick_body(const Geom& g, const BrickParams&
                 }
               }
             }
+          }
+          // kept iff 0 < d2 <= the radius^2 of this pair (types above 3 use type 0's)
+          auto pair_kept = [&](uint32_t ib) {
+            const float4 c = L.pf[ib];
+            const float dx = af.x - c.x, dy = af.y - c.y, dz = af.z - c.z;
+            const float d2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+            const uint32_t tb = L.pt[ib];
+            float tl = tlo[0], th = thi[0];
+#pragma unroll
+            for (int q = 1; q < 4; q++) {
+              tl = tb == (uint32_t)q ? tlo[q] : tl;
+              th = tb == (uint32_t)q ? thi[q] : th;
+            }
+            bool keep = d2 > zf && d2 < tl;
+            if (!keep && d2 <= th) {
+              if (!have_pa) pa = r[A.slot];
+              have_pa = true;
+              const double4 pb = r[region_slot(bp, L, ib)];
+              const double ex = pa.x - pb.x;
+              const double ey = pa.y - pb.y;
+              const double ez = pa.z - pb.z;
+              const double e2 = (ex * ex + ey * ey) + ez * ez;
+              double lim = thr[0];
+#pragma unroll
+              for (int q = 1; q < 4; q++) lim = tb == (uint32_t)q ? thr[q] : lim;
+              keep = e2 > 0.0 && e2 <= lim;
+            }
+            return keep;
+          };
+          if constexpr (LANES > 1) {
+            if (PAIRWISE) {
+              for (uint32_t left = m; left;) {
+                const uint32_t bit = 0x80000000u >> __builtin_clz(left);
+                left ^= bit;
+                if (!pair_kept(lb + (uint32_t)__builtin_clz(bit))) m ^= bit;
+              }
+            }
+            const uint32_t mine = (uint32_t)__popc(m), c = threadIdx.x % LANES;
+            const uint32_t n0 = quad_get<0>(mine), n1 = quad_get<1>(mine), n2 = quad_get<2>(mine), n3 = quad_get<3>(mine);
+            uint32_t q = cnt + (c > 0 ? n0 : 0u) + (c > 1 ? n1 : 0u) + (c > 2 ? n2 : 0u);
+            cnt += n0 + n1 + n2 + n3;
+            // a list that passes cap stores nothing more: the caller rebuilds with a larger cap
+            if (cnt > bp.cap) m = 0;
+            while (m) {
+              const uint32_t k = (uint32_t)__builtin_clz(m);
+              m ^= 0x80000000u >> k;
+              out[lpos(q, t, T)] = (uint16_t)(lb + k);
+              ++q;
+            }
+            continue;
+          }
+          if (!PAIRWISE) {
             // a list that would pass cap stores nothing more (its count still grows, so the
             // caller rebuilds with a larger cap)
             const uint32_t pcnt = (uint32_t)__popc(m);
@@ -576,35 +633,7 @@ __device__ __forceinline__ void nbh_brick_body(const Geom& g, const BrickParams&
           while (m) {
             const uint32_t k = (uint32_t)__builtin_clz(m);
             m ^= 0x80000000u >> k;
-            if (PAIRWISE) {
-              // kept iff 0 < d2 <= the radius^2 of this pair (types above 3 use type 0's)
-              const uint32_t ib = lb + k;
-              const float4 c = L.pf[ib];
-              const float dx = af.x - c.x, dy = af.y - c.y, dz = af.z - c.z;
-              const float d2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-              const uint32_t tb = L.pt[ib];
-              float tl = tlo[0], th = thi[0];
-#pragma unroll
-              for (int q = 1; q < 4; q++) {
-                tl = tb == (uint32_t)q ? tlo[q] : tl;
-                th = tb == (uint32_t)q ? thi[q] : th;
-              }
-              bool keep = d2 > zf && d2 < tl;
-              if (!keep && d2 <= th) {
-                if (!have_pa) pa = r[A.slot];
-                have_pa = true;
-                const double4 pb = r[region_slot(bp, L, ib)];
-                const double ex = pa.x - pb.x;
-                const double ey = pa.y - pb.y;
-                const double ez = pa.z - pb.z;
-                const double e2 = (ex * ex + ey * ey) + ez * ez;
-                double lim = thr[0];
-#pragma unroll
-                for (int q = 1; q < 4; q++) lim = tb == (uint32_t)q ? thr[q] : lim;
-                keep = e2 > 0.0 && e2 <= lim;
-              }
-              if (!keep) continue;
-            }
+            if (PAIRWISE && !pair_kept(lb + k)) continue;
             plo = __builtin_amdgcn_alignbit(phi, plo, 16);
             phi = __builtin_amdgcn_alignbit(lb + k, phi, 16);
             ++cnt;
@@ -612,6 +641,22 @@ __device__ __forceinline__ void nbh_brick_body(const Geom& g, const BrickParams&
           }
         }
       }
+    if constexpr (LANES > 1) {
+      // every list of the workgroup ends with the sentinel up to a multiple of kQuadBatch of the
+      // longest, so the force reads whole batches, with one or four lanes an atom
+      if (!A.live) cnt = 0;
+      if (threadIdx.x % LANES == 0) bcnt[(size_t)b * T + t] = cnt;
+      const uint32_t wm = wave_max_b(cnt);
+      if ((threadIdx.x & 63u) == 0) L.wsum[threadIdx.x >> 6] = wm;
+      __syncthreads();
+      uint32_t longest = 0;
+      for (uint32_t w = 0; w < (blockDim.x >> 6); w++) longest = max(longest, L.wsum[w]);
+      if (threadIdx.x == 0 && longest > 0) atomicMax(max_cnt, longest);
+      const uint32_t end = min((longest + kQuadBatch - 1) / kQuadBatch * kQuadBatch, bp.cap);
+      const uint16_t pad = (uint16_t)R;
+      for (uint32_t q = min(cnt, bp.cap) + threadIdx.x % LANES; q < end; q += LANES) out[lpos(q, t, T)] = pad;
+      return;
+    }
     // close the lane's list: the partial group and whole groups of the sentinel up to the
     // wave's batch boundary, so force kernels need no per-lane bound inside a batch
     if (!A.live) cnt = 0;
@@ -752,14 +797,14 @@ __device__ __forceinline__ void nbh_brick_body(const Geom& g, const BrickParams&
   for (uint32_t q = min(cnt, bp.cap); q < pad_end; q++) out[lpos(q, t, T)] = sentinel;
 }
 
-template <bool FILTER, bool PAIRWISE, bool PREF = false>
+template <bool FILTER, bool PAIRWISE, bool PREF = false, uint32_t LANES = 1>
 __global__ void __launch_bounds__(1024) k_nbh_brick_mask(Geom g, BrickParams bp, const double4* __restrict__ r,
                                                          const uint32_t* __restrict__ cell_off, const uint32_t* __restrict__ cell_n,
                                                          double max2, int half_symmetric, int skip_ghosts, uint16_t* __restrict__ blist,
                                                          uint32_t* __restrict__ bcnt, uint32_t* __restrict__ max_cnt, PairCut pc) {
   const uint32_t b = brick_of_block<true>(bp);
   if (b >= bp.nbricks) return;  // whole workgroup, before any barrier
-  nbh_brick_body<FILTER, PAIRWISE, PREF>(g, bp, b, r, cell_off, cell_n, max2, half_symmetric, skip_ghosts, blist, bcnt, max_cnt, &pc);
+  nbh_brick_body<FILTER, PAIRWISE, PREF, LANES>(g, bp, b, r, cell_off, cell_n, max2, half_symmetric, skip_ghosts, blist, bcnt, max_cnt, &pc);
 }
 
 // ------------------------------------------------------------------ pair traversal
@@ -819,7 +864,7 @@ __device__ __forceinline__ void compute_pair_brick_body(const Geom& g, const Bri
 #pragma unroll
   for (int w = 0; w < W; w++) wn[w] = t < T ? load_list_group(lst + (size_t)w * T) : make_uint2(0u, 0u);
   if (!brick_setup(g, bp, P, L, r, cell_off, cell_n, kPosF64)) return;
-  const LaneAtom At = lane_atom(bp, L);
+  const LaneAtom At = lane_atom(bp, L, threadIdx.x);
   const uint32_t n = At.live ? n_list : 0u;
   const uint32_t nmax = wave_max_b(n);
   double4 ra;
@@ -960,6 +1005,150 @@ __global__ void __launch_bounds__(1024) k_lj_brick(Geom g, BrickParams bp, const
                                                                           LennardJonesForceFunctor<MIXED>{lj}, lj.rc2, A, dth, nx);
 }
 
+// ------------------------------------------------------------------ four lanes an atom
+// The LJ force of a box too small to fill the chip, where a launch takes as long as one lane
+// needs for its list.  Four lanes share an atom: of four consecutive entries each evaluates
+// one, the coefficients go round the four lanes, and lane c adds component c of the four pairs
+// in list order (lane 3 the energies), so the sums are those of one lane an atom bit for bit.
+// Component c of a neighbour is read from LDS again rather than sent across.  A group of four
+// entries costs a lane about 70 instead of 4 x 42 instructions.  The quad's lanes load four
+// consecutive groups of the list with one load each, kAhead such loads in flight.
+template <bool MIXED, bool ACCUM, int EPI>
+__device__ __forceinline__ void lj_quad_brick_body(const Geom& g, const BrickParams& bp, uint32_t b, const double4* __restrict__ r,
+                                                   const uint32_t* __restrict__ cell_off, const uint32_t* __restrict__ cell_n,
+                                                   const uint16_t* __restrict__ blist, const uint32_t* __restrict__ bcnt,
+                                                   const LJConst& lj, const PState& A, double dth, const NextStep& nx) {
+  static_assert(!(EPI == EPI_NEXT && ACCUM), "a fused step starts the force from 0");
+  constexpr bool ENERGY = EPI != EPI_NEXT, NEXT = EPI == EPI_NEXT;
+  constexpr uint32_t kAhead = 4;
+  using Coef = std::conditional_t<MIXED, float, double>;
+  extern __shared__ __align__(16) char lds[];
+  const BrickLds L = brick_lds(bp, lds);
+  const BrickPos P = brick_pos(g, bp, b);
+  if (NEXT && threadIdx.x == 0) {  // ordered before every wave's count by brick_setup's barriers
+    L.wcnt[0] = 0;
+    L.wcnt[1] = 0;
+  }
+  const uint32_t t = threadIdx.x / kQuad, c = threadIdx.x % kQuad, T = bp.T;
+  const uint32_t n_list = bcnt[(size_t)b * T + t];
+  // batch k of the list is the groups 4 k .. 4 k + 3, the lane's own is 4 k + c; every slab
+  // holds whole batches (cap is a multiple of kQuadBatch)
+  const uint2* const lst = reinterpret_cast<const uint2*>(blist + (size_t)b * bp.cap * T) + (size_t)c * T + t;
+  uint2 ahead[kAhead];
+#pragma unroll
+  for (uint32_t k = 0; k < kAhead; k++)
+    ahead[k] = k * kQuadBatch < bp.cap ? load_list_group(lst + (size_t)(4 * k) * T) : make_uint2(0u, 0u);
+  if (!brick_setup(g, bp, P, L, r, cell_off, cell_n, kPosF64)) return;
+  const LaneAtom At = lane_atom(bp, L, t);
+  const uint32_t nmax = wave_max_b(At.live ? n_list : 0u);
+  const double ax = L.px[3 * At.ia], ay = L.py[3 * At.ia], az = L.pz[3 * At.ia];
+  const uint32_t comp = min(c, 2u);
+  const double own = L.px[3 * At.ia + comp];
+  const bool last = c == 3;
+  double sum = 0.0;  // component c of the force; lane 3: the energy
+  // four entries of one group, added in order; term(dx, dy, dz, e) is the pair's coefficient
+  auto group = [&](uint2 w, auto&& term) {
+    const uint32_t j[4] = {w.x & 0xffffu, w.x >> 16, w.y & 0xffffu, w.y >> 16};
+    const uint32_t mine = ((c & 2u) ? w.y : w.x) >> (16u * (c & 1u)) & 0xffffu;
+    const double* const q = L.px + 3 * mine;
+    Coef e = 0;
+    const Coef coef = term(q[0] - ax, q[1] - ay, q[2] - az, e);
+    double d[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      d[u] = L.px[3 * j[u] + comp] - own;
+      if (ENERGY && last) d[u] = 1.0;
+    }
+    Coef k[4] = {quad_get<0>(coef), quad_get<1>(coef), quad_get<2>(coef), quad_get<3>(coef)};
+    if (ENERGY) {
+      const Coef ke[4] = {quad_get<0>(e), quad_get<1>(e), quad_get<2>(e), quad_get<3>(e)};
+#pragma unroll
+      for (int u = 0; u < 4; u++) k[u] = last ? ke[u] : k[u];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      if (MIXED) sum = fma((double)k[u], d[u], sum);
+      else sum += (double)k[u] * d[u];
+    }
+  };
+  auto walk = [&](auto&& term) {
+    for (uint32_t q0 = 0; q0 < nmax; q0 += kAhead * kQuadBatch) {
+#pragma unroll
+      for (uint32_t k = 0; k < kAhead; k++) {
+        if (q0 + k * kQuadBatch >= nmax) break;
+        const uint2 w = ahead[k];
+        const uint32_t nq = q0 + (k + kAhead) * kQuadBatch;
+        if (nq < nmax) ahead[k] = load_list_group(lst + (size_t)(nq >> 2) * T);
+        group(make_uint2(quad_get<0>(w.x), quad_get<0>(w.y)), term);
+        group(make_uint2(quad_get<1>(w.x), quad_get<1>(w.y)), term);
+        group(make_uint2(quad_get<2>(w.x), quad_get<2>(w.y)), term);
+        group(make_uint2(quad_get<3>(w.x), quad_get<3>(w.y)), term);
+      }
+    }
+  };
+  if constexpr (MIXED) {
+    walk([&](double dx, double dy, double dz, float& e) { return lj_term_mixed<ENERGY>(lj, dx, dy, dz, e); });
+  } else {
+    PairRange rng;
+    walk([&](double dx, double dy, double dz, double& e) { return lj_term_fp64<ENERGY>(lj, dx, dy, dz, rng, e); });
+    if (__builtin_expect(__any(lj.any != 0u || rng.outside()), 0)) {  // as in compute_pair_brick_body
+      sum = 0.0;
+#pragma unroll
+      for (uint32_t k = 0; k < kAhead; k++)
+        ahead[k] = k * kQuadBatch < bp.cap ? load_list_group(lst + (size_t)(4 * k) * T) : make_uint2(0u, 0u);
+      walk([&](double dx, double dy, double dz, double& e) { return lj_term_fp64_any<ENERGY>(lj, dx, dy, dz, e); });
+    }
+  }
+  bool over = false;
+  if (At.live) {
+    const uint32_t s = At.slot;
+    if (!NEXT && last) A.ep[s] = (ACCUM ? A.ep[s] : 0.0) + sum;
+    double a = 0.0 + sum;
+    if (!NEXT && !last) {
+      double* const f = c == 0 ? A.fx : c == 1 ? A.fy : A.fz;
+      a = (ACCUM ? f[s] : 0.0) + sum;
+      f[s] = a;
+    }
+    if (EPI != EPI_NONE) {
+      double x = own;  // the next position's component; lane 3: the type
+      double dd = 0.0;
+      if (!last) {
+        double* const vel = c == 0 ? A.vx : c == 1 ? A.vy : A.vz;
+        double u = vel[s] + a * dth;
+        if (NEXT) {
+          x += u * nx.dt + a * nx.dt2;
+          u += a * dth;
+          const int ri = (int)(At.rc % (uint32_t)bp.RX), rj = (int)((At.rc / (uint32_t)bp.RX) % (uint32_t)bp.RY),
+                    rk = (int)(At.rc / ((uint32_t)bp.RX * (uint32_t)bp.RY));
+          const double o = c == 0 ? g.ox : c == 1 ? g.oy : g.oz;
+          const int loc = c == 0 ? P.gi0 - 1 + ri : c == 1 ? P.gj0 - 1 + rj : P.gk0 - 1 + rk;
+          dd = x - restore_u32_double(nx.backup[3 * (size_t)s + c], cell_origin(o, g.gl, loc, g.cs), g.cs);
+        }
+        vel[s] = u;
+      } else if (NEXT) {
+        x = reinterpret_cast<const double*>(r)[4 * (size_t)s + 3];
+      }
+      if (NEXT) {
+        reinterpret_cast<double*>(nx.r_next)[4 * (size_t)s + c] = x;
+        // particle_displ_over, counted once an atom (the quad's lanes are all here)
+        const double d0 = quad_get<0>(dd), d1 = quad_get<1>(dd), d2 = quad_get<2>(dd);
+        over = c == 0 && ((d0 * d0 + d1 * d1) + d2 * d2) >= nx.thr2;
+      }
+    }
+  }
+  if (NEXT) wave_group_count_add(over, nx.count, L.wcnt);
+}
+
+template <bool MIXED, bool ACCUM, int EPI>
+__global__ void __launch_bounds__(1024) k_lj_quad_brick(Geom g, BrickParams bp, const double4* __restrict__ r,
+                                                        const uint32_t* __restrict__ cell_off, const uint32_t* __restrict__ cell_n,
+                                                        const uint16_t* __restrict__ blist, const uint32_t* __restrict__ bcnt, LJConst lj,
+                                                        PState A, double dth, NextStep nx) {
+  const uint32_t b = brick_of_block<MIXED>(bp);
+  if (b >= bp.nbricks) return;  // whole workgroup, before any barrier
+  lj_quad_brick_body<MIXED, ACCUM, EPI>(g, bp, b, r, cell_off, cell_n, blist, bcnt, lj, A, dth, nx);
+}
+
 // Any other force functor on brick lists (no fused epilogue): f += pairs (ACCUM, after
 // zero_particle_force).
 template <class F>
@@ -995,7 +1184,7 @@ __device__ __forceinline__ void ljmm_brick_body(const Geom& g, const BrickParams
     L.wcnt[1] = 0;
   }
   if (!brick_setup(g, bp, P, L, r, cell_off, cell_n, kPosF64)) return;
-  const LaneAtom At = lane_atom(bp, L);
+  const LaneAtom At = lane_atom(bp, L, threadIdx.x);
   const uint32_t t = threadIdx.x, T = bp.T;
   const uint32_t n = At.live ? bcnt[(size_t)b * T + t] : 0u;
   const uint32_t nmax = wave_max_b(n);
@@ -1207,7 +1396,7 @@ __global__ void __launch_bounds__(1024) k_brick_to_slots(Geom g, BrickParams bp,
   const BrickLds L = brick_lds(bp, lds);
   const BrickPos P = brick_pos(g, bp, b);
   if (!brick_setup(g, bp, P, L, nullptr, cell_off, cell_n, kPosNone)) return;
-  const LaneAtom A = lane_atom(bp, L);
+  const LaneAtom A = lane_atom(bp, L, threadIdx.x);
   if (!A.live) return;
   const uint32_t t = threadIdx.x, T = bp.T;
   const uint32_t n = min(bcnt[(size_t)b * T + t], bp.cap);
@@ -1237,6 +1426,7 @@ BrickParams brick_params(const Geom& g, int Bi, int Bj, int Bk) {
   bp.RZ = Bk + 2;
   bp.nrc = bp.RX * bp.RY * bp.RZ;
   bp.nbc = Bi * Bj * Bk;
+  bp.lanes = 1;
   return bp;
 }
 
@@ -1301,6 +1491,7 @@ hipError_t launch_nbh_brick(const Geom& g, BrickParams bp, const double4* r, con
                             uint32_t* bcnt, uint32_t* max_cnt, hipStream_t st) {
   const uint32_t lds = brick_layout(bp);
   hipError_t e;
+  if (bp.lanes != 1 && (half_symmetric || skip_ghosts || !prefilter)) return hipErrorInvalidValue;
   if (half_symmetric || skip_ghosts) {
     if (pc.nt > 0) return hipErrorInvalidValue;
     e = set_lds((const void*)k_nbh_brick_mask<true, false>, lds);
@@ -1310,10 +1501,10 @@ hipError_t launch_nbh_brick(const Geom& g, BrickParams bp, const double4* r, con
   } else if (pc.nt > 0 && prefilter) {
     BrickParams bq = bp;
     const uint32_t lds_b = brick_layout(bq, true, true);
-    e = set_lds((const void*)k_nbh_brick_mask<false, true, true>, lds_b);
+    auto* const fn = bq.lanes == kQuad ? k_nbh_brick_mask<false, true, true, kQuad> : k_nbh_brick_mask<false, true, true>;
+    e = set_lds((const void*)fn, lds_b);
     if (e != hipSuccess) return e;
-    k_nbh_brick_mask<false, true, true><<<kXcds * bq.per_xcd, bq.T, lds_b, st>>>(g, bq, r, cell_off, cell_n, max2, 0, 0, blist, bcnt,
-                                                                                max_cnt, pc);
+    fn<<<kXcds * bq.per_xcd, bq.T * bq.lanes, lds_b, st>>>(g, bq, r, cell_off, cell_n, max2, 0, 0, blist, bcnt, max_cnt, pc);
   } else if (pc.nt > 0) {
     e = set_lds((const void*)k_nbh_brick_mask<false, true>, lds);
     if (e != hipSuccess) return e;
@@ -1322,10 +1513,10 @@ hipError_t launch_nbh_brick(const Geom& g, BrickParams bp, const double4* r, con
   } else if (prefilter) {
     BrickParams bq = bp;  // the same bricks and lists, the prefilter's smaller LDS layout
     const uint32_t lds_b = brick_layout(bq, true);
-    e = set_lds((const void*)k_nbh_brick_mask<false, false, true>, lds_b);
+    auto* const fn = bq.lanes == kQuad ? k_nbh_brick_mask<false, false, true, kQuad> : k_nbh_brick_mask<false, false, true>;
+    e = set_lds((const void*)fn, lds_b);
     if (e != hipSuccess) return e;
-    k_nbh_brick_mask<false, false, true><<<kXcds * bq.per_xcd, bq.T, lds_b, st>>>(g, bq, r, cell_off, cell_n, max2, 0, 0, blist, bcnt,
-                                                                                 max_cnt, pc);
+    fn<<<kXcds * bq.per_xcd, bq.T * bq.lanes, lds_b, st>>>(g, bq, r, cell_off, cell_n, max2, 0, 0, blist, bcnt, max_cnt, pc);
   } else {
     e = set_lds((const void*)k_nbh_brick_mask<false, false>, lds);
     if (e != hipSuccess) return e;
@@ -1341,9 +1532,10 @@ template <bool MIXED, bool ACCUM, int EPI>
 static hipError_t ljb_launch(const Geom& g, const BrickParams& bp, uint32_t lds, const double4* r, const uint32_t* cell_off,
                              const uint32_t* cell_n, const uint16_t* blist, const uint32_t* bcnt, const LJConst& lj, const PState& A,
                              double dth, const NextStep& nx, hipStream_t st) {
-  hipError_t e = set_lds((const void*)k_lj_brick<MIXED, ACCUM, EPI, LJB_UNROLL>, lds);
+  auto* const fn = bp.lanes == kQuad ? k_lj_quad_brick<MIXED, ACCUM, EPI> : k_lj_brick<MIXED, ACCUM, EPI, LJB_UNROLL>;
+  hipError_t e = set_lds((const void*)fn, lds);
   if (e != hipSuccess) return e;
-  k_lj_brick<MIXED, ACCUM, EPI, LJB_UNROLL><<<kXcds * bp.per_xcd, bp.T, lds, st>>>(g, bp, r, cell_off, cell_n, blist, bcnt, lj, A, dth, nx);
+  fn<<<kXcds * bp.per_xcd, bp.T * bp.lanes, lds, st>>>(g, bp, r, cell_off, cell_n, blist, bcnt, lj, A, dth, nx);
   return hipGetLastError();
 }
 

@@ -89,6 +89,7 @@ struct xnb_ctx {
   bool use_bricks = true;
   BrickParams bp{};
   int brick_dims[3] = {0, 0, 0};  // 0: choose automatically
+  int brick_lanes = 0;            // lanes per atom (1 or kQuad); 0: choose automatically
   DArr<uint16_t> blist;
   DArr<uint32_t> bcnt;
   bool slot_lists_current = false;  // nbr/nbr_cnt mirror the brick lists

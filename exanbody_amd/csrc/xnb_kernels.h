@@ -17,6 +17,8 @@ constexpr uint32_t kXcds = 8;
 // Brick lists are padded per wave to a multiple of this many entries with the region's
 // sentinel atom (far away, so every pair with it fails the cutoff test).
 constexpr uint32_t kListBatch = 8;
+// Lists of quad bricks (four lanes an atom) are padded per workgroup to a multiple of this many.
+constexpr uint32_t kQuad = 4, kQuadBatch = 16;
 
 struct BrickParams {
   int Bi, Bj, Bk;     // brick size in cells
@@ -25,7 +27,8 @@ struct BrickParams {
   int nrc, nbc;       // region cells, brick cells
   uint32_t nbricks;
   uint32_t per_xcd;  // bricks per XCD: workgroup i runs brick (i % 8) * per_xcd + i / 8
-  uint32_t T;     // threads per workgroup (>= brick atoms, nrc, nbc; multiple of 64)
+  uint32_t T;     // atoms a workgroup holds (>= brick atoms, nrc, nbc; multiple of 64)
+  uint32_t lanes;  // lanes per atom of the build and the LJ force (1 or kQuad): T * lanes threads
   uint32_t Rmax;  // largest region atom count
   uint32_t cap;   // list rows per brick slab
   uint32_t* status;  // device word: bit 0 set when a region exceeds Rmax, bit 1 when a brick exceeds T

@@ -229,6 +229,62 @@ __device__ inline void lj_pair_fp64_any(const LJConst& lj, const double4& ra, co
   if (ENERGY) te += in ? lj.eps4 * (ratio12 - ratio6) : 0.0;
 }
 
+// One pair's coefficient (f += coefficient * d) and energy, for the traversal that adds them up
+// elsewhere: what lj_batch_fp64, lj_pair_fp64_any and lj_pair_mixed multiply and add.
+template <bool ENERGY>
+__device__ inline double lj_term_fp64(const LJConst& lj, double dx, double dy, double dz, PairRange& rng, double& e) {
+  const double d2 = (dx * dx + dy * dy) + dz * dz;
+  rng.add(d2);
+  const uint32_t hi = d2 <= lj.rc2 ? (uint32_t)__double2hiint(d2) : 0x7e700000u;
+  const double inv_r = inv_sqrt_normal(__hiloint2double((int)hi, __double2loint(d2)));
+  const double ratio = lj.sigma * inv_r;
+  const double ratio2 = ratio * ratio;
+  const double ratio6 = ratio2 * ratio2 * ratio2;
+  const double ratio12 = ratio6 * ratio6;
+  double de = (lj.m24eps * fma(2., ratio12, -ratio6)) * inv_r;
+  de *= inv_r;
+  if (ENERGY) e = lj.eps4 * (ratio12 - ratio6);
+  return de;
+}
+template <bool ENERGY>
+__device__ inline double lj_term_fp64_any(const LJConst& lj, double dx, double dy, double dz, double& e) {
+  const double d2 = (dx * dx + dy * dy) + dz * dz;
+  const bool in = d2 > 0.0 && d2 <= lj.rc2;
+  const double inv_r = 1.0 / sqrt(in ? d2 : 1.0);
+  const double ratio = lj.sigma * inv_r;
+  const double ratio2 = ratio * ratio;
+  const double ratio6 = ratio2 * ratio2 * ratio2;
+  const double ratio12 = ratio6 * ratio6;
+  double de = (lj.m24eps * (2. * ratio12 - ratio6)) * inv_r;
+  de *= inv_r;
+  if (ENERGY) e = in ? lj.eps4 * (ratio12 - ratio6) : 0.0;
+  return in ? de : 0.0;
+}
+template <bool ENERGY>
+__device__ inline float lj_term_mixed(const LJConst& lj, double dx, double dy, double dz, float& e) {
+  const double d2 = fma(dz, dz, fma(dy, dy, dx * dx));
+  const bool in = d2 > 0.0 && d2 <= lj.rc2;
+  const float inv_r2 = in ? __builtin_amdgcn_rcpf((float)d2) : 0.0f;
+  float s6;
+  const float c = lj_coef_f32(inv_r2, lj.sigma6f, lj.m24epsf, s6);
+  if (ENERGY) e = lj_energy_f32(s6, lj.eps4f);
+  return c;
+}
+
+// Lane U's value in every lane of its group of four.
+template <int U>
+__device__ inline uint32_t quad_get(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, U * 0x55, 0xf, 0xf, true);
+}
+template <int U>
+__device__ inline float quad_get(float x) {
+  return __uint_as_float(quad_get<U>(__float_as_uint(x)));
+}
+template <int U>
+__device__ inline double quad_get(double x) {
+  return __hiloint2double((int)quad_get<U>((uint32_t)__double2hiint(x)), (int)quad_get<U>((uint32_t)__double2loint(x)));
+}
+
 // ------------------------------------------------------------------ force functors
 // LennardJonesForceFunctor (lennard_jones.cu:59-125) for the pair traversal: the buffer-less
 // form (lennard_jones.cu:105-124, plus the per-atom energy field) and the batched form the
