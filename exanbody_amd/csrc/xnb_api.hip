@@ -329,6 +329,9 @@ constexpr uint32_t kQuadAtoms = 32768;
 // idle CUs cost more than the larger staged share of smaller bricks.  60,000-atom slab,
 // force: 112 bricks 70 us, 196 bricks 45 us; 131,072 atoms: 250 bricks 36 us, 500 bricks 41 us.
 constexpr uint32_t kEnoughBricks = 192;
+// Shapes are looked at together up to this many bricks: some microseconds, against about 25 for
+// another launch and read-back.
+constexpr uint32_t kStatBricks = 8192;
 
 // Brick dims, lanes, T and Rmax for the current cell occupancy; NOT_APPLICABLE if nothing fits LDS.
 int choose_bricks(xnb_ctx* c, uint32_t cap, bool quads, BrickParams& out) {
@@ -353,28 +356,41 @@ int choose_bricks(xnb_ctx* c, uint32_t cap, bool quads, BrickParams& out) {
     for (const auto& d : quad) add(d, kQuad, &d == &quad[3]);
   for (int q = 0; q < 9; q++)
     if ((q != 1 && q != 2) || c->batch_shapes) add(wide[q], 1u, c->batch_shapes || q == 8);
-  for (int q = 0; q < ncand; q++) {
-    BrickParams bp = brick_params(c->g, cand[q].dims[0], cand[q].dims[1], cand[q].dims[2]);
-    if (!cand[q].any && bp.nbricks < kEnoughBricks) continue;
-    HIPCHK(c, hipMemsetAsync(c->u32s.p + 3, 0, 2 * sizeof(uint32_t), c->st));
-    launch_brick_stats(c->g, bp, c->cell_n.p, c->u32s.p + 3, c->st);
+  for (int q = 0; q < ncand;) {
+    // the next shapes, as many at once as are cheap to look at (a large box's first one fits)
+    BrickShapes sh{};
+    uint32_t bricks = 0;
+    for (; q < ncand && sh.n < kStatShapes; q++) {
+      BrickParams bp = brick_params(c->g, cand[q].dims[0], cand[q].dims[1], cand[q].dims[2]);
+      if (!cand[q].any && bp.nbricks < kEnoughBricks) continue;
+      if (sh.n && bricks + bp.nbricks > kStatBricks) break;
+      bp.lanes = cand[q].lanes;
+      bricks += bp.nbricks;
+      sh.shape[sh.n++] = bp;
+    }
+    if (!sh.n) break;
+    HIPCHK(c, hipMemsetAsync(c->u32s.p + 16, 0, 2 * kStatShapes * sizeof(uint32_t), c->st));
+    launch_brick_stats(c->g, sh, c->cell_n.p, c->u32s.p + 16, c->st);
     HIPCHK(c, hipGetLastError());
-    HIPCHK(c, hipMemcpyAsync(c->h_u32, c->u32s.p + 3, 2 * sizeof(uint32_t), hipMemcpyDeviceToHost, c->st));
-    HIPCHK(c, hipStreamSynchronize(c->st));
-    // head room for later rebuilds of a batched box (brick_margin > 1): atoms may regroup
-    const uint32_t nb_max = (uint32_t)std::ceil(c->h_u32[0] * c->brick_margin);
-    const uint32_t r_max = (uint32_t)std::ceil(c->h_u32[1] * c->brick_margin);
-    uint32_t T = std::max<uint32_t>({nb_max, (uint32_t)bp.nrc, (uint32_t)bp.nbc, 64u});
-    T = (T + 63) / 64 * 64;
-    bp.lanes = cand[q].lanes;
-    if (T * bp.lanes > 1024 || r_max >= 65535u) continue;
-    bp.T = T;
-    bp.Rmax = std::max<uint32_t>(r_max, 1u);
-    bp.cap = cap;
-    bp.status = c->u32s.p + 6;
-    if (brick_layout(bp) > c->lds_limit) continue;
-    out = bp;
-    return XNB_OK;
+    uint32_t most[2 * kStatShapes];
+    int e;
+    if ((e = read_u32(c, c->u32s.p + 16, most, 2 * kStatShapes))) return e;
+    for (uint32_t k = 0; k < sh.n; k++) {
+      BrickParams& bp = sh.shape[k];
+      // head room for later rebuilds of a batched box (brick_margin > 1): atoms may regroup
+      const uint32_t nb_max = (uint32_t)std::ceil(most[2 * k] * c->brick_margin);
+      const uint32_t r_max = (uint32_t)std::ceil(most[2 * k + 1] * c->brick_margin);
+      uint32_t T = std::max<uint32_t>({nb_max, (uint32_t)bp.nrc, (uint32_t)bp.nbc, 64u});
+      T = (T + 63) / 64 * 64;
+      if (T * bp.lanes > 1024 || r_max >= 65535u) continue;
+      bp.T = T;
+      bp.Rmax = std::max<uint32_t>(r_max, 1u);
+      bp.cap = cap;
+      bp.status = c->u32s.p + 6;
+      if (brick_layout(bp) > c->lds_limit) continue;
+      out = bp;
+      return XNB_OK;
+    }
   }
   return NOT_APPLICABLE;
 }
@@ -597,7 +613,7 @@ int xnb_create(xnb_ctx** out, const xnb_domain* d, int device) {
     return fail(nullptr, XNB_E_HIP, "stream creation failed");
   }
   int e;
-  if ((e = set_geometry(c, 0.0)) || (e = dalloc(c, c->u32s, 16)) || (e = dalloc(c, c->u64s, 8)) || (e = dalloc(c, c->red_out, 2))) {
+  if ((e = set_geometry(c, 0.0)) || (e = dalloc(c, c->u32s, 32)) || (e = dalloc(c, c->u64s, 8)) || (e = dalloc(c, c->red_out, 2))) {
     xnb_destroy(c);
     return e;
   }

@@ -368,23 +368,47 @@ __device__ inline LaneAtom lane_atom(const BrickParams& bp, const BrickLds& L, u
 }
 
 // ------------------------------------------------------------------ statistics
-// per brick: atoms in the brick and in its region -> maxima
-__global__ void k_brick_stats(Geom g, BrickParams bp, const uint32_t* __restrict__ cell_n, uint32_t* __restrict__ out) {
-  const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= bp.nbricks) return;
-  const BrickPos P = brick_pos(g, bp, b);
-  uint32_t R = 0, nb = 0;
-  for (int rk = 0; rk <= P.nk + 1; rk++)
-    for (int rj = 0; rj <= P.nj + 1; rj++)
-      for (int ri = 0; ri <= P.ni + 1; ri++) {
-        const int gi = P.gi0 - 1 + ri, gj = P.gj0 - 1 + rj, gk = P.gk0 - 1 + rk;
-        if (gi >= g.di || gj >= g.dj || gk >= g.dk) continue;
-        const uint32_t n = cell_n[cell_index(g, gi, gj, gk)];
-        R += n;
-        if (ri >= 1 && ri <= P.ni && rj >= 1 && rj <= P.nj && rk >= 1 && rk <= P.nk) nb += n;
-      }
-  atomicMax(&out[0], nb);
-  atomicMax(&out[1], R);
+// Largest brick and region atom counts of up to kStatShapes brick shapes: out[2 k] and
+// out[2 k + 1] of shape k (0 on entry).  Bound by latency (a few hundred bricks): a wave takes a
+// brick, its lanes the region's cells, so the counts arrive in two or three loads instead of one
+// after another (one thread a brick: 29 us a launch at 250 bricks of 144 region cells, 18 us at
+// a dozen), and one launch with one read-back serves all the shapes that are tried.
+__global__ void __launch_bounds__(256) k_brick_stats(Geom g, BrickShapes sh, const uint32_t* __restrict__ cell_n,
+                                                     uint32_t* __restrict__ out) {
+  __shared__ uint32_t wmax[4][2];
+  const BrickParams bp = sh.shape[blockIdx.y];
+  const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
+  uint32_t nb_max = 0, R_max = 0;
+  for (uint32_t b = 4 * blockIdx.x + w; b < bp.nbricks; b += 4 * gridDim.x) {
+    const BrickPos P = brick_pos(g, bp, b);
+    uint32_t R = 0, nb = 0;
+    for (uint32_t c = lane; c < (uint32_t)bp.nrc; c += 64) {
+      const int ri = (int)(c % (uint32_t)bp.RX), rj = (int)((c / (uint32_t)bp.RX) % (uint32_t)bp.RY),
+                rk = (int)(c / ((uint32_t)bp.RX * (uint32_t)bp.RY));
+      const int gi = P.gi0 - 1 + ri, gj = P.gj0 - 1 + rj, gk = P.gk0 - 1 + rk;
+      if (ri > P.ni + 1 || rj > P.nj + 1 || rk > P.nk + 1 || gi >= g.di || gj >= g.dj || gk >= g.dk) continue;
+      const uint32_t n = cell_n[cell_index(g, gi, gj, gk)];
+      R += n;
+      if (ri >= 1 && ri <= P.ni && rj >= 1 && rj <= P.nj && rk >= 1 && rk <= P.nk) nb += n;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      R += (uint32_t)__shfl_xor((int)R, o, 64);
+      nb += (uint32_t)__shfl_xor((int)nb, o, 64);
+    }
+    nb_max = max(nb_max, nb);
+    R_max = max(R_max, R);
+  }
+  if (lane == 0) {
+    wmax[w][0] = nb_max;
+    wmax[w][1] = R_max;
+  }
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    uint32_t m = 0;
+    for (int q = 0; q < 4; q++) m = max(m, wmax[q][threadIdx.x]);
+    if (m) atomicMax(&out[2 * blockIdx.y + threadIdx.x], m);
+  }
 }
 
 // ------------------------------------------------------------------ build
@@ -1459,8 +1483,10 @@ uint32_t brick_layout(BrickParams& bp, bool f32_build, bool f32_types) {
   return align8(o);
 }
 
-void launch_brick_stats(const Geom& g, const BrickParams& bp, const uint32_t* cell_n, uint32_t* out, hipStream_t st) {
-  k_brick_stats<<<(bp.nbricks + 255) / 256, 256, 0, st>>>(g, bp, cell_n, out);
+void launch_brick_stats(const Geom& g, const BrickShapes& sh, const uint32_t* cell_n, uint32_t* out, hipStream_t st) {
+  uint32_t most = 0;
+  for (uint32_t k = 0; k < sh.n; k++) most = std::max(most, sh.shape[k].nbricks);
+  k_brick_stats<<<dim3(std::min((most + 3) / 4, 1024u), sh.n), 256, 0, st>>>(g, sh, cell_n, out);
 }
 
 // Brick kernels keep all their LDS in the dynamic block, which then starts at LDS address 0:

@@ -223,7 +223,13 @@ BrickParams brick_params(const Geom& g, int Bi, int Bj, int Bk);
 // neighbour build's (FP32 positions; types only with f32_types, for per-pair radii)
 uint32_t brick_layout(BrickParams& bp, bool f32_build = false, bool f32_types = false);
 uint32_t brick_list_granule();
-void launch_brick_stats(const Geom& g, const BrickParams& bp, const uint32_t* cell_n, uint32_t* out, hipStream_t st);
+// brick shapes whose occupancy is looked at together; out: 2 words a shape, 0 on entry
+constexpr uint32_t kStatShapes = 4;
+struct BrickShapes {
+  uint32_t n;
+  BrickParams shape[kStatShapes];
+};
+void launch_brick_stats(const Geom& g, const BrickShapes& sh, const uint32_t* cell_n, uint32_t* out, hipStream_t st);
 // prefilter: the unfiltered builds test candidates in FP32 with an FP64 band (the same lists)
 hipError_t launch_nbh_brick(const Geom& g, BrickParams bp, const double4* r, const uint32_t* cell_off, const uint32_t* cell_n, double max2,
                             const PairCut& pc, int half_symmetric, int skip_ghosts, bool prefilter, uint16_t* blist, uint32_t* bcnt,
