@@ -395,6 +395,15 @@ int choose_bricks(xnb_ctx* c, uint32_t cap, bool quads, BrickParams& out) {
   return NOT_APPLICABLE;
 }
 
+void bind_regions(xnb_ctx* c, BrickParams& bp, bool derive) {
+  bp.reg = c->breg.p;
+  bp.lane = c->blane.p;
+  bp.derive = derive && c->N < kDeriveSlots ? 1u : 0u;
+  bp.n_inner = c->N;
+  bp.ghost_src = c->ghost_src.p;
+  bp.ghost_shift = c->ghost_shift.p;
+}
+
 int op_nbh_brick(xnb_ctx* c, double nbh_dist, const xnb_chunk_neighbors_config& cfg, const PairCut& pc) {
   const double max2 = nbh_dist * nbh_dist;
   int e;
@@ -407,6 +416,9 @@ int op_nbh_brick(xnb_ctx* c, double nbh_dist, const xnb_chunk_neighbors_config& 
     if ((e = choose_bricks(c, cap, quads, bp))) return e;
     if ((e = dalloc(c, c->blist, (size_t)bp.nbricks * bp.cap * bp.T))) return e;
     if ((e = dalloc(c, c->bcnt, (size_t)bp.nbricks * bp.T))) return e;
+    if ((e = dalloc(c, c->breg, brick_reg_words(bp)))) return e;
+    if ((e = dalloc(c, c->blane, (size_t)bp.nbricks * bp.T))) return e;
+    bind_regions(c, bp, c->derive_ghosts);
     HIPCHK(c, hipMemsetAsync(c->u32s.p + 2, 0, sizeof(uint32_t), c->st));
     HIPCHK(c, hipMemsetAsync(c->u32s.p + 6, 0, sizeof(uint32_t), c->st));
     tstart(c, XNB_TIMER_NBH);
@@ -496,7 +508,7 @@ int launch_force(xnb_ctx* c, int precision, bool accum, bool push, bool ghost, d
                  const NextStep* next = nullptr) {
   if (c->list_kind == 1 && !ghost) {
     const int epi = next ? EPI_NEXT : (push ? EPI_KICK : EPI_NONE);
-    hipError_t he = launch_lj_brick(precision, accum, epi, c->g, c->bp, c->A, c->cell_off.p, c->cell_n.p, c->blist.p, c->bcnt.p, eps,
+    hipError_t he = launch_lj_brick(precision, accum, epi, c->g, c->bp, c->A, c->blist.p, c->bcnt.p, eps,
                                     sigma, rcut, dth, next, c->st);
     if (he != hipSuccess) return fail(c, XNB_E_HIP, std::string("brick LJ kernel: ") + hipGetErrorString(he));
     return XNB_OK;
@@ -514,7 +526,7 @@ int launch_force(xnb_ctx* c, int precision, bool accum, bool push, bool ghost, d
 int launch_force_multimat(xnb_ctx* c, int precision, const LJMulti& mm, int ntypes, double dth, const NextStep* next) {
   if (c->list_kind == 1) {
     const int epi = next ? EPI_NEXT : EPI_KICK;
-    hipError_t he = launch_ljmm_brick(precision, ntypes, epi, c->g, c->bp, c->A, c->cell_off.p, c->cell_n.p, c->blist.p, c->bcnt.p, mm,
+    hipError_t he = launch_ljmm_brick(precision, ntypes, epi, c->g, c->bp, c->A, c->blist.p, c->bcnt.p, mm,
                                       dth, next, c->st);
     if (he != hipSuccess) return fail(c, XNB_E_HIP, std::string("brick multimat kernel: ") + hipGetErrorString(he));
     return XNB_OK;
@@ -534,6 +546,7 @@ int full_update(xnb_ctx* c, bool forces, const PairCut* pc) {
   if ((e = op_amr(c, kSubGridDensity, forces))) return e;
   if ((e = op_backup(c))) return e;
   if ((e = op_ghost_all(c, true, forces))) return e;
+  c->derive_ghosts = true;
   xnb_chunk_neighbors_config cfg{1, 0, 0, 0, 0};
   return op_nbh(c, c->nbh_dist_lab, cfg, 0, pc);
 }
@@ -545,6 +558,19 @@ int ensure_full_lists(xnb_ctx* c) {
   if (!c->lists_valid || !c->lists_pruned) return XNB_OK;
   xnb_chunk_neighbors_config cfg{1, 0, 0, 0, 0};
   return op_nbh(c, c->nbh_dist_lab, cfg, 0, nullptr);
+}
+
+// Brick lists' reg words name ghosts the way the caller needs them.
+int ensure_regions(xnb_ctx* c, bool derive) {
+  c->derive_ghosts = derive;
+  if (!c->lists_valid || c->list_kind != 1) return XNB_OK;
+  BrickParams bp = c->bp;
+  bind_regions(c, bp, derive);
+  if (bp.derive == c->bp.derive) return XNB_OK;
+  const hipError_t he = launch_brick_regions(c->g, bp, c->cell_off.p, c->cell_n.p, c->st);
+  if (he != hipSuccess) return fail(c, XNB_E_HIP, std::string("brick regions: ") + hipGetErrorString(he));
+  c->bp = bp;
+  return XNB_OK;
 }
 
 int check_ctx(xnb_ctx* c) {
@@ -1121,6 +1147,7 @@ int xnb_lennard_jones_force(xnb_ctx* c, const xnb_lj_params* p, double rcut, int
   if (!p || (precision != XNB_PRECISION_FP64 && precision != XNB_PRECISION_MIXED)) return fail(c, XNB_E_ARG, "bad LJ arguments");
   if (!c->lists_valid) return fail(c, XNB_E_STATE, "no neighbour lists (chunk_neighbors)");
   if ((e = ensure_full_lists(c))) return e;
+  if ((e = ensure_regions(c, false))) return e;
   c->last_rcut = rcut;
   tstart(c, XNB_TIMER_FORCE);
   e = launch_force(c, precision, true, false, ghost != 0, p->epsilon, p->sigma, rcut, 0.0);
@@ -1136,13 +1163,12 @@ int xnb_lennard_jones_force_multimat(xnb_ctx* c, int ntypes, const double* eps, 
   if ((e = check_ctx(c))) return e;
   if (ntypes <= 0 || ntypes > 4 || !eps || !sigma || !rcut) return fail(c, XNB_E_ARG, "bad multimat arguments (1..4 types)");
   if (!c->lists_valid) return fail(c, XNB_E_STATE, "no neighbour lists");
-  if ((e = ensure_full_lists(c))) return e;
+  if ((e = ensure_full_lists(c)) || (e = ensure_regions(c, false))) return e;
   LJMulti mm;
   if (make_lj_multi(ntypes, eps, sigma, rcut, mm)) return fail(c, XNB_E_ARG, "too many type pairs");
   tstart(c, XNB_TIMER_FORCE);
   if (c->list_kind == 1) {
-    hipError_t he = launch_ljmm_brick(precision, ntypes, EPI_NONE, c->g, c->bp, c->A, c->cell_off.p, c->cell_n.p, c->blist.p, c->bcnt.p,
-                                      mm, 0.0, nullptr, c->st);
+    hipError_t he = launch_ljmm_brick(precision, ntypes, EPI_NONE, c->g, c->bp, c->A, c->blist.p, c->bcnt.p, mm, 0.0, nullptr, c->st);
     if (he != hipSuccess) return fail(c, XNB_E_HIP, std::string("brick multimat kernel: ") + hipGetErrorString(he));
   } else {
     if ((e = ensure_slot_lists(c))) return e;
@@ -1161,7 +1187,7 @@ int xnb_gravitational_force(xnb_ctx* c, double G, int ntypes, const double* type
   if (ntypes < 1 || ntypes > kGravityTypes || !type_mass || !(rcut > 0.0))
     return fail(c, XNB_E_ARG, "bad gravitational_force arguments (1..16 types, rcut > 0)");
   if (!c->lists_valid) return fail(c, XNB_E_STATE, "no neighbour lists (chunk_neighbors)");
-  if ((e = ensure_full_lists(c))) return e;
+  if ((e = ensure_full_lists(c)) || (e = ensure_regions(c, false))) return e;
   const uint32_t n_atoms = ghost ? c->N + c->G : c->N;
   // every type indexes the mass table (the reference reads m_type_mass[type] unchecked)
   HIPCHK(c, hipMemsetAsync(c->u32s.p + 9, 0, sizeof(uint32_t), c->st));
@@ -1176,7 +1202,7 @@ int xnb_gravitational_force(xnb_ctx* c, double G, int ntypes, const double* type
   const double rc2 = rcut * rcut;
   tstart(c, XNB_TIMER_FORCE);
   if (c->list_kind == 1 && !ghost) {
-    hipError_t he = launch_gravity_brick(c->g, c->bp, c->A, c->cell_off.p, c->cell_n.p, c->blist.p, c->bcnt.p, gf, rc2, c->st);
+    hipError_t he = launch_gravity_brick(c->g, c->bp, c->A, c->blist.p, c->bcnt.p, gf, rc2, c->st);
     if (he != hipSuccess) return fail(c, XNB_E_HIP, std::string("brick gravitational kernel: ") + hipGetErrorString(he));
   } else {
     if ((e = ensure_slot_lists(c))) return e;
@@ -1320,6 +1346,7 @@ int run_loop(xnb_ctx* c, xnb_run_params* p, const LJMulti* mm, int ntypes, const
   // lists pruned by another run's radii: start from full lists
   if (c->lists_pruned && (!mm || std::memcmp(&pc, &c->pc_used, sizeof(PairCut)) != 0))
     if ((e = ensure_full_lists(c))) return e;
+  if ((e = ensure_regions(c, true))) return e;
   c->pc_used = pc;
   const double dt = p->dt * 1.0, dt2 = dt * dt * 0.5, dth = p->dt * 0.5;
   const double thr2 = c->max_displ * c->max_displ;
@@ -1353,7 +1380,9 @@ int run_loop(xnb_ctx* c, xnb_run_params* p, const LJMulti* mm, int ntypes, const
       if ((e = full_update(c, false, mm ? &pc : nullptr))) return e;  // f, ep: overwritten by this step's force kernel
       p->n_rebuilds++;
       if (interval) rebuilt[(size_t)step - 1] = 1;
-    } else {
+    } else if (step == p->steps || c->list_kind != 1 || !c->bp.derive) {
+      // ghost_update_r: the force of brick lists places ghosts by their sources, so only the
+      // positions a run leaves behind are refreshed (131,072 atoms: 4.7 us of a 40 us step)
       tstart(c, XNB_TIMER_GHOST);
       launch_ghost_update_r(c->g, c->N, c->G, c->A.r, c->ghost_src.p, c->ghost_shift.p, c->st);
       tstop(c);

@@ -167,6 +167,7 @@ void frame_from_ctx(xnb_batch* B, int i, const xnb_run_params& p) {
   f.bp.status = B->dwords.p + 4 * (size_t)i;
   f.bpn = f.bp;
   brick_layout(f.bpn, true);
+  brick_force_layout(f.bp, false);
   f.N = c->N;
   f.G = c->G;
   f.cap = (uint32_t)std::min<size_t>(c->cap, 0xffffffffu);
@@ -270,7 +271,8 @@ std::vector<uint32_t> bricks_table(const std::vector<int>& boxes, const std::vec
   return t;
 }
 
-uint32_t brick_lds_bytes(BrickParams bp, bool f32_build = false) { return brick_layout(bp, f32_build); }
+// LDS of a box's batched build (build) or force
+uint32_t brick_lds_bytes(BrickParams bp, bool build) { return build ? brick_layout(bp, true) : brick_force_layout(bp, false); }
 
 // Workgroups of a box's bricks that fit one CU at once (LDS bytes and the waves the
 // kernel's registers allow), 1..4.
@@ -486,6 +488,7 @@ int batch_box_nbh(xnb_batch* B, xnb_ctx* c) {
   int e = XNB_OK;
   bool done = false;
   c->batch_shapes = true;
+  c->derive_ghosts = true;
   if (B->brick_lds_cap < keep) {
     c->lds_limit = B->brick_lds_cap;
     e = op_nbh(c, c->nbh_dist_lab, cfg, 0);
@@ -644,7 +647,7 @@ int xnb_batch_attach(xnb_batch* B, xnb_ctx* c, const xnb_run_params* p, int* slo
   if ((e = ensure_capacity(c, (size_t)std::ceil((c->N + c->G) * B->slot_margin) + 256, (size_t)c->N + c->G))) return e;
   if ((e = batch_box_nbh(B, c))) return e;
   if (c->list_kind != 1) return bfail(B, XNB_E_STATE, "box geometry is not on the brick path (cell edge < nbh_dist)");
-  if (brick_lds_bytes(c->bp) > B->lds_limit) return bfail(B, XNB_E_CAPACITY, "box bricks exceed LDS");
+  if (brick_lds_bytes(c->bp, false) > B->lds_limit) return bfail(B, XNB_E_CAPACITY, "box bricks exceed LDS");
   // force-table entries hold the brick index in kWorkEpiShift bits
   if (c->bp.nbricks > kWorkBrickMask + 1) return bfail(B, XNB_E_CAPACITY, "box has too many bricks for a batch");
   if (hipStreamSynchronize(c->st) != hipSuccess) return bfail(B, XNB_E_HIP, "box stream");
@@ -764,6 +767,8 @@ int xnb_batch_step(xnb_batch* B, int nsteps, int* n_active) {
     std::vector<uint32_t> nG;
     for (int i : quiet) {
       BatchBox& bb = B->box[i];
+      // the force places ghosts by their sources: refreshed on a box's last step, for its reader
+      if (bb.f.bp.derive && bb.done + 1 < bb.steps) continue;
       if (bb.f.G > bb.ghost_span) bb.ghost_span = bb.f.G + bb.f.G / 10 + 1;
       if (bb.ghost_span) {
         q2.push_back(i);
@@ -941,7 +946,7 @@ int xnb_batch_autotune(xnb_batch* B, double* lds_frac_out) {
       ctx_from_frame(B, i, B->par);
       int e2;
       if ((e2 = batch_box_nbh(B, c))) return bfail(B, e2, std::string("autotune layout: ") + c->err);
-      if (c->list_kind != 1 || brick_lds_bytes(c->bp) > B->lds_limit || c->bp.nbricks > kWorkBrickMask + 1)
+      if (c->list_kind != 1 || brick_lds_bytes(c->bp, false) > B->lds_limit || c->bp.nbricks > kWorkBrickMask + 1)
         return bfail(B, XNB_E_CAPACITY, "autotune layout: a box left the batch's brick path");
       BHIP(B, hipStreamSynchronize(c->st));
       frame_from_ctx(B, i, bb.p);

@@ -212,13 +212,33 @@ __device__ inline uint32_t region_slot(const BrickParams& bp, const BrickLds& L,
   return L.roff[c] + (idx - L.rpref[c]);
 }
 
-// Region tables (+ positions per pos_mode) into LDS.  Needs nrc <= blockDim.x and
+// What the force kernels need of a brick's region is written down once, by the build: reg, one
+// word per region atom in LDS order (its slot; NONE for the Rmax + 1 - R words behind the last,
+// which take the list padding's sentinel), and lane, one word per atom of the brick (its LDS
+// index and brick cell).  A force launch then stages with two dependent loads and one barrier,
+// instead of reading the cell tables, two scans, a row table and a search per atom.  With
+// BrickParams::derive a ghost's word names its source and shift in place of its own slot, so the
+// force needs no refreshed ghost positions.
+static constexpr uint32_t kRegionSlotBits = 26;
+static constexpr uint32_t kRegionSlotMask = (1u << kRegionSlotBits) - 1u;
+static constexpr uint32_t kNoShift = 1u | 1u << 2 | 1u << 4;  // pack_shift(0, 0, 0)
+static_assert(kDeriveSlots == 1u << kRegionSlotBits, "slots that fit a word beside the shift code");
+
+__device__ inline uint32_t region_word(const BrickParams& bp, uint32_t slot) {
+  if (!bp.derive) return slot;
+  if (slot < bp.n_inner) return slot | kNoShift << kRegionSlotBits;
+  const uint32_t q = slot - bp.n_inner;
+  return bp.ghost_src[q] | bp.ghost_shift[q] << kRegionSlotBits;
+}
+__device__ inline uint32_t region_word_slot(const BrickParams& bp, uint32_t w) { return bp.derive ? w & kRegionSlotMask : w; }
+
+// Region tables (+ positions per pos_mode) into LDS, and the brick's reg words.  Needs nrc <= blockDim.x and
 // nbc <= blockDim.x.  Ends with a workgroup barrier.  Returns false (the same for every
 // thread, with bp.status flagged) when the region holds more than Rmax atoms or the brick
 // more than T, the sizes its LDS and lists were laid out for.
 __device__ inline bool brick_setup(const Geom& g, const BrickParams& bp, const BrickPos& P, const BrickLds& L,
                                    const double4* __restrict__ r, const uint32_t* __restrict__ cell_off,
-                                   const uint32_t* __restrict__ cell_n, int pos_mode) {
+                                   const uint32_t* __restrict__ cell_n, int pos_mode, uint32_t* __restrict__ reg = nullptr) {
   const uint32_t t = threadIdx.x;
   const bool f32 = pos_mode == kPosF32 || pos_mode == kPosF32N;
   if (f32 && t == 0) L.wcnt[0] = 0u;  // ordered before the max by the scan's barrier
@@ -288,12 +308,17 @@ __device__ inline bool brick_setup(const Geom& g, const BrickParams& bp, const B
     // Up to kStageRound region atoms per thread and round, every load issued before the first
     // LDS store: one memory round trip per round (a loop that stored each load before issuing
     // the next spent ~0.36 ms of a 0.94 ms mixed force launch at 8.4M atoms staging).
+    uint32_t slot0[kStageRound];  // the first round's slots
     for (uint32_t base = t; base < R; base += (uint32_t)kStageRound * blockDim.x) {
       double4 p[kStageRound];
 #pragma unroll
       for (int u = 0; u < kStageRound; u++) {
         const uint32_t idx = base + (uint32_t)u * blockDim.x;
-        if (idx < R) p[u] = r[region_slot(bp, L, idx)];
+        if (idx < R) {
+          const uint32_t slot = region_slot(bp, L, idx);
+          p[u] = r[slot];
+          if (base == t) slot0[u] = slot;
+        }
       }
       if (f32) {
 #pragma unroll
@@ -334,6 +359,18 @@ __device__ inline bool brick_setup(const Geom& g, const BrickParams& bp, const B
     }
     if (f32 && cmax) __hip_atomic_fetch_max(&L.wcnt[0], cmax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     __syncthreads();
+    // The reg words go out behind the last barrier (a barrier waits for stores: before it they
+    // cost the build of 8,388,608 atoms 0.2 of 2.6 ms) and past the caches, whose room the lists'
+    // scattered stores need.
+    if (reg) {
+#pragma unroll
+      for (int u = 0; u < kStageRound; u++) {
+        const uint32_t idx = t + (uint32_t)u * blockDim.x;
+        if (idx <= bp.Rmax) __builtin_nontemporal_store(idx < R ? region_word(bp, slot0[u]) : NONE, reg + idx);
+      }
+      for (uint32_t idx = t + (uint32_t)kStageRound * blockDim.x; idx <= bp.Rmax; idx += blockDim.x)
+        __builtin_nontemporal_store(idx < R ? region_word(bp, region_slot(bp, L, idx)) : NONE, reg + idx);
+    }
   }
   return true;
 }
@@ -344,6 +381,7 @@ struct LaneAtom {
   uint32_t p;     // index in cell
   uint32_t ia;    // LDS index
   uint32_t slot;  // global slot
+  uint32_t bc;    // brick cell
 };
 
 // atom t of the brick
@@ -355,9 +393,11 @@ __device__ inline LaneAtom lane_atom(const BrickParams& bp, const BrickLds& L, u
     A.p = 0;
     A.ia = 0;
     A.slot = 0;
+    A.bc = 0;
     return A;
   }
   const uint32_t bc = upper_index(L.bpref, (uint32_t)bp.nbc, t);
+  A.bc = bc;
   const int ci = (int)(bc % (uint32_t)bp.Bi), cj = (int)((bc / (uint32_t)bp.Bi) % (uint32_t)bp.Bj),
             ck = (int)(bc / ((uint32_t)bp.Bi * (uint32_t)bp.Bj));
   A.rc = (uint32_t)(((ck + 1) * bp.RY + cj + 1) * bp.RX + ci + 1);
@@ -365,6 +405,116 @@ __device__ inline LaneAtom lane_atom(const BrickParams& bp, const BrickLds& L, u
   A.ia = L.rpref[A.rc] + A.p;
   A.slot = L.roff[A.rc] + A.p;
   return A;
+}
+
+// ------------------------------------------------------------------ force staging
+// A lane's atom as the force kernels know it, from its lane and reg words.
+struct ForceAtom {
+  bool live;
+  uint32_t ia;    // LDS index
+  uint32_t slot;  // global slot
+  uint32_t bc;    // brick cell
+};
+__device__ inline uint32_t lane_word(const BrickParams& bp, uint32_t b, uint32_t t) {
+  return t < bp.T ? bp.lane[(size_t)b * bp.T + t] : NONE;
+}
+__device__ inline ForceAtom force_atom(const BrickParams& bp, uint32_t b, uint32_t w) {
+  ForceAtom A;
+  A.live = w != NONE;
+  A.ia = A.live ? w & 0xffffu : 0u;
+  A.bc = A.live ? w >> 16 : 0u;
+  A.slot = A.live ? region_word_slot(bp, bp.reg[(size_t)b * (bp.Rmax + 1u) + A.ia]) : 0u;
+  return A;
+}
+// grid coordinates of the atom's cell
+__device__ inline void force_cell(const BrickParams& bp, const BrickPos& P, uint32_t bc, int& gi, int& gj, int& gk) {
+  gi = P.gi0 + (int)(bc % (uint32_t)bp.Bi);
+  gj = P.gj0 + (int)((bc / (uint32_t)bp.Bi) % (uint32_t)bp.Bj);
+  gk = P.gk0 + (int)(bc / ((uint32_t)bp.Bi * (uint32_t)bp.Bj));
+}
+
+// Positions (and types, TYPES) of brick b's region into LDS by its reg words, the sentinel in
+// the rows behind the last atom.  Up to five atoms a thread and round, all of a round's
+// words loaded, then all its positions, then the LDS stores: with 4.2 region atoms a lane the
+// whole region comes in one round.  Four with types: five took the mixed multimat kernel
+// from 66 to 86 registers, one workgroup per CU.  No barrier: the caller's next one covers it.
+template <bool TYPES>
+__device__ __forceinline__ void stage_region(const Geom& g, const BrickParams& bp, uint32_t b, const double4* __restrict__ r,
+                                             const BrickLds& L) {
+  constexpr int kForceRound = TYPES ? 4 : 5;
+  const uint32_t rows = bp.Rmax + 1u;
+  const uint32_t* __restrict__ reg = bp.reg + (size_t)b * rows;
+  for (uint32_t base = threadIdx.x; base < rows; base += (uint32_t)kForceRound * blockDim.x) {
+    uint32_t w[kForceRound];
+    double x[kForceRound], y[kForceRound], z[kForceRound];
+    uint8_t ty[kForceRound];
+#pragma unroll
+    for (int u = 0; u < kForceRound; u++) {
+      const uint32_t idx = base + (uint32_t)u * blockDim.x;
+      w[u] = idx < rows ? __builtin_nontemporal_load(reg + idx) : NONE;
+    }
+#pragma unroll
+    for (int u = 0; u < kForceRound; u++) {
+      x[u] = y[u] = z[u] = 1e30;
+      ty[u] = 0;
+      if (w[u] != NONE) {
+        const double4* const q = r + region_word_slot(bp, w[u]);
+        x[u] = q->x;
+        y[u] = q->y;
+        z[u] = q->z;
+        if (TYPES) ty[u] = (uint8_t)q->w;
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kForceRound; u++) {
+      const uint32_t idx = base + (uint32_t)u * blockDim.x, code = w[u] >> kRegionSlotBits;
+      if (bp.derive && w[u] != NONE && code != kNoShift) {
+        // as ghost_update_r writes it
+        x[u] = shift_coord(x[u], (int)(code & 3u) - 1, g.ox, g.ex);
+        y[u] = shift_coord(y[u], (int)((code >> 2) & 3u) - 1, g.oy, g.ey);
+        z[u] = shift_coord(z[u], (int)((code >> 4) & 3u) - 1, g.oz, g.ez);
+      }
+      if (idx < rows) {
+        L.px[3 * idx] = x[u];
+        L.py[3 * idx] = y[u];
+        L.pz[3 * idx] = z[u];
+        if (TYPES) L.pt[idx] = ty[u];
+      }
+    }
+  }
+}
+
+// LDS of the force kernels (brick_force_layout): positions at address 0, types, the two words
+// of wave_group_count_add
+__device__ inline BrickLds force_lds(const BrickParams& bp, char* lds) {
+  BrickLds L{};
+  L.px = (double*)lds;
+  L.py = L.px + 1;
+  L.pz = L.px + 2;
+  L.pt = (uint8_t*)(lds + bp.off_type);
+  L.wcnt = (uint32_t*)(lds + bp.off_wsum);
+  return L;
+}
+
+// reg words of every brick again, for lists that stay (ghosts by slot or by source)
+__global__ void __launch_bounds__(1024) k_brick_regions(Geom g, BrickParams bp, const uint32_t* __restrict__ cell_off,
+                                                        const uint32_t* __restrict__ cell_n) {
+  extern __shared__ __align__(16) char lds[];
+  const uint32_t b = brick_of_block<true>(bp);
+  if (b >= bp.nbricks) return;  // whole workgroup, before any barrier
+  const BrickLds L = brick_lds(bp, lds);
+  const BrickPos P = brick_pos(g, bp, b);
+  if (!brick_setup(g, bp, P, L, nullptr, cell_off, cell_n, kPosNone)) return;
+  const uint32_t R = L.rpref[bp.nrc];
+  uint32_t* const reg = bp.reg + (size_t)b * (bp.Rmax + 1u);
+  for (uint32_t idx = threadIdx.x; idx <= bp.Rmax; idx += blockDim.x) {
+    if (idx >= R) {
+      reg[idx] = NONE;
+      continue;
+    }
+    const uint32_t c = upper_index(L.rpref, (uint32_t)bp.nrc, idx);
+    reg[idx] = region_word(bp, L.roff[c] + (idx - L.rpref[c]));
+  }
 }
 
 // ------------------------------------------------------------------ statistics
@@ -442,9 +592,12 @@ __device__ __forceinline__ void nbh_brick_body(const Geom& g, const BrickParams&
   extern __shared__ __align__(16) char lds[];
   const BrickLds L = brick_lds(bp, lds);
   const BrickPos P = brick_pos(g, bp, b);
-  if (!brick_setup(g, bp, P, L, r, cell_off, cell_n, PREF ? (PAIRWISE ? kPosF32N : kPosF32) : kPosF64)) return;
+  if (!brick_setup(g, bp, P, L, r, cell_off, cell_n, PREF ? (PAIRWISE ? kPosF32N : kPosF32) : kPosF64,
+                   bp.reg + (size_t)b * (bp.Rmax + 1u)))
+    return;
   const uint32_t t = threadIdx.x / LANES, T = bp.T;
   const LaneAtom A = lane_atom(bp, L, t);
+  if (threadIdx.x % LANES == 0 && t < T) __builtin_nontemporal_store(A.live ? A.ia | A.bc << 16 : NONE, bp.lane + (size_t)b * T + t);
   uint16_t* out = blist + (size_t)b * bp.cap * T;
   // every lane, live or not, tests against its own LDS atom when past the candidate cell's
   // end (A.ia = 0 for lanes without an atom), so d2 == 0 rejects those candidates
@@ -855,8 +1008,7 @@ __global__ void __launch_bounds__(1024) k_nbh_brick_mask(Geom g, BrickParams bp,
 // so no workgroup reads a position another one has already advanced.
 template <class F, bool ACCUM, int EPI, int U>
 __device__ __forceinline__ void compute_pair_brick_body(const Geom& g, const BrickParams& bp, uint32_t b,
-                                                        const double4* __restrict__ r, const uint32_t* __restrict__ cell_off,
-                                                        const uint32_t* __restrict__ cell_n, const uint16_t* __restrict__ blist,
+                                                        const double4* __restrict__ r, const uint16_t* __restrict__ blist,
                                                         const uint32_t* __restrict__ bcnt, const F& func, double rc2, const PState& A,
                                                         double dth, const NextStep& nx) {
   using Tr = ComputePairTraits<F>;
@@ -867,13 +1019,13 @@ __device__ __forceinline__ void compute_pair_brick_body(const Geom& g, const Bri
   constexpr bool BUFFERED = Tr::ComputeBufferCompatible;
   constexpr bool ENERGY = Tr::CentralEnergy && EPI != EPI_NEXT;
   extern __shared__ __align__(16) char lds[];
-  const BrickLds L = brick_lds(bp, lds);
-  const BrickPos P = brick_pos(g, bp, b);
-  if (EPI == EPI_NEXT && threadIdx.x == 0) {  // ordered before every wave's count by brick_setup's barriers
+  const BrickLds L = force_lds(bp, lds);
+  if (EPI == EPI_NEXT && threadIdx.x == 0) {  // ordered before every wave's count by the staging's barrier
     L.wcnt[0] = 0;
     L.wcnt[1] = 0;
   }
   const uint32_t t = threadIdx.x, T = bp.T;
+  const uint32_t lw = lane_word(bp, b, t);
   // U entries per batch = U / 4 eight-byte loads per lane; the next batch's loads are issued
   // before the current batch is computed.  Batches never pass cap (a multiple of U), and the
   // build padded every list of the wave with the sentinel up to a multiple of U.
@@ -887,8 +1039,9 @@ __device__ __forceinline__ void compute_pair_brick_body(const Geom& g, const Bri
   uint2 wn[W];
 #pragma unroll
   for (int w = 0; w < W; w++) wn[w] = t < T ? load_list_group(lst + (size_t)w * T) : make_uint2(0u, 0u);
-  if (!brick_setup(g, bp, P, L, r, cell_off, cell_n, kPosF64)) return;
-  const LaneAtom At = lane_atom(bp, L, threadIdx.x);
+  stage_region<!Tr::Batched>(g, bp, b, r, L);
+  __syncthreads();
+  const ForceAtom At = force_atom(bp, b, lw);
   const uint32_t n = At.live ? n_list : 0u;
   const uint32_t nmax = wave_max_b(n);
   double4 ra;
@@ -1006,9 +1159,9 @@ __device__ __forceinline__ void compute_pair_brick_body(const Geom& g, const Bri
         ux += ax * dth;
         uy += ay * dth;
         uz += az * dth;
-        const int ri = (int)(At.rc % (uint32_t)bp.RX), rj = (int)((At.rc / (uint32_t)bp.RX) % (uint32_t)bp.RY),
-                  rk = (int)(At.rc / ((uint32_t)bp.RX * (uint32_t)bp.RY));
-        over = displaced_ijk(g, p, P.gi0 - 1 + ri, P.gj0 - 1 + rj, P.gk0 - 1 + rk, nx.backup, s, nx.thr2);
+        int gi, gj, gk;
+        force_cell(bp, brick_pos(g, bp, b), At.bc, gi, gj, gk);
+        over = displaced_ijk(g, p, gi, gj, gk, nx.backup, s, nx.thr2);
       }
       __builtin_nontemporal_store(ux, &A.vx[s]);
       __builtin_nontemporal_store(uy, &A.vy[s]);
@@ -1020,12 +1173,11 @@ __device__ __forceinline__ void compute_pair_brick_body(const Geom& g, const Bri
 
 template <bool MIXED, bool ACCUM, int EPI, int U>
 __global__ void __launch_bounds__(1024) k_lj_brick(Geom g, BrickParams bp, const double4* __restrict__ r,
-                                                   const uint32_t* __restrict__ cell_off, const uint32_t* __restrict__ cell_n,
                                                    const uint16_t* __restrict__ blist, const uint32_t* __restrict__ bcnt,
                                                    LJConst lj, PState A, double dth, NextStep nx) {
   const uint32_t b = brick_of_block<MIXED>(bp);
   if (b >= bp.nbricks) return;  // whole workgroup, before any barrier
-  compute_pair_brick_body<LennardJonesForceFunctor<MIXED>, ACCUM, EPI, U>(g, bp, b, r, cell_off, cell_n, blist, bcnt,
+  compute_pair_brick_body<LennardJonesForceFunctor<MIXED>, ACCUM, EPI, U>(g, bp, b, r, blist, bcnt,
                                                                           LennardJonesForceFunctor<MIXED>{lj}, lj.rc2, A, dth, nx);
 }
 
@@ -1039,7 +1191,6 @@ __global__ void __launch_bounds__(1024) k_lj_brick(Geom g, BrickParams bp, const
 // consecutive groups of the list with one load each, kAhead such loads in flight.
 template <bool MIXED, bool ACCUM, int EPI>
 __device__ __forceinline__ void lj_quad_brick_body(const Geom& g, const BrickParams& bp, uint32_t b, const double4* __restrict__ r,
-                                                   const uint32_t* __restrict__ cell_off, const uint32_t* __restrict__ cell_n,
                                                    const uint16_t* __restrict__ blist, const uint32_t* __restrict__ bcnt,
                                                    const LJConst& lj, const PState& A, double dth, const NextStep& nx) {
   static_assert(!(EPI == EPI_NEXT && ACCUM), "a fused step starts the force from 0");
@@ -1047,14 +1198,14 @@ __device__ __forceinline__ void lj_quad_brick_body(const Geom& g, const BrickPar
   constexpr uint32_t kAhead = 4;
   using Coef = std::conditional_t<MIXED, float, double>;
   extern __shared__ __align__(16) char lds[];
-  const BrickLds L = brick_lds(bp, lds);
-  const BrickPos P = brick_pos(g, bp, b);
-  if (NEXT && threadIdx.x == 0) {  // ordered before every wave's count by brick_setup's barriers
+  const BrickLds L = force_lds(bp, lds);
+  if (NEXT && threadIdx.x == 0) {  // ordered before every wave's count by the staging's barrier
     L.wcnt[0] = 0;
     L.wcnt[1] = 0;
   }
   const uint32_t t = threadIdx.x / kQuad, c = threadIdx.x % kQuad, T = bp.T;
   const uint32_t n_list = bcnt[(size_t)b * T + t];
+  const uint32_t lw = lane_word(bp, b, t);
   // batch k of the list is the groups 4 k .. 4 k + 3, the lane's own is 4 k + c; every slab
   // holds whole batches (cap is a multiple of kQuadBatch)
   const uint2* const lst = reinterpret_cast<const uint2*>(blist + (size_t)b * bp.cap * T) + (size_t)c * T + t;
@@ -1062,8 +1213,9 @@ __device__ __forceinline__ void lj_quad_brick_body(const Geom& g, const BrickPar
 #pragma unroll
   for (uint32_t k = 0; k < kAhead; k++)
     ahead[k] = k * kQuadBatch < bp.cap ? load_list_group(lst + (size_t)(4 * k) * T) : make_uint2(0u, 0u);
-  if (!brick_setup(g, bp, P, L, r, cell_off, cell_n, kPosF64)) return;
-  const LaneAtom At = lane_atom(bp, L, t);
+  stage_region<false>(g, bp, b, r, L);
+  __syncthreads();
+  const ForceAtom At = force_atom(bp, b, lw);
   const uint32_t nmax = wave_max_b(At.live ? n_list : 0u);
   const double ax = L.px[3 * At.ia], ay = L.py[3 * At.ia], az = L.pz[3 * At.ia];
   const uint32_t comp = min(c, 2u);
@@ -1142,10 +1294,10 @@ __device__ __forceinline__ void lj_quad_brick_body(const Geom& g, const BrickPar
         if (NEXT) {
           x += u * nx.dt + a * nx.dt2;
           u += a * dth;
-          const int ri = (int)(At.rc % (uint32_t)bp.RX), rj = (int)((At.rc / (uint32_t)bp.RX) % (uint32_t)bp.RY),
-                    rk = (int)(At.rc / ((uint32_t)bp.RX * (uint32_t)bp.RY));
+          int gi, gj, gk;
+          force_cell(bp, brick_pos(g, bp, b), At.bc, gi, gj, gk);
           const double o = c == 0 ? g.ox : c == 1 ? g.oy : g.oz;
-          const int loc = c == 0 ? P.gi0 - 1 + ri : c == 1 ? P.gj0 - 1 + rj : P.gk0 - 1 + rk;
+          const int loc = c == 0 ? gi : c == 1 ? gj : gk;
           dd = x - restore_u32_double(nx.backup[3 * (size_t)s + c], cell_origin(o, g.gl, loc, g.cs), g.cs);
         }
         vel[s] = u;
@@ -1165,24 +1317,22 @@ __device__ __forceinline__ void lj_quad_brick_body(const Geom& g, const BrickPar
 
 template <bool MIXED, bool ACCUM, int EPI>
 __global__ void __launch_bounds__(1024) k_lj_quad_brick(Geom g, BrickParams bp, const double4* __restrict__ r,
-                                                        const uint32_t* __restrict__ cell_off, const uint32_t* __restrict__ cell_n,
                                                         const uint16_t* __restrict__ blist, const uint32_t* __restrict__ bcnt, LJConst lj,
                                                         PState A, double dth, NextStep nx) {
   const uint32_t b = brick_of_block<MIXED>(bp);
   if (b >= bp.nbricks) return;  // whole workgroup, before any barrier
-  lj_quad_brick_body<MIXED, ACCUM, EPI>(g, bp, b, r, cell_off, cell_n, blist, bcnt, lj, A, dth, nx);
+  lj_quad_brick_body<MIXED, ACCUM, EPI>(g, bp, b, r, blist, bcnt, lj, A, dth, nx);
 }
 
 // Any other force functor on brick lists (no fused epilogue): f += pairs (ACCUM, after
 // zero_particle_force).
 template <class F>
 __global__ void __launch_bounds__(1024) k_compute_pair_brick(Geom g, BrickParams bp, const double4* __restrict__ r,
-                                                             const uint32_t* __restrict__ cell_off, const uint32_t* __restrict__ cell_n,
                                                              const uint16_t* __restrict__ blist, const uint32_t* __restrict__ bcnt, F func,
                                                              double rc2, PState A) {
   const uint32_t b = brick_of_block<true>(bp);
   if (b >= bp.nbricks) return;  // whole workgroup, before any barrier
-  compute_pair_brick_body<F, true, EPI_NONE, LJB_UNROLL_B>(g, bp, b, r, cell_off, cell_n, blist, bcnt, func, rc2, A, 0.0, NextStep{});
+  compute_pair_brick_body<F, true, EPI_NONE, LJB_UNROLL_B>(g, bp, b, r, blist, bcnt, func, rc2, A, 0.0, NextStep{});
 }
 
 // ------------------------------------------------------------------ multimat force
@@ -1197,20 +1347,21 @@ __global__ void __launch_bounds__(1024) k_compute_pair_brick(Geom g, BrickParams
 // zero_particle_force); otherwise f starts from 0.0 like a zeroed force.  EPI as in k_lj_brick.
 template <bool MIXED, int NT, bool ACCUM, int EPI, int U>
 __device__ __forceinline__ void ljmm_brick_body(const Geom& g, const BrickParams& bp, uint32_t b, const double4* __restrict__ r,
-                                                const uint32_t* __restrict__ cell_off, const uint32_t* __restrict__ cell_n,
                                                 const uint16_t* __restrict__ blist, const uint32_t* __restrict__ bcnt,
                                                 const LJMulti& mm, const PState& A, double dth, const NextStep& nx) {
   extern __shared__ __align__(16) char lds[];
-  const BrickLds L = brick_lds(bp, lds);
-  const BrickPos P = brick_pos(g, bp, b);
-  if (EPI == EPI_NEXT && threadIdx.x == 0) {  // ordered before every wave's count by brick_setup's barriers
+  const BrickLds L = force_lds(bp, lds);
+  if (EPI == EPI_NEXT && threadIdx.x == 0) {  // ordered before every wave's count by the staging's barrier
     L.wcnt[0] = 0;
     L.wcnt[1] = 0;
   }
-  if (!brick_setup(g, bp, P, L, r, cell_off, cell_n, kPosF64)) return;
-  const LaneAtom At = lane_atom(bp, L, threadIdx.x);
   const uint32_t t = threadIdx.x, T = bp.T;
-  const uint32_t n = At.live ? bcnt[(size_t)b * T + t] : 0u;
+  const uint32_t lw = lane_word(bp, b, t);
+  const uint32_t n_list = t < T ? bcnt[(size_t)b * T + t] : 0u;
+  stage_region<true>(g, bp, b, r, L);
+  __syncthreads();
+  const ForceAtom At = force_atom(bp, b, lw);
+  const uint32_t n = At.live ? n_list : 0u;
   const uint32_t nmax = wave_max_b(n);
   const double ax0 = L.px[3 * At.ia], ay0 = L.py[3 * At.ia], az0 = L.pz[3 * At.ia];
   const unsigned ta = L.pt[At.ia];
@@ -1385,9 +1536,9 @@ __device__ __forceinline__ void ljmm_brick_body(const Geom& g, const BrickParams
         ux += fx * dth;
         uy += fy * dth;
         uz += fz * dth;
-        const int ri = (int)(At.rc % (uint32_t)bp.RX), rj = (int)((At.rc / (uint32_t)bp.RX) % (uint32_t)bp.RY),
-                  rk = (int)(At.rc / ((uint32_t)bp.RX * (uint32_t)bp.RY));
-        over = displaced_ijk(g, p, P.gi0 - 1 + ri, P.gj0 - 1 + rj, P.gk0 - 1 + rk, nx.backup, s, nx.thr2);
+        int gi, gj, gk;
+        force_cell(bp, brick_pos(g, bp, b), At.bc, gi, gj, gk);
+        over = displaced_ijk(g, p, gi, gj, gk, nx.backup, s, nx.thr2);
       }
       __builtin_nontemporal_store(ux, &A.vx[s]);
       __builtin_nontemporal_store(uy, &A.vy[s]);
@@ -1399,12 +1550,11 @@ __device__ __forceinline__ void ljmm_brick_body(const Geom& g, const BrickParams
 
 template <bool MIXED, int NT, bool ACCUM, int EPI>
 __global__ void __launch_bounds__(1024) k_ljmm_brick(Geom g, BrickParams bp, const double4* __restrict__ r,
-                                                     const uint32_t* __restrict__ cell_off, const uint32_t* __restrict__ cell_n,
                                                      const uint16_t* __restrict__ blist, const uint32_t* __restrict__ bcnt, LJMulti mm,
                                                      PState A, double dth, NextStep nx) {
   const uint32_t b = brick_of_block<MIXED>(bp);
   if (b >= bp.nbricks) return;  // whole workgroup, before any barrier
-  ljmm_brick_body<MIXED, NT, ACCUM, EPI, LJB_UNROLL_B>(g, bp, b, r, cell_off, cell_n, blist, bcnt, mm, A, dth, nx);
+  ljmm_brick_body<MIXED, NT, ACCUM, EPI, LJB_UNROLL_B>(g, bp, b, r, blist, bcnt, mm, A, dth, nx);
 }
 
 // ------------------------------------------------------------------ conversion
@@ -1483,6 +1633,18 @@ uint32_t brick_layout(BrickParams& bp, bool f32_build, bool f32_types) {
   return align8(o);
 }
 
+// LDS layout of the force kernels; returns its bytes
+uint32_t brick_force_layout(BrickParams& bp, bool types) {
+  bp.off_pos = 0;
+  uint32_t o = 24u * (bp.Rmax + 1u);
+  bp.off_type = o;
+  if (types) o = align8(o + bp.Rmax + 1u);
+  bp.off_wsum = o;
+  return align8(o + 2u * 4u);
+}
+
+size_t brick_reg_words(const BrickParams& bp) { return (size_t)bp.nbricks * (bp.Rmax + 1u); }
+
 void launch_brick_stats(const Geom& g, const BrickShapes& sh, const uint32_t* cell_n, uint32_t* out, hipStream_t st) {
   uint32_t most = 0;
   for (uint32_t k = 0; k < sh.n; k++) most = std::max(most, sh.shape[k].nbricks);
@@ -1555,27 +1717,26 @@ hipError_t launch_nbh_brick(const Geom& g, BrickParams bp, const double4* r, con
 static constexpr int LJB_UNROLL = LJB_UNROLL_B;
 
 template <bool MIXED, bool ACCUM, int EPI>
-static hipError_t ljb_launch(const Geom& g, const BrickParams& bp, uint32_t lds, const double4* r, const uint32_t* cell_off,
-                             const uint32_t* cell_n, const uint16_t* blist, const uint32_t* bcnt, const LJConst& lj, const PState& A,
+static hipError_t ljb_launch(const Geom& g, const BrickParams& bp, uint32_t lds, const double4* r, const uint16_t* blist, const uint32_t* bcnt, const LJConst& lj, const PState& A,
                              double dth, const NextStep& nx, hipStream_t st) {
   auto* const fn = bp.lanes == kQuad ? k_lj_quad_brick<MIXED, ACCUM, EPI> : k_lj_brick<MIXED, ACCUM, EPI, LJB_UNROLL>;
   hipError_t e = set_lds((const void*)fn, lds);
   if (e != hipSuccess) return e;
-  fn<<<kXcds * bp.per_xcd, bp.T * bp.lanes, lds, st>>>(g, bp, r, cell_off, cell_n, blist, bcnt, lj, A, dth, nx);
+  fn<<<kXcds * bp.per_xcd, bp.T * bp.lanes, lds, st>>>(g, bp, r, blist, bcnt, lj, A, dth, nx);
   return hipGetLastError();
 }
 
 uint32_t brick_list_granule() { return LJB_UNROLL; }
 
-hipError_t launch_lj_brick(int precision, bool accum, int epi, const Geom& g, BrickParams bp, const PState& A, const uint32_t* cell_off,
-                           const uint32_t* cell_n, const uint16_t* blist, const uint32_t* bcnt, double eps, double sigma, double rcut,
+hipError_t launch_lj_brick(int precision, bool accum, int epi, const Geom& g, BrickParams bp, const PState& A,
+                           const uint16_t* blist, const uint32_t* bcnt, double eps, double sigma, double rcut,
                            double dth, const NextStep* next, hipStream_t st) {
   const LJConst lj = make_lj_const(eps, sigma, rcut);
-  const uint32_t lds = brick_layout(bp);
+  const uint32_t lds = brick_force_layout(bp, false);
   const NextStep nx = next ? *next : NextStep{};
   const bool next_epi = epi == EPI_NEXT;
   if (next_epi && (accum || !next)) return hipErrorInvalidValue;
-#define XNB_LJB_ARGS g, bp, lds, A.r, cell_off, cell_n, blist, bcnt, lj, A, dth, nx, st
+#define XNB_LJB_ARGS g, bp, lds, A.r, blist, bcnt, lj, A, dth, nx, st
   if (precision) {
     if (epi == EPI_NEXT) return ljb_launch<true, false, EPI_NEXT>(XNB_LJB_ARGS);
     if (accum) return epi ? ljb_launch<true, true, EPI_KICK>(XNB_LJB_ARGS) : ljb_launch<true, true, EPI_NONE>(XNB_LJB_ARGS);
@@ -1588,51 +1749,55 @@ hipError_t launch_lj_brick(int precision, bool accum, int epi, const Geom& g, Br
 }
 
 template <bool MIXED, int NT, bool ACCUM, int EPI>
-static hipError_t ljmm_launch(const Geom& g, const BrickParams& bp, uint32_t lds, const uint32_t* cell_off, const uint32_t* cell_n,
-                              const uint16_t* blist, const uint32_t* bcnt, const LJMulti& mm, const PState& A, double dth,
+static hipError_t ljmm_launch(const Geom& g, const BrickParams& bp, uint32_t lds, const uint16_t* blist, const uint32_t* bcnt, const LJMulti& mm, const PState& A, double dth,
                               const NextStep& nx, hipStream_t st) {
   hipError_t e = set_lds((const void*)k_ljmm_brick<MIXED, NT, ACCUM, EPI>, lds);
   if (e != hipSuccess) return e;
-  k_ljmm_brick<MIXED, NT, ACCUM, EPI><<<kXcds * bp.per_xcd, bp.T, lds, st>>>(g, bp, A.r, cell_off, cell_n, blist, bcnt, mm, A, dth, nx);
+  k_ljmm_brick<MIXED, NT, ACCUM, EPI><<<kXcds * bp.per_xcd, bp.T, lds, st>>>(g, bp, A.r, blist, bcnt, mm, A, dth, nx);
   return hipGetLastError();
 }
 
 template <bool MIXED, int NT>
-static hipError_t ljmm_dispatch(int epi, const Geom& g, const BrickParams& bp, uint32_t lds, const uint32_t* cell_off,
-                                const uint32_t* cell_n, const uint16_t* blist, const uint32_t* bcnt, const LJMulti& mm, const PState& A,
+static hipError_t ljmm_dispatch(int epi, const Geom& g, const BrickParams& bp, uint32_t lds, const uint16_t* blist, const uint32_t* bcnt, const LJMulti& mm, const PState& A,
                                 double dth, const NextStep& nx, hipStream_t st) {
   switch (epi) {
-    case EPI_NONE: return ljmm_launch<MIXED, NT, true, EPI_NONE>(g, bp, lds, cell_off, cell_n, blist, bcnt, mm, A, dth, nx, st);
-    case EPI_KICK: return ljmm_launch<MIXED, NT, false, EPI_KICK>(g, bp, lds, cell_off, cell_n, blist, bcnt, mm, A, dth, nx, st);
-    default: return ljmm_launch<MIXED, NT, false, EPI_NEXT>(g, bp, lds, cell_off, cell_n, blist, bcnt, mm, A, dth, nx, st);
+    case EPI_NONE: return ljmm_launch<MIXED, NT, true, EPI_NONE>(g, bp, lds, blist, bcnt, mm, A, dth, nx, st);
+    case EPI_KICK: return ljmm_launch<MIXED, NT, false, EPI_KICK>(g, bp, lds, blist, bcnt, mm, A, dth, nx, st);
+    default: return ljmm_launch<MIXED, NT, false, EPI_NEXT>(g, bp, lds, blist, bcnt, mm, A, dth, nx, st);
   }
 }
 
 // Multimat force on brick lists.  epi EPI_NONE accumulates into f (after zero_particle_force);
 // the other epilogues start f from 0, as the run loop's zero + force.  ntypes 1..4.
-hipError_t launch_ljmm_brick(int precision, int ntypes, int epi, const Geom& g, BrickParams bp, const PState& A, const uint32_t* cell_off,
-                             const uint32_t* cell_n, const uint16_t* blist, const uint32_t* bcnt, const LJMulti& mm, double dth,
+hipError_t launch_ljmm_brick(int precision, int ntypes, int epi, const Geom& g, BrickParams bp, const PState& A, const uint16_t* blist, const uint32_t* bcnt, const LJMulti& mm, double dth,
                              const NextStep* next, hipStream_t st) {
   if (ntypes < 1 || ntypes > 4) return hipErrorInvalidValue;
   if (epi == EPI_NEXT && !next) return hipErrorInvalidValue;
-  const uint32_t lds = brick_layout(bp);
+  const uint32_t lds = brick_force_layout(bp, true);
   const NextStep nx = next ? *next : NextStep{};
   if (precision) {
-    if (ntypes <= 2) return ljmm_dispatch<true, 2>(epi, g, bp, lds, cell_off, cell_n, blist, bcnt, mm, A, dth, nx, st);
-    return ljmm_dispatch<true, 4>(epi, g, bp, lds, cell_off, cell_n, blist, bcnt, mm, A, dth, nx, st);
+    if (ntypes <= 2) return ljmm_dispatch<true, 2>(epi, g, bp, lds, blist, bcnt, mm, A, dth, nx, st);
+    return ljmm_dispatch<true, 4>(epi, g, bp, lds, blist, bcnt, mm, A, dth, nx, st);
   }
-  if (ntypes <= 2) return ljmm_dispatch<false, 2>(epi, g, bp, lds, cell_off, cell_n, blist, bcnt, mm, A, dth, nx, st);
-  return ljmm_dispatch<false, 4>(epi, g, bp, lds, cell_off, cell_n, blist, bcnt, mm, A, dth, nx, st);
+  if (ntypes <= 2) return ljmm_dispatch<false, 2>(epi, g, bp, lds, blist, bcnt, mm, A, dth, nx, st);
+  return ljmm_dispatch<false, 4>(epi, g, bp, lds, blist, bcnt, mm, A, dth, nx, st);
 }
 
-hipError_t launch_gravity_brick(const Geom& g, BrickParams bp, const PState& A, const uint32_t* cell_off, const uint32_t* cell_n,
-                                const uint16_t* blist, const uint32_t* bcnt, const GravitationalForceFunctor& gf, double rc2,
+hipError_t launch_gravity_brick(const Geom& g, BrickParams bp, const PState& A, const uint16_t* blist, const uint32_t* bcnt, const GravitationalForceFunctor& gf, double rc2,
                                 hipStream_t st) {
-  const uint32_t lds = brick_layout(bp);
+  const uint32_t lds = brick_force_layout(bp, true);
   hipError_t e = set_lds((const void*)k_compute_pair_brick<GravitationalForceFunctor>, lds);
   if (e != hipSuccess) return e;
-  k_compute_pair_brick<GravitationalForceFunctor><<<kXcds * bp.per_xcd, bp.T, lds, st>>>(g, bp, A.r, cell_off, cell_n, blist, bcnt, gf,
+  k_compute_pair_brick<GravitationalForceFunctor><<<kXcds * bp.per_xcd, bp.T, lds, st>>>(g, bp, A.r, blist, bcnt, gf,
                                                                                          rc2, A);
+  return hipGetLastError();
+}
+
+hipError_t launch_brick_regions(const Geom& g, BrickParams bp, const uint32_t* cell_off, const uint32_t* cell_n, hipStream_t st) {
+  const uint32_t lds = brick_layout(bp);
+  hipError_t e = set_lds((const void*)k_brick_regions, lds);
+  if (e != hipSuccess) return e;
+  k_brick_regions<<<kXcds * bp.per_xcd, bp.T, lds, st>>>(g, bp, cell_off, cell_n);
   return hipGetLastError();
 }
 
@@ -1676,7 +1841,7 @@ __device__ __forceinline__ void lj_batch_case(const BoxFrame& f, uint32_t b, uin
   // the next step's count: local step k = gstep - gstep0 + 1, count of step k + 1 at [k]
   const NextStep nx{f.rbuf[cur ^ 1u], f.backup, f.dt, f.dt2, f.thr2, f.counts + (gstep - f.gstep0 + 1)};
   compute_pair_brick_body<LennardJonesForceFunctor<MIXED>, false, EPI, LJB_UNROLL_B>(
-      f.g, f.bp, b, A.r, f.cell_off, f.cell_n, f.blist, f.bcnt, LennardJonesForceFunctor<MIXED>{f.lj}, f.lj.rc2, A, f.dth, nx);
+      f.g, f.bp, b, A.r, f.blist, f.bcnt, LennardJonesForceFunctor<MIXED>{f.lj}, f.lj.rc2, A, f.dth, nx);
 }
 
 // Force of every brick of the listed boxes, all of one precision (one kernel per precision,

@@ -91,7 +91,10 @@ struct xnb_ctx {
   int brick_dims[3] = {0, 0, 0};  // 0: choose automatically
   int brick_lanes = 0;            // lanes per atom (1 or kQuad); 0: choose automatically
   DArr<uint16_t> blist;
-  DArr<uint32_t> bcnt;
+  DArr<uint32_t> bcnt, breg, blane;
+  // ghosts in the brick lists' reg words by source and shift (the run loops and batches, whose
+  // ghosts always follow their sources) or by slot (operators, which read the ghosts as they are)
+  bool derive_ghosts = false;
   bool slot_lists_current = false;  // nbr/nbr_cnt mirror the brick lists
   bool fuse_push = true;            // force kernel performs the next step's first half (brick lists)
   bool nbh_prefilter = true;        // unfiltered brick builds test in FP32 with an FP64 band (same lists)
@@ -157,6 +160,7 @@ int op_nbh(xnb_ctx* c, double nbh_dist, const xnb_chunk_neighbors_config& cfg, i
 // forces false: f and ep neither carried by the move nor copied to ghosts; pc: per type-pair list radii
 int full_update(xnb_ctx* c, bool forces = true, const PairCut* pc = nullptr);
 int ensure_full_lists(xnb_ctx* c);
+int ensure_regions(xnb_ctx* c, bool derive);
 void tstart(xnb_ctx* c, int id);
 void tstop(xnb_ctx* c);
 

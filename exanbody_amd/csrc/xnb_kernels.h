@@ -35,7 +35,16 @@ struct BrickParams {
   uint32_t off_rcnt, off_rpref, off_roff, off_bpref, off_pos, off_type;  // LDS byte offsets
   uint32_t off_rdel, off_crow;  // staging tables: per region row, per 64 region atoms
   uint32_t off_wsum;            // 32 scan words, then the 2 wave-group counter words
+  // the region as the force kernels read it, written by the build (see region_word)
+  uint32_t* reg;                // (Rmax + 1) words per brick
+  uint32_t* lane;               // T words per brick
+  uint32_t derive;              // 1: ghosts by source slot and shift, 0: by their own slot
+  uint32_t n_inner;             // slots below are inner, the ghosts follow
+  const uint32_t *ghost_src, *ghost_shift;
 };
+
+// derive needs every inner slot below this (the shift code shares its word)
+constexpr uint32_t kDeriveSlots = 1u << 26;
 
 // Per type-pair list radii of a multi-material run: a candidate b of an atom a is kept when
 // d2 <= thr2[type a][type b] (each at most the build's nbh_dist^2); nt = 0: one radius for all.
@@ -77,7 +86,7 @@ struct PState {
 // batch).  Kernels may update ab, rcur and G; the host keeps a mirror.
 struct BoxFrame {
   Geom g;
-  BrickParams bp;  // bp.status == words + 0
+  BrickParams bp;  // the force's LDS layout; bp.status == words + 0
   BrickParams bpn;  // bp with the prefiltered neighbour build's LDS layout
   uint32_t N, G, cap;
   uint32_t ab;     // 1: the roles of the A and B field arrays are exchanged
@@ -198,9 +207,8 @@ void launch_nbh_build(const Geom& g, uint32_t n_atoms, const double4* r, const u
 uint32_t lj_list_granule();
 void launch_gravity_slots(uint32_t n_atoms, const PState& A, const uint32_t* nbr, const uint32_t* nbr_cnt, uint32_t cap,
                           const GravitationalForceFunctor& gf, double rc2, hipStream_t st);
-hipError_t launch_gravity_brick(const Geom& g, BrickParams bp, const PState& A, const uint32_t* cell_off, const uint32_t* cell_n,
-                                const uint16_t* blist, const uint32_t* bcnt, const GravitationalForceFunctor& gf, double rc2,
-                                hipStream_t st);
+hipError_t launch_gravity_brick(const Geom& g, BrickParams bp, const PState& A, const uint16_t* blist, const uint32_t* bcnt,
+                                const GravitationalForceFunctor& gf, double rc2, hipStream_t st);
 void launch_max_type(uint32_t n, const double4* r, uint32_t* out, hipStream_t st);
 void launch_lj(int precision, bool accum, bool push, uint32_t n_atoms, const PState& A, const uint32_t* nbr,
                const uint32_t* nbr_cnt, uint32_t cap, double eps, double sigma, double rcut, double dth, hipStream_t st);
@@ -222,6 +230,10 @@ BrickParams brick_params(const Geom& g, int Bi, int Bj, int Bk);
 // LDS layout of the brick kernels (offsets into bp), its bytes; f32_build: the prefiltered
 // neighbour build's (FP32 positions; types only with f32_types, for per-pair radii)
 uint32_t brick_layout(BrickParams& bp, bool f32_build = false, bool f32_types = false);
+uint32_t brick_force_layout(BrickParams& bp, bool types);  // of the force kernels
+size_t brick_reg_words(const BrickParams& bp);
+// bp.reg again for bp.derive (the lists and lane words stay)
+hipError_t launch_brick_regions(const Geom& g, BrickParams bp, const uint32_t* cell_off, const uint32_t* cell_n, hipStream_t st);
 uint32_t brick_list_granule();
 // brick shapes whose occupancy is looked at together; out: 2 words a shape, 0 on entry
 constexpr uint32_t kStatShapes = 4;
@@ -234,11 +246,11 @@ void launch_brick_stats(const Geom& g, const BrickShapes& sh, const uint32_t* ce
 hipError_t launch_nbh_brick(const Geom& g, BrickParams bp, const double4* r, const uint32_t* cell_off, const uint32_t* cell_n, double max2,
                             const PairCut& pc, int half_symmetric, int skip_ghosts, bool prefilter, uint16_t* blist, uint32_t* bcnt,
                             uint32_t* max_cnt, hipStream_t st);
-hipError_t launch_lj_brick(int precision, bool accum, int epi, const Geom& g, BrickParams bp, const PState& A, const uint32_t* cell_off,
-                           const uint32_t* cell_n, const uint16_t* blist, const uint32_t* bcnt, double eps, double sigma, double rcut,
+hipError_t launch_lj_brick(int precision, bool accum, int epi, const Geom& g, BrickParams bp, const PState& A,
+                           const uint16_t* blist, const uint32_t* bcnt, double eps, double sigma, double rcut,
                            double dth, const NextStep* next, hipStream_t st);
-hipError_t launch_ljmm_brick(int precision, int ntypes, int epi, const Geom& g, BrickParams bp, const PState& A, const uint32_t* cell_off,
-                             const uint32_t* cell_n, const uint16_t* blist, const uint32_t* bcnt, const LJMulti& mm, double dth,
+hipError_t launch_ljmm_brick(int precision, int ntypes, int epi, const Geom& g, BrickParams bp, const PState& A,
+                             const uint16_t* blist, const uint32_t* bcnt, const LJMulti& mm, double dth,
                              const NextStep* next, hipStream_t st);
 hipError_t launch_brick_to_slots(const Geom& g, BrickParams bp, const uint32_t* cell_off, const uint32_t* cell_n, const uint16_t* blist,
                                  const uint32_t* bcnt, uint32_t* nbr, uint32_t* nbr_cnt, uint32_t cap, hipStream_t st);

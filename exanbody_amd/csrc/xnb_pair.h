@@ -333,11 +333,15 @@ struct LennardJonesForceFunctor {
   __device__ __forceinline__ void batch(const double4& ra, const NbhBatch<U>& nb, double& fx, double& fy, double& fz,
                                         double& ep) const {
     if (MIXED) {
-      double4 rb[U];
 #pragma unroll
-      for (int u = 0; u < U; u++) rb[u] = nb(u);
+      for (int h = 0; h < U; h += 4) {
+        double4 rb[4];
 #pragma unroll
-      for (int u = 0; u < U; u++) lj_pair_mixed<ENERGY>(p, ra, rb[u], fx, fy, fz, ep);
+        for (int u = 0; u < 4; u++) rb[u] = nb(h + u);
+#pragma unroll
+        for (int u = 0; u < 4; u++) lj_pair_mixed<ENERGY>(p, ra, rb[u], fx, fy, fz, ep);
+        __builtin_amdgcn_sched_barrier(0);
+      }
     } else {
 #pragma unroll
       for (int u = 0; u < U; u++) lj_pair_fp64_any<ENERGY>(p, ra, nb(u), fx, fy, fz, ep);
