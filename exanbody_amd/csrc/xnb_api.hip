@@ -231,29 +231,36 @@ int scan(xnb_ctx* c, const uint32_t* in, uint32_t n, uint32_t add, uint32_t* out
 
 // ---- operators
 
+// words of u32s cleared by a move: its flags, the rebuild_amr count, and those of the list
+// build that follows in a full update (longest list, brick status, brick sizes)
+constexpr uint32_t kMoveWords = 1u << 0, kAmrWords = 1u << 8, kBuildWords = 1u << 2 | 1u << 6 | 0xffu << 16;
+
 // check false: the out-of-domain flag (u32s[0]) is left for the caller to read (op_ghost_all
-// reads it with the ghost count in one transfer)
-int op_move(xnb_ctx* c, bool forces = true, bool check = true) {
+// reads it with the ghost count in one transfer).  update: the move of a full update, which also
+// lists rebuild_amr's cells and clears the words of the list build.
+int op_move(xnb_ctx* c, bool forces = true, bool check = true, bool update = false) {
   const Geom& g = c->g;
+  int e;
   c->lists_valid = false;
   c->ghosts_valid = false;
   c->backup_valid = false;
-  // the out-of-domain flag describes this move, also when there is nothing to move
-  HIPCHK(c, hipMemsetAsync(c->u32s.p, 0, sizeof(uint32_t), c->st));
-  if (c->N == 0) return XNB_OK;
+  if (update && (e = dalloc(c, c->amr_list, g.ncells))) return e;
   tstart(c, XNB_TIMER_REBIN);
-  HIPCHK(c, hipMemsetAsync(c->cnt_out.p, 0, g.ncells * sizeof(uint32_t), c->st));
-  HIPCHK(c, hipMemsetAsync(c->cnt_in.p, 0, g.ncells * sizeof(uint32_t), c->st));
-  HIPCHK(c, hipMemsetAsync(c->in_cur.p, 0, g.ncells * sizeof(uint32_t), c->st));
+  // the out-of-domain flag describes this move, also when there is nothing to move
+  launch_move_zero(g.ncells, c->cnt_out.p, c->cnt_in.p, c->in_cur.p, c->u32s.p, kMoveWords | (update ? kAmrWords | kBuildWords : 0u),
+                   c->st);
+  if (c->N == 0) {
+    tstop(c);
+    HIPCHK(c, hipGetLastError());
+    return XNB_OK;
+  }
   launch_move_flag(g, c->N, c->A.r, c->slot_cell_A.p, c->mv_dst.p, c->cnt_out.p, c->cnt_in.p, c->u32s.p, c->st);
   launch_move_pack(g, c->cell_off.p, c->cell_n.p, c->cnt_out.p, c->cnt_in.p, c->mv_dst.p, c->pk.p, c->newloc.p, c->new_n.p, c->st);
-  int e;
   if ((e = scan(c, c->new_n.p, g.ncells, 0, c->new_off.p))) return e;
   launch_move_scatter(c->N, c->A, c->B, c->slot_cell_A.p, c->mv_dst.p, c->newloc.p, c->cell_off.p, c->new_off.p, c->cell_n.p,
                       c->cnt_out.p, c->in_cur.p, c->in_list.p, c->slot_cell_B.p, forces, c->st);
-  launch_move_incoming(g, c->A, c->B, c->new_off.p, c->cell_n.p, c->cnt_out.p, c->cnt_in.p, c->in_list.p, c->slot_cell_B.p, forces,
-                       c->st);
-  launch_set_inner_cells(g, c->new_n.p, c->new_off.p, c->cell_n.p, c->cell_off.p, c->st);
+  launch_move_finish(g, c->N, c->A, c->B, c->mv_dst.p, c->new_off.p, c->new_n.p, c->cnt_in.p, c->in_list.p, c->slot_cell_B.p,
+                     c->cell_n.p, c->cell_off.p, forces, update ? kSubGridDensity : 0.0, c->amr_list.p, c->u32s.p + 8, c->u32s.p, c->st);
   tstop(c);
   HIPCHK(c, hipGetLastError());
   uint32_t errflag = 0;
@@ -262,52 +269,6 @@ int op_move(xnb_ctx* c, bool forces = true, bool check = true) {
   // ghost cells are empty until ghost_update_all rebuilds them
   c->G = 0;
   if (errflag) return fail(c, XNB_E_OUTSIDE, "a particle left the domain along a non-periodic axis");
-  return XNB_OK;
-}
-
-// move_check: also report the out-of-domain flag of a preceding op_move(c, ..., false).
-// forces: images copy f and ep of their sources (false: f and ep of the images are 0)
-int op_ghost_all(xnb_ctx* c, bool move_check, bool forces) {
-  const Geom& g = c->g;
-  int e;
-  tstart(c, XNB_TIMER_GHOST);
-  launch_ghost_count(g, c->A.r, c->cell_off.p, c->cell_n.p, c->gcnt.p, c->st);
-  if ((e = scan(c, c->gcnt.p, g.ncells, 0, c->goff.p))) return e;
-  tstop(c);
-  uint32_t w[2] = {0, 0};  // u32s[0]: bit 1 out of the domain, bit 2 too dense; u32s[1]: ghost count
-  if ((e = read_u32(c, c->u32s.p, w, 2))) return e;
-  if (w[0] & 2u) return fail(c, XNB_E_CAPACITY, "rebuild_amr: a cell holds more than 4096 particles");
-  if (move_check && w[0]) return fail(c, XNB_E_OUTSIDE, "a particle left the domain along a non-periodic axis");
-  const uint32_t G = w[1];
-  if ((e = ensure_capacity(c, (size_t)c->N + G, c->N))) return e;
-  tstart(c, XNB_TIMER_GHOST);
-  launch_ghost_fill(g, c->N, c->A, c->goff.p, c->cell_off.p, c->cell_n.p, c->slot_cell_A.p, c->ghost_src.p, c->ghost_shift.p,
-                    (uint32_t)std::min<size_t>(c->cap, 0xffffffffu), c->u32s.p + 7, forces, c->st);
-  tstop(c);
-  HIPCHK(c, hipGetLastError());
-  c->G = G;
-  c->ghosts_valid = true;
-  c->lists_valid = false;
-  return XNB_OK;
-}
-
-// rebuild_amr after a move (ghost cells empty): dense inner cells sorted by sub-cell through
-// the spare buffers; u32s[8] counts the listed cells, a cell too dense to sort sets bit 2 of
-// u32s[0] (reported with the ghost count, or by xnb_rebuild_amr)
-int op_amr(xnb_ctx* c, double density, bool forces) {
-  if (c->N == 0) return XNB_OK;
-  int e;
-  if ((e = dalloc(c, c->amr_list, c->g.ncells))) return e;
-  HIPCHK(c, hipMemsetAsync(c->u32s.p + 8, 0, sizeof(uint32_t), c->st));
-  launch_rebuild_amr(c->g, density, c->A, c->B, c->cell_off.p, c->cell_n.p, c->amr_list.p, c->u32s.p + 8, c->u32s.p, forces, c->st);
-  HIPCHK(c, hipGetLastError());
-  return XNB_OK;
-}
-
-int op_backup(xnb_ctx* c) {
-  launch_backup_r(c->g, c->N, c->A.r, c->slot_cell_A.p, c->backup.p, c->st);
-  HIPCHK(c, hipGetLastError());
-  c->backup_valid = true;
   return XNB_OK;
 }
 
@@ -333,48 +294,140 @@ constexpr uint32_t kEnoughBricks = 192;
 // another launch and read-back.
 constexpr uint32_t kStatBricks = 8192;
 
-// Brick dims, lanes, T and Rmax for the current cell occupancy; NOT_APPLICABLE if nothing fits LDS.
-int choose_bricks(xnb_ctx* c, uint32_t cap, bool quads, BrickParams& out) {
+// Brick shapes to try, in order.
+struct ShapeList {
   struct Cand {
     int dims[3];
     uint32_t lanes;
     bool any;  // taken whatever its brick count
-  };
+  } cand[2 + 4 + 9];
+  int n = 0;
+  void add(const int (&d)[3], uint32_t lanes, bool any) { cand[n++] = Cand{{d[0], d[1], d[2]}, lanes, any}; }
+};
+
+void list_shapes(const xnb_ctx* c, bool quads, ShapeList& l) {
   // Larger bricks first.  (4,3,2) and (3,3,2) only for batched boxes: under the batch's LDS cap
   // they beat (4,2,2) (512-box batch: 3.58e9 -> 3.90e9 atom-steps/s), while the two-species slab
   // run alone is faster on (4,2,2) bricks.  Batched boxes share the chip: no brick count to reach.
   static const int wide[][3] = {{4, 4, 2}, {4, 3, 2}, {3, 3, 2}, {4, 2, 2}, {2, 2, 2}, {4, 2, 1}, {2, 2, 1}, {2, 1, 1}, {1, 1, 1}};
   static const int quad[][3] = {{2, 2, 2}, {2, 2, 1}, {2, 1, 1}, {1, 1, 1}};
-  Cand cand[2 + 4 + 9];
-  int ncand = 0;
-  auto add = [&](const int (&d)[3], uint32_t lanes, bool any) { cand[ncand++] = Cand{{d[0], d[1], d[2]}, lanes, any}; };
   if (c->brick_dims[0] > 0) {
-    if (quads) add(c->brick_dims, kQuad, true);
-    add(c->brick_dims, 1u, true);
+    if (quads) l.add(c->brick_dims, kQuad, true);
+    l.add(c->brick_dims, 1u, true);
   }
   if (quads)
-    for (const auto& d : quad) add(d, kQuad, &d == &quad[3]);
+    for (const auto& d : quad) l.add(d, kQuad, &d == &quad[3]);
   for (int q = 0; q < 9; q++)
-    if ((q != 1 && q != 2) || c->batch_shapes) add(wide[q], 1u, c->batch_shapes || q == 8);
-  for (int q = 0; q < ncand;) {
-    // the next shapes, as many at once as are cheap to look at (a large box's first one fits)
-    BrickShapes sh{};
-    uint32_t bricks = 0;
-    for (; q < ncand && sh.n < kStatShapes; q++) {
-      BrickParams bp = brick_params(c->g, cand[q].dims[0], cand[q].dims[1], cand[q].dims[2]);
-      if (!cand[q].any && bp.nbricks < kEnoughBricks) continue;
-      if (sh.n && bricks + bp.nbricks > kStatBricks) break;
-      bp.lanes = cand[q].lanes;
-      bricks += bp.nbricks;
-      sh.shape[sh.n++] = bp;
-    }
+    if ((q != 1 && q != 2) || c->batch_shapes) l.add(wide[q], 1u, c->batch_shapes || q == 8);
+}
+
+// The next shapes to look at together, from l.cand[at] on: as many as are cheap (a large box's
+// first one fits).
+void next_shapes(const xnb_ctx* c, const ShapeList& l, int& at, BrickShapes& sh) {
+  sh = BrickShapes{};
+  uint32_t bricks = 0;
+  for (; at < l.n && sh.n < kStatShapes; at++) {
+    BrickParams bp = brick_params(c->g, l.cand[at].dims[0], l.cand[at].dims[1], l.cand[at].dims[2]);
+    if (!l.cand[at].any && bp.nbricks < kEnoughBricks) continue;
+    if (sh.n && bricks + bp.nbricks > kStatBricks) break;
+    bp.lanes = l.cand[at].lanes;
+    bricks += bp.nbricks;
+    sh.shape[sh.n++] = bp;
+  }
+}
+
+// four lanes an atom: lists of the prefiltered build, for a box run by itself
+bool quad_lists(const xnb_ctx* c, const xnb_chunk_neighbors_config& cfg) {
+  return (c->brick_lanes ? c->brick_lanes == (int)kQuad : c->N <= kQuadAtoms) && !c->batch_shapes && c->nbh_prefilter &&
+         !cfg.half_symmetric && !cfg.skip_ghosts;
+}
+
+// lists on bricks are tried first
+bool brick_lists(const xnb_ctx* c, double nbh_dist, int all_cells) {
+  return !all_cells && (int)std::ceil(nbh_dist / c->g.cs) == 1 && c->g.gl >= 1 && c->use_bricks && c->N > 0;
+}
+
+// move_check: also report the out-of-domain flag of a preceding op_move(c, ..., false).
+// forces: images copy f and ep of their sources (false: f and ep of the images are 0).  update:
+// within a full update, with backup_r, and the first brick shapes of the list build to come are
+// looked at before the read-back and come with it (c->early)
+int op_ghost_all(xnb_ctx* c, bool move_check, bool forces, bool update) {
+  const Geom& g = c->g;
+  int e;
+  tstart(c, XNB_TIMER_GHOST);
+  if (update) launch_backup_ghost_count(g, c->N, c->A.r, c->slot_cell_A.p, c->backup.p, c->cell_off.p, c->cell_n.p, c->gcnt.p, c->st);
+  else launch_ghost_count(g, c->A.r, c->cell_off.p, c->cell_n.p, c->gcnt.p, c->st);
+  if (update) c->backup_valid = true;
+  if ((e = scan(c, c->gcnt.p, g.ncells, 0, c->goff.p))) return e;
+  c->early.n = 0;
+  if (update && brick_lists(c, c->nbh_dist_lab, 0)) {
+    ShapeList l;
+    int at = 0;
+    list_shapes(c, quad_lists(c, xnb_chunk_neighbors_config{1, 0, 0, 0, 0}), l);
+    next_shapes(c, l, at, c->early);
+    if (c->early.n) launch_brick_stats(g, c->early, c->cell_n.p, c->gcnt.p, c->u32s.p + 16, c->st);
+  }
+  tstop(c);
+  HIPCHK(c, hipGetLastError());
+  uint32_t w[16 + 2 * kStatShapes] = {};  // u32s[0]: bit 1 out of the domain, bit 2 too dense; u32s[1]: ghost count
+  if ((e = read_u32(c, c->u32s.p, w, c->early.n ? 16 + 2 * (int)kStatShapes : 2))) return e;
+  std::copy(w + 16, w + 16 + 2 * kStatShapes, c->early_sizes);
+  if (w[0] & 2u) return fail(c, XNB_E_CAPACITY, "rebuild_amr: a cell holds more than 4096 particles");
+  if (move_check && w[0]) return fail(c, XNB_E_OUTSIDE, "a particle left the domain along a non-periodic axis");
+  const uint32_t G = w[1];
+  if ((e = ensure_capacity(c, (size_t)c->N + G, c->N))) return e;
+  tstart(c, XNB_TIMER_GHOST);
+  launch_ghost_fill(g, c->N, c->A, c->goff.p, c->cell_off.p, c->cell_n.p, c->slot_cell_A.p, c->ghost_src.p, c->ghost_shift.p,
+                    (uint32_t)std::min<size_t>(c->cap, 0xffffffffu), c->u32s.p + 7, forces, c->st);
+  tstop(c);
+  HIPCHK(c, hipGetLastError());
+  c->G = G;
+  c->ghosts_valid = true;
+  c->lists_valid = false;
+  return XNB_OK;
+}
+
+// rebuild_amr after a move (ghost cells empty): dense inner cells sorted by sub-cell through
+// the spare buffers; u32s[8] counts the listed cells, a cell too dense to sort sets bit 2 of
+// u32s[0] (reported with the ghost count, or by xnb_rebuild_amr).  marked: the move listed them.
+int op_amr(xnb_ctx* c, double density, bool forces, bool marked) {
+  if (c->N == 0) return XNB_OK;
+  int e;
+  if ((e = dalloc(c, c->amr_list, c->g.ncells))) return e;
+  if (!marked) HIPCHK(c, hipMemsetAsync(c->u32s.p + 8, 0, sizeof(uint32_t), c->st));
+  launch_rebuild_amr(c->g, density, c->A, c->B, c->cell_off.p, c->cell_n.p, c->amr_list.p, c->u32s.p + 8, c->u32s.p, forces, marked,
+                     c->st);
+  HIPCHK(c, hipGetLastError());
+  return XNB_OK;
+}
+
+int op_backup(xnb_ctx* c) {
+  launch_backup_r(c->g, c->N, c->A.r, c->slot_cell_A.p, c->backup.p, c->st);
+  HIPCHK(c, hipGetLastError());
+  c->backup_valid = true;
+  return XNB_OK;
+}
+
+// Brick dims, lanes, T and Rmax for the current cell occupancy; NOT_APPLICABLE if nothing fits LDS.
+// The first shapes' sizes may have come with the ghost count (c->early).
+int choose_bricks(xnb_ctx* c, uint32_t cap, bool quads, BrickParams& out) {
+  ShapeList l;
+  list_shapes(c, quads, l);
+  for (int at = 0;;) {
+    BrickShapes sh;
+    next_shapes(c, l, at, sh);
     if (!sh.n) break;
-    HIPCHK(c, hipMemsetAsync(c->u32s.p + 16, 0, 2 * kStatShapes * sizeof(uint32_t), c->st));
-    launch_brick_stats(c->g, sh, c->cell_n.p, c->u32s.p + 16, c->st);
-    HIPCHK(c, hipGetLastError());
     uint32_t most[2 * kStatShapes];
-    int e;
-    if ((e = read_u32(c, c->u32s.p + 16, most, 2 * kStatShapes))) return e;
+    if (c->early.n) {
+      std::copy(c->early_sizes, c->early_sizes + 2 * kStatShapes, most);
+      c->early.n = 0;
+    } else {
+      HIPCHK(c, hipMemsetAsync(c->u32s.p + 16, 0, 2 * kStatShapes * sizeof(uint32_t), c->st));
+      launch_brick_stats(c->g, sh, c->cell_n.p, nullptr, c->u32s.p + 16, c->st);
+      HIPCHK(c, hipGetLastError());
+      int e;
+      if ((e = read_u32(c, c->u32s.p + 16, most, 2 * kStatShapes))) return e;
+    }
     for (uint32_t k = 0; k < sh.n; k++) {
       BrickParams& bp = sh.shape[k];
       // head room for later rebuilds of a batched box (brick_margin > 1): atoms may regroup
@@ -408,9 +461,8 @@ int op_nbh_brick(xnb_ctx* c, double nbh_dist, const xnb_chunk_neighbors_config& 
   const double max2 = nbh_dist * nbh_dist;
   int e;
   uint32_t cap = (c->nbr_cap + list_granule() - 1) / list_granule() * list_granule();
-  // four lanes an atom: lists of the prefiltered build, for a box run by itself
-  const bool quads = (c->brick_lanes ? c->brick_lanes == (int)kQuad : c->N <= kQuadAtoms) && !c->batch_shapes && c->nbh_prefilter &&
-                     !cfg.half_symmetric && !cfg.skip_ghosts;
+  const bool quads = quad_lists(c, cfg);
+  bool clear = !c->early.n;  // a full update's move cleared the words below
   for (int attempt = 0; attempt < 3; attempt++) {
     BrickParams bp;
     if ((e = choose_bricks(c, cap, quads, bp))) return e;
@@ -419,8 +471,8 @@ int op_nbh_brick(xnb_ctx* c, double nbh_dist, const xnb_chunk_neighbors_config& 
     if ((e = dalloc(c, c->breg, brick_reg_words(bp)))) return e;
     if ((e = dalloc(c, c->blane, (size_t)bp.nbricks * bp.T))) return e;
     bind_regions(c, bp, c->derive_ghosts);
-    HIPCHK(c, hipMemsetAsync(c->u32s.p + 2, 0, sizeof(uint32_t), c->st));
-    HIPCHK(c, hipMemsetAsync(c->u32s.p + 6, 0, sizeof(uint32_t), c->st));
+    if (clear) HIPCHK(c, hipMemsetAsync(c->u32s.p + 2, 0, 5 * sizeof(uint32_t), c->st));
+    clear = true;
     tstart(c, XNB_TIMER_NBH);
     hipError_t he = launch_nbh_brick(c->g, bp, c->A.r, c->cell_off.p, c->cell_n.p, max2, pc, cfg.half_symmetric, cfg.skip_ghosts,
                                      c->nbh_prefilter, c->blist.p, c->bcnt.p, c->u32s.p + 2, c->st);
@@ -452,7 +504,7 @@ int op_nbh(xnb_ctx* c, double nbh_dist, const xnb_chunk_neighbors_config& cfg, i
   if (lay > 15) return fail(c, XNB_E_ARG, "neighbour distance spans more than 15 cells");
   int e;
   c->lists_pruned = false;
-  if (!all_cells && lay == 1 && c->g.gl >= 1 && c->use_bricks && c->N > 0) {
+  if (brick_lists(c, nbh_dist, all_cells)) {
     const PairCut none{};
     e = op_nbh_brick(c, nbh_dist, cfg, (pc && !cfg.half_symmetric && !cfg.skip_ghosts) ? *pc : none);
     if (e != NOT_APPLICABLE) return e;
@@ -542,10 +594,12 @@ int launch_force_multimat(xnb_ctx* c, int precision, const LJMulti& mm, int ntyp
 
 int full_update(xnb_ctx* c, bool forces, const PairCut* pc) {
   int e;
-  if ((e = op_move(c, forces, false))) return e;
-  if ((e = op_amr(c, kSubGridDensity, forces))) return e;
-  if ((e = op_backup(c))) return e;
-  if ((e = op_ghost_all(c, true, forces))) return e;
+  if ((e = op_move(c, forces, false, true))) return e;
+  if ((e = op_amr(c, kSubGridDensity, forces, true))) return e;
+  if ((e = op_ghost_all(c, true, forces, true))) {
+    c->early.n = 0;
+    return e;
+  }
   c->derive_ghosts = true;
   xnb_chunk_neighbors_config cfg{1, 0, 0, 0, 0};
   return op_nbh(c, c->nbh_dist_lab, cfg, 0, pc);

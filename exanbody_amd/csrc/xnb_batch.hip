@@ -401,7 +401,8 @@ hipError_t launch_step(xnb_batch* B, const uint32_t* W, const StepLayout& L, boo
   if (L.nreb) {
     launch_batch_zero_words(B->dwords.p, W + L.o_list, L.nreb, B->st);
     launch_batch_zero_words(B->amr_count.p, W + L.o_zero, 1, B->st);  // its entry is box 0: words 0..3
-    launch_batch_move(B->dF.p, W + L.o_rs, (uint32_t)L.n_rs, W + L.o_rc, (uint32_t)L.n_rc, W + L.o_list, L.nreb, L.par, B->st);
+    launch_batch_move(B->dF.p, W + L.o_rs, (uint32_t)L.n_rs, W + L.o_rc, (uint32_t)L.n_rc, W + L.o_list, L.nreb,
+                      B->amr_list.p, B->amr_count.p, L.par, B->st);
     launch_batch_ghosts(B->dF.p, W + L.o_rs, (uint32_t)L.n_rs, W + L.o_rc, (uint32_t)L.n_rc, W + L.o_rg, (uint32_t)L.n_rg,
                         W + L.o_list, L.nreb, B->amr_list.p, B->amr_count.p, L.par, B->st);
     const hipError_t he = launch_split(B, L.lb.size(), 0, [&](size_t i, hipStream_t s) {

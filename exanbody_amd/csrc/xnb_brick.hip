@@ -524,7 +524,7 @@ __global__ void __launch_bounds__(1024) k_brick_regions(Geom g, BrickParams bp, 
 // after another (one thread a brick: 29 us a launch at 250 bricks of 144 region cells, 18 us at
 // a dozen), and one launch with one read-back serves all the shapes that are tried.
 __global__ void __launch_bounds__(256) k_brick_stats(Geom g, BrickShapes sh, const uint32_t* __restrict__ cell_n,
-                                                     uint32_t* __restrict__ out) {
+                                                     const uint32_t* __restrict__ ghosts, uint32_t* __restrict__ out) {
   __shared__ uint32_t wmax[4][2];
   const BrickParams bp = sh.shape[blockIdx.y];
   const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
@@ -537,7 +537,8 @@ __global__ void __launch_bounds__(256) k_brick_stats(Geom g, BrickShapes sh, con
                 rk = (int)(c / ((uint32_t)bp.RX * (uint32_t)bp.RY));
       const int gi = P.gi0 - 1 + ri, gj = P.gj0 - 1 + rj, gk = P.gk0 - 1 + rk;
       if (ri > P.ni + 1 || rj > P.nj + 1 || rk > P.nk + 1 || gi >= g.di || gj >= g.dj || gk >= g.dk) continue;
-      const uint32_t n = cell_n[cell_index(g, gi, gj, gk)];
+      const uint32_t* const src = ghosts && is_ghost(g, gi, gj, gk) ? ghosts : cell_n;
+      const uint32_t n = src[cell_index(g, gi, gj, gk)];
       R += n;
       if (ri >= 1 && ri <= P.ni && rj >= 1 && rj <= P.nj && rk >= 1 && rk <= P.nk) nb += n;
     }
@@ -1645,10 +1646,11 @@ uint32_t brick_force_layout(BrickParams& bp, bool types) {
 
 size_t brick_reg_words(const BrickParams& bp) { return (size_t)bp.nbricks * (bp.Rmax + 1u); }
 
-void launch_brick_stats(const Geom& g, const BrickShapes& sh, const uint32_t* cell_n, uint32_t* out, hipStream_t st) {
+void launch_brick_stats(const Geom& g, const BrickShapes& sh, const uint32_t* cell_n, const uint32_t* ghosts, uint32_t* out,
+                        hipStream_t st) {
   uint32_t most = 0;
   for (uint32_t k = 0; k < sh.n; k++) most = std::max(most, sh.shape[k].nbricks);
-  k_brick_stats<<<dim3(std::min((most + 3) / 4, 1024u), sh.n), 256, 0, st>>>(g, sh, cell_n, out);
+  k_brick_stats<<<dim3(std::min((most + 3) / 4, 1024u), sh.n), 256, 0, st>>>(g, sh, cell_n, ghosts, out);
 }
 
 // Brick kernels keep all their LDS in the dynamic block, which then starts at LDS address 0:

@@ -89,6 +89,10 @@ struct xnb_ctx {
   bool use_bricks = true;
   BrickParams bp{};
   int brick_dims[3] = {0, 0, 0};  // 0: choose automatically
+  // first shapes of the list build a full update is about to do, looked at with its ghost count
+  // (early.n = 0: none), and their largest brick and region atom counts
+  BrickShapes early{};
+  uint32_t early_sizes[2 * kStatShapes] = {};
   int brick_lanes = 0;            // lanes per atom (1 or kQuad); 0: choose automatically
   DArr<uint16_t> blist;
   DArr<uint32_t> bcnt, breg, blane;
@@ -153,9 +157,9 @@ void swap_buffers(xnb_ctx* c);
 int ensure_capacity(xnb_ctx* c, size_t ncap, size_t keep);
 int check_ctx(xnb_ctx* c);
 int scan(xnb_ctx* c, const uint32_t* in, uint32_t n, uint32_t add, uint32_t* out);
-int op_ghost_all(xnb_ctx* c, bool move_check = false, bool forces = true);
+int op_ghost_all(xnb_ctx* c, bool move_check = false, bool forces = true, bool update = false);
 int op_backup(xnb_ctx* c);
-int op_amr(xnb_ctx* c, double density, bool forces);
+int op_amr(xnb_ctx* c, double density, bool forces, bool marked = false);
 int op_nbh(xnb_ctx* c, double nbh_dist, const xnb_chunk_neighbors_config& cfg, int all_cells, const PairCut* pc = nullptr);
 // forces false: f and ep neither carried by the move nor copied to ghosts; pc: per type-pair list radii
 int full_update(xnb_ctx* c, bool forces = true, const PairCut* pc = nullptr);

@@ -131,10 +131,10 @@ static_assert((kMaxBatchBoxes - 1) <= (0xffffffffu >> kWorkBoxShift), "box index
 void launch_batch_zero_cells(const BoxFrame* F, const uint32_t* work, uint32_t nwork, hipStream_t st);
 void launch_batch_zero_words(uint32_t* words, const uint32_t* boxes, uint32_t n, hipStream_t st);
 void launch_batch_move(BoxFrame* F, const uint32_t* wslots, uint32_t nslots, const uint32_t* wcells, uint32_t ncells,
-                       const uint32_t* boxes, uint32_t nboxes, uint32_t par, hipStream_t st);
-// rebuild_amr, backup_r, ghost_comm_scheme + ghost_update_all of the listed boxes after their
-// move; amr_list holds one word per cell of the listed boxes, *amr_count is 0 on entry; a box
-// with a cell too dense for rebuild_amr gets status bit 8
+                       const uint32_t* boxes, uint32_t nboxes, uint32_t* amr_list, uint32_t* amr_count, uint32_t par, hipStream_t st);
+// the sorting of rebuild_amr, backup_r, ghost_comm_scheme + ghost_update_all of the listed boxes after their
+// move, which listed their dense cells (amr_list: one word per cell of the listed boxes,
+// *amr_count 0 before the move; a box with a cell too dense for rebuild_amr gets status bit 8)
 void launch_batch_ghosts(BoxFrame* F, const uint32_t* wslots, uint32_t nslots, const uint32_t* wcells, uint32_t ncells,
                          const uint32_t* wghost, uint32_t nghost, const uint32_t* boxes, uint32_t nboxes, uint32_t* amr_list,
                          uint32_t* amr_count, uint32_t par, hipStream_t st);
@@ -171,16 +171,21 @@ void launch_move_scatter(uint32_t N, const PState& A, const PState& B, const uin
                          const uint32_t* newloc, const uint32_t* cell_off, const uint32_t* new_off, const uint32_t* cell_n,
                          const uint32_t* cnt_out, uint32_t* in_cur, uint32_t* in_list, uint32_t* slot_cell_B, bool forces,
                          hipStream_t st);
-void launch_move_incoming(const Geom& g, const PState& A, const PState& B, const uint32_t* new_off, const uint32_t* cell_n,
-                          const uint32_t* cnt_out, const uint32_t* cnt_in, uint32_t* in_list, uint32_t* slot_cell_B,
-                          bool forces, hipStream_t st);
-void launch_set_inner_cells(const Geom& g, const uint32_t* new_n, const uint32_t* new_off, uint32_t* cell_n, uint32_t* cell_off,
-                            hipStream_t st);
+// density > 0: also the first half of rebuild_amr (dense cells listed; *amr_count 0 on entry)
+void launch_move_finish(const Geom& g, uint32_t N, const PState& A, const PState& B, const uint32_t* mv_dst, const uint32_t* new_off,
+                        const uint32_t* new_n, const uint32_t* cnt_in, const uint32_t* in_list, uint32_t* slot_cell_B, uint32_t* cell_n,
+                        uint32_t* cell_off, bool forces, double density, uint32_t* amr_list, uint32_t* amr_count, uint32_t* too_dense,
+                        hipStream_t st);
+// the move's per-cell counters and the words of u32s whose bit is set in `words` = 0
+void launch_move_zero(uint32_t ncells, uint32_t* cnt_out, uint32_t* cnt_in, uint32_t* in_cur, uint32_t* u32s, uint32_t words,
+                      hipStream_t st);
+void launch_backup_ghost_count(const Geom& g, uint32_t N, const double4* r, const uint32_t* slot_cell, uint32_t* backup,
+                               const uint32_t* cell_off, const uint32_t* cell_n, uint32_t* gcnt, hipStream_t st);
 // rebuild_amr: dense inner cells of A sorted by sub-cell, through B (spare) and back.  list: one
-// word per cell; *count must be 0 on entry; a cell of more than 4096 particles sets bit 2 of
+// word per cell; *count must be 0 on entry, or marked set and the list that of the move; a cell of more than 4096 particles sets bit 2 of
 // *too_dense and stays unsorted
 void launch_rebuild_amr(const Geom& g, double density, const PState& A, const PState& B, const uint32_t* cell_off,
-                        const uint32_t* cell_n, uint32_t* list, uint32_t* count, uint32_t* too_dense, bool forces, hipStream_t st);
+                        const uint32_t* cell_n, uint32_t* list, uint32_t* count, uint32_t* too_dense, bool forces, bool marked, hipStream_t st);
 // sub_grid_density of rebuild_amr in the reference's update deck (update-particles.msp:8-11),
 // used by the run loops and batches
 constexpr double kSubGridDensity = 6.5;
@@ -241,7 +246,9 @@ struct BrickShapes {
   uint32_t n;
   BrickParams shape[kStatShapes];
 };
-void launch_brick_stats(const Geom& g, const BrickShapes& sh, const uint32_t* cell_n, uint32_t* out, hipStream_t st);
+// ghosts: the ghost cells' counts (null: cell_n holds them)
+void launch_brick_stats(const Geom& g, const BrickShapes& sh, const uint32_t* cell_n, const uint32_t* ghosts, uint32_t* out,
+                        hipStream_t st);
 // prefilter: the unfiltered builds test candidates in FP32 with an FP64 band (the same lists)
 hipError_t launch_nbh_brick(const Geom& g, BrickParams bp, const double4* r, const uint32_t* cell_off, const uint32_t* cell_n, double max2,
                             const PairCut& pc, int half_symmetric, int skip_ghosts, bool prefilter, uint16_t* blist, uint32_t* bcnt,

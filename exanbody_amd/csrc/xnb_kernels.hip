@@ -9,6 +9,8 @@
 // contraction.  Explicit fma() is used only in the mixed-precision force kernel.
 #include "xnb_kernels.h"
 
+#include <algorithm>
+
 namespace xnb {
 
 // ----------------------------------------------------------------------------- scans
@@ -90,11 +92,54 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_scan_apply(const uint32_t* in,
   }
 }
 
+// One workgroup, 8 items a thread and tile: up to kScanOneBlock items take one launch of a few
+// microseconds where the three kernels above take three of 4 us each, one after another.
+static constexpr uint32_t kScanOneBlock = 32768;
+__global__ void __launch_bounds__(1024) k_scan_one_block(const uint32_t* in, uint32_t n, uint32_t add, uint32_t* out,
+                                                         uint32_t* total) {
+  __shared__ uint32_t wsum[16];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  uint32_t carry = 0;
+  for (uint32_t tile = 0; tile < n; tile += 1024u * SCAN_ITEMS) {
+    const uint32_t base = tile + threadIdx.x * SCAN_ITEMS;
+    uint32_t v[SCAN_ITEMS], s = 0;
+#pragma unroll
+    for (int q = 0; q < SCAN_ITEMS; q++) {
+      v[q] = base + q < n ? in[base + q] : 0u;
+      s += v[q];
+    }
+    uint32_t x = s;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t y = __shfl_up(x, o, 64);
+      if (lane >= o) x += y;
+    }
+    if (lane == 63) wsum[w] = x;
+    __syncthreads();
+    uint32_t off = carry + add + x - s;
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+      if (q < w) off += wsum[q];
+      carry += wsum[q];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < SCAN_ITEMS; q++) {
+      if (base + q < n) out[base + q] = off;
+      off += v[q];
+    }
+  }
+  if (threadIdx.x == 0) *total = carry;
+}
+
 // in and out may alias.  bsum needs ceil(n/SCAN_TILE) <= SCAN_TILE entries.
 void scan_exclusive(const uint32_t* in, uint32_t n, uint32_t add, uint32_t* out, uint32_t* bsum, uint32_t* total,
                     hipStream_t st) {
-  uint32_t nb = (n + SCAN_TILE - 1) / SCAN_TILE;
-  if (nb == 0) nb = 1;
+  if (n <= kScanOneBlock) {
+    k_scan_one_block<<<1, 1024, 0, st>>>(in, n, add, out, total);
+    return;
+  }
+  const uint32_t nb = (n + SCAN_TILE - 1) / SCAN_TILE;
   k_scan_tile_sums<<<nb, SCAN_THREADS, 0, st>>>(in, n, bsum);
   k_scan_bsums<<<1, SCAN_THREADS, 0, st>>>(bsum, nb, total);
   k_scan_apply<<<nb, SCAN_THREADS, 0, st>>>(in, n, bsum, add, out);
@@ -159,7 +204,46 @@ __global__ void k_move_flag(Geom g, uint32_t N, const double4* __restrict__ r, c
   move_flag_item(g, N, r, slot_cell, mv_dst, cnt_out, cnt_in, err, s);
 }
 
-// one thread per cell: swap-with-last packing (move_particles_across_cells.h:186-209)
+__device__ inline uint32_t top_bit(unsigned long long x) { return 63u - (uint32_t)__builtin_clzll(x); }
+__device__ inline uint32_t top_bit(unsigned __int128 x) {
+  const unsigned long long hi = (unsigned long long)(x >> 64);
+  return hi ? 64u + top_bit(hi) : top_bit((unsigned long long)x);
+}
+
+// Swap-with-last packing of a cell of n particles, at most the bits of M: from the last index
+// down, the place of a particle that left takes the cell's last one.  Who stayed and which
+// places were refilled are bits, so the only loop over memory that waits for itself is the one
+// over the few particles that left.
+template <class M>
+__device__ inline void move_pack_bits(const uint32_t* __restrict__ dst, uint32_t* __restrict__ pk, uint32_t* __restrict__ newloc,
+                                      uint32_t n) {
+  const M one = 1;
+  M stay = 0, left = 0, filled = 0;
+#pragma unroll 8
+  for (uint32_t q = 0; q < n; q++) {
+    const bool s = dst[q] == NONE;
+    stay |= (M)s << q;
+    left |= (M)!s << q;
+  }
+  uint32_t m = n;
+  while (left) {
+    const uint32_t q = top_bit(left);
+    left ^= one << q;
+    if (q + 1 < m) {
+      const uint32_t last = (uint32_t)(filled >> (m - 1)) & 1u ? pk[m - 1] : m - 1;
+      pk[q] = last;
+      newloc[last] = q;  // moved again by a later q: overwritten
+      filled |= one << q;
+    }
+    --m;
+  }
+  for (uint32_t q = 0; q < m; q++)
+    if ((uint32_t)(stay >> q) & 1u) newloc[q] = q;
+}
+
+// One thread per cell: packing (move_particles_across_cells.h:186-209).  Written out and searched
+// particle by particle in memory, which cells of more than 128 particles still do, a launch took
+// 36 us for a box of 500 atoms (62 a cell) and 23 us for one of 131,072.
 __device__ inline void move_pack_item(Geom g, const uint32_t* __restrict__ cell_off, const uint32_t* __restrict__ cell_n,
                             const uint32_t* __restrict__ cnt_out, const uint32_t* __restrict__ cnt_in,
                             const uint32_t* __restrict__ mv_dst, uint32_t* __restrict__ pk, uint32_t* __restrict__ newloc,
@@ -173,6 +257,11 @@ __device__ inline void move_pack_item(Geom g, const uint32_t* __restrict__ cell_
   const uint32_t n = cell_n[c], off = cell_off[c], nout = cnt_out[c];
   new_n[c] = n - nout + cnt_in[c];
   if (nout == 0) return;  // every particle keeps its index (the scatter derives it)
+  if (n <= 128) {
+    if (n <= 64) move_pack_bits<unsigned long long>(mv_dst + off, pk + off, newloc + off, n);
+    else move_pack_bits<unsigned __int128>(mv_dst + off, pk + off, newloc + off, n);
+    return;
+  }
   for (uint32_t q = 0; q < n; q++) pk[off + q] = (mv_dst[off + q] == NONE) ? q : NONE;
   int m = (int)n;
   for (int q = (int)n - 1; q >= 0; q--) {
@@ -242,57 +331,34 @@ __global__ void k_move_scatter(uint32_t N, PState A, PState B, const uint32_t* _
                     forces != 0);
 }
 
-// one thread per cell: order incoming movers by source slot, copy them with wrapped positions
-__device__ inline void move_incoming_item(Geom g, PState A, PState B, const uint32_t* __restrict__ new_off,
-                                const uint32_t* __restrict__ cell_n, const uint32_t* __restrict__ cnt_out,
-                                const uint32_t* __restrict__ cnt_in, uint32_t* __restrict__ in_list,
-                                uint32_t* __restrict__ slot_cell_B, uint32_t c, bool forces) {
-  const uint32_t nin = cnt_in[c];
-  if (nin == 0) return;
-  const uint32_t b = new_off[c] + (cell_n[c] - cnt_out[c]);
-  for (uint32_t q = 1; q < nin; q++) {  // insertion sort (few movers per cell)
-    uint32_t v = in_list[b + q];
-    int p = (int)q - 1;
-    while (p >= 0 && in_list[b + p] > v) {
-      in_list[b + p + 1] = in_list[b + p];
-      --p;
-    }
-    in_list[b + p + 1] = v;
-  }
-  for (uint32_t q = 0; q < nin; q++) {
-    const uint32_t s = in_list[b + q], t = b + q;
-    copy_particle(A, s, B, t, forces);
-    double4 p = A.r[s];
-    int li, lj, lk;
-    periodic_location(g, p.x, p.y, p.z, li, lj, lk);
-    B.r[t] = p;
-    slot_cell_B[t] = c;
-  }
+// One thread per source slot: a mover's place among the incoming of its cell is the number of
+// them from lower slots (their list is in no order); it is copied there with its position
+// wrapped.  One thread per destination cell sorted its list in memory first and then copied
+// mover by mover (500 atoms 18 us a launch, 8,388,608 atoms 93 us).
+__device__ inline void move_incoming_item(Geom g, PState A, PState B, const uint32_t* __restrict__ mv_dst,
+                                const uint32_t* __restrict__ new_off, const uint32_t* __restrict__ new_n,
+                                const uint32_t* __restrict__ cnt_in, const uint32_t* __restrict__ in_list,
+                                uint32_t* __restrict__ slot_cell_B, uint32_t s, bool forces) {
+  const uint32_t c = mv_dst[s];
+  if (c == NONE) return;
+  const uint32_t nin = cnt_in[c], b = new_off[c] + new_n[c] - nin;
+  uint32_t t = b;
+  for (uint32_t q = 0; q < nin; q++) t += in_list[b + q] < s ? 1u : 0u;
+  copy_particle(A, s, B, t, forces);
+  double4 p = A.r[s];
+  int li, lj, lk;
+  periodic_location(g, p.x, p.y, p.z, li, lj, lk);
+  B.r[t] = p;
+  slot_cell_B[t] = c;
 }
 
-__global__ void k_move_incoming(Geom g, PState A, PState B, const uint32_t* __restrict__ new_off,
-                                const uint32_t* __restrict__ cell_n, const uint32_t* __restrict__ cnt_out,
-                                const uint32_t* __restrict__ cnt_in, uint32_t* __restrict__ in_list,
-                                uint32_t* __restrict__ slot_cell_B, int forces) {
-  const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= g.ncells) return;
-  move_incoming_item(g, A, B, new_off, cell_n, cnt_out, cnt_in, in_list, slot_cell_B, c, forces != 0);
-}
-
-__device__ inline void set_inner_cells_item(uint32_t ncells, const uint32_t* __restrict__ new_n, const uint32_t* __restrict__ new_off,
-                                  Geom g, uint32_t* __restrict__ cell_n, uint32_t* __restrict__ cell_off, uint32_t c) {
+__device__ inline void set_inner_cells_item(const Geom& g, const uint32_t* __restrict__ new_n, const uint32_t* __restrict__ new_off,
+                                            uint32_t* __restrict__ cell_n, uint32_t* __restrict__ cell_off, uint32_t c) {
   int i, j, k;
   cell_ijk(g, c, i, j, k);
   if (is_ghost(g, i, j, k)) return;
   cell_n[c] = new_n[c];
   cell_off[c] = new_off[c];
-}
-
-__global__ void k_set_inner_cells(uint32_t ncells, const uint32_t* __restrict__ new_n, const uint32_t* __restrict__ new_off,
-                                  Geom g, uint32_t* __restrict__ cell_n, uint32_t* __restrict__ cell_off) {
-  const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= ncells) return;
-  set_inner_cells_item(ncells, new_n, new_off, g, cell_n, cell_off, c);
 }
 
 // -------------------------------------------------------------------- rebuild_amr
@@ -366,6 +432,7 @@ __device__ inline void amr_sort_wave(const Geom& g, double density, const PState
   for (uint32_t p = lane; p < n; p += 64) {
     const uint32_t kp = keys[p];
     uint32_t rank = 0;
+#pragma unroll 8
     for (uint32_t t = 0; t < n; t++) {
       const uint32_t kt = keys[t];
       rank += (kt < kp || (kt == kp && t < p)) ? 1u : 0u;
@@ -379,6 +446,31 @@ __device__ inline void amr_back_wave(const PState& A, const PState& B, const uin
                                      const uint32_t* __restrict__ cell_n, uint32_t c, bool forces) {
   const uint32_t n = cell_n[c], off = cell_off[c];
   for (uint32_t p = threadIdx.x; p < n; p += 64) copy_particle(B, off + p, A, off + p, forces);
+}
+
+// The end of a move: thread t copies mover t and closes cell t (its new range, and, with
+// density > 0, its mark for rebuild_amr).
+__global__ void __launch_bounds__(256) k_move_finish(Geom g, uint32_t N, PState A, PState B, const uint32_t* __restrict__ mv_dst,
+                                                     const uint32_t* __restrict__ new_off, const uint32_t* __restrict__ new_n,
+                                                     const uint32_t* __restrict__ cnt_in, const uint32_t* __restrict__ in_list,
+                                                     uint32_t* __restrict__ slot_cell_B, uint32_t* __restrict__ cell_n,
+                                                     uint32_t* __restrict__ cell_off, int forces, double density,
+                                                     uint32_t* __restrict__ list, uint32_t* __restrict__ count,
+                                                     uint32_t* __restrict__ too_dense) {
+  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < g.ncells) {
+    set_inner_cells_item(g, new_n, new_off, cell_n, cell_off, t);
+    if (density > 0.0) amr_mark_item(g, density, new_n, t, 0u, list, count, too_dense, 2u);
+  }
+  if (t < N) move_incoming_item(g, A, B, mv_dst, new_off, new_n, cnt_in, in_list, slot_cell_B, t, forces != 0);
+}
+
+// what a move starts from: its per-cell counters and the words given by bits of `words`
+__global__ void __launch_bounds__(256) k_move_zero(uint32_t ncells, uint32_t* __restrict__ cnt_out, uint32_t* __restrict__ cnt_in,
+                                                   uint32_t* __restrict__ in_cur, uint32_t* __restrict__ u32s, uint32_t words) {
+  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < ncells) cnt_out[t] = cnt_in[t] = in_cur[t] = 0;
+  if (t < 32 && (words >> t) & 1u) u32s[t] = 0;
 }
 
 __global__ void k_amr_mark(Geom g, double density, const uint32_t* __restrict__ cell_n, uint32_t* __restrict__ list,
@@ -569,6 +661,20 @@ __global__ void k_backup_r(Geom g, uint32_t N, const double4* __restrict__ r, co
   const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= N) return;
   backup_r_item(g, N, r, slot_cell, backup, s);
+}
+
+// backup_r in the first nb_slots workgroups, the ghost cells' counts in the others
+__global__ void __launch_bounds__(256) k_backup_ghost_count(Geom g, uint32_t N, uint32_t nb_slots, const double4* __restrict__ r,
+                                                            const uint32_t* __restrict__ slot_cell, uint32_t* __restrict__ backup,
+                                                            const uint32_t* __restrict__ cell_off, const uint32_t* __restrict__ cell_n,
+                                                            uint32_t* __restrict__ gcnt) {
+  if (blockIdx.x < nb_slots) {
+    const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s < N) backup_r_item(g, N, r, slot_cell, backup, s);
+    return;
+  }
+  uint32_t c;
+  if (ghost_wave_cell(g, (blockIdx.x - nb_slots) * blockDim.x + threadIdx.x, c)) ghost_count_wave(g, r, cell_off, cell_n, gcnt, c);
 }
 
 // particle_displ_over (particle_displ_over.cu:38-77)
@@ -1160,19 +1266,28 @@ void launch_move_scatter(uint32_t N, const PState& A, const PState& B, const uin
   k_move_scatter<<<nblk(N, 256), 256, 0, st>>>(N, A, B, slot_cell, mv_dst, newloc, cell_off, new_off, cell_n, cnt_out, in_cur,
                                                in_list, slot_cell_B, forces ? 1 : 0);
 }
-void launch_move_incoming(const Geom& g, const PState& A, const PState& B, const uint32_t* new_off, const uint32_t* cell_n,
-                          const uint32_t* cnt_out, const uint32_t* cnt_in, uint32_t* in_list, uint32_t* slot_cell_B,
-                          bool forces, hipStream_t st) {
-  k_move_incoming<<<nblk(g.ncells, 128), 128, 0, st>>>(g, A, B, new_off, cell_n, cnt_out, cnt_in, in_list, slot_cell_B,
-                                                        forces ? 1 : 0);
+void launch_move_finish(const Geom& g, uint32_t N, const PState& A, const PState& B, const uint32_t* mv_dst, const uint32_t* new_off,
+                        const uint32_t* new_n, const uint32_t* cnt_in, const uint32_t* in_list, uint32_t* slot_cell_B, uint32_t* cell_n,
+                        uint32_t* cell_off, bool forces, double density, uint32_t* amr_list, uint32_t* amr_count, uint32_t* too_dense,
+                        hipStream_t st) {
+  k_move_finish<<<nblk(std::max(N, g.ncells), 256), 256, 0, st>>>(g, N, A, B, mv_dst, new_off, new_n, cnt_in, in_list, slot_cell_B,
+                                                                   cell_n, cell_off, forces ? 1 : 0, density, amr_list, amr_count,
+                                                                   too_dense);
 }
-void launch_set_inner_cells(const Geom& g, const uint32_t* new_n, const uint32_t* new_off, uint32_t* cell_n, uint32_t* cell_off,
-                            hipStream_t st) {
-  k_set_inner_cells<<<nblk(g.ncells, 256), 256, 0, st>>>(g.ncells, new_n, new_off, g, cell_n, cell_off);
+void launch_move_zero(uint32_t ncells, uint32_t* cnt_out, uint32_t* cnt_in, uint32_t* in_cur, uint32_t* u32s, uint32_t words,
+                      hipStream_t st) {
+  k_move_zero<<<nblk(std::max(ncells, 32u), 256), 256, 0, st>>>(ncells, cnt_out, cnt_in, in_cur, u32s, words);
+}
+void launch_backup_ghost_count(const Geom& g, uint32_t N, const double4* r, const uint32_t* slot_cell, uint32_t* backup,
+                               const uint32_t* cell_off, const uint32_t* cell_n, uint32_t* gcnt, hipStream_t st) {
+  const uint32_t nb_slots = (N + 255) / 256, nb_ghost = (ghost_cell_count(g) * 64u + 255) / 256;
+  if (nb_slots + nb_ghost)
+    k_backup_ghost_count<<<nb_slots + nb_ghost, 256, 0, st>>>(g, N, nb_slots, r, slot_cell, backup, cell_off, cell_n, gcnt);
 }
 void launch_rebuild_amr(const Geom& g, double density, const PState& A, const PState& B, const uint32_t* cell_off,
-                        const uint32_t* cell_n, uint32_t* list, uint32_t* count, uint32_t* too_dense, bool forces, hipStream_t st) {
-  k_amr_mark<<<nblk(g.ncells, 256), 256, 0, st>>>(g, density, cell_n, list, count, too_dense);
+                        const uint32_t* cell_n, uint32_t* list, uint32_t* count, uint32_t* too_dense, bool forces, bool marked,
+                        hipStream_t st) {
+  if (!marked) k_amr_mark<<<nblk(g.ncells, 256), 256, 0, st>>>(g, density, cell_n, list, count, too_dense);
   k_amr_sort<<<kAmrGrid, 64, 0, st>>>(g, density, A, B, cell_off, cell_n, list, count, forces ? 1 : 0);
   k_amr_back<<<kAmrGrid, 64, 0, st>>>(A, B, cell_off, cell_n, list, count, forces ? 1 : 0);
 }
@@ -1445,34 +1560,28 @@ __global__ void __launch_bounds__(kBatchSlotBlock) kb_move_scatter(const BoxFram
 
 __global__ void __launch_bounds__(kBatchSlotBlock) kb_move_incoming(const BoxFrame* __restrict__ F, const uint32_t* __restrict__ work,
                                                                      uint32_t par) {
-  uint32_t box, c;
-  if (!batch_item(work, box, c)) return;
+  uint32_t box, s;
+  if (!batch_item(work, box, s)) return;
   const BoxFrame& f = F[box];
-  if (c >= f.g.ncells) return;
+  if (s >= f.N) return;
   const FrameState X = frame_state(f, par);
-  move_incoming_item(f.g, X.A, X.B, f.new_off, f.cell_n, f.cnt_out, f.cnt_in, f.in_list, X.scB, c, false);
+  move_incoming_item(f.g, X.A, X.B, f.mv_dst, f.new_off, f.new_n, f.cnt_in, f.in_list, X.scB, s, false);
 }
 
-__global__ void __launch_bounds__(kBatchSlotBlock) kb_set_inner_cells(const BoxFrame* __restrict__ F, const uint32_t* __restrict__ work) {
+// cells of the rebuilding boxes after their move: new ranges, and dense cells listed for
+// rebuild_amr (entry box << kWorkBoxShift | cell)
+__global__ void __launch_bounds__(kBatchSlotBlock) kb_close_cells(const BoxFrame* __restrict__ F, const uint32_t* __restrict__ work,
+                                                                  uint32_t* __restrict__ list, uint32_t* __restrict__ count) {
   uint32_t box, c;
   if (!batch_item(work, box, c)) return;
   const BoxFrame& f = F[box];
   if (c >= f.g.ncells) return;
-  set_inner_cells_item(f.g.ncells, f.new_n, f.new_off, f.g, f.cell_n, f.cell_off, c);
+  set_inner_cells_item(f.g, f.new_n, f.new_off, f.cell_n, f.cell_off, c);
+  amr_mark_item(f.g, kSubGridDensity, f.new_n, c, box << kWorkBoxShift, list, count, f.words + 0, 8u);
 }
 
-// rebuild_amr of the rebuilding boxes (after kb_flip: X.A current, X.B spare): dense cells of
-// every box listed (entry box << kWorkBoxShift | cell) over the cells work table, then sorted and
-// copied back by one wave each
-__global__ void __launch_bounds__(kBatchSlotBlock) kb_amr_mark(const BoxFrame* __restrict__ F, const uint32_t* __restrict__ work,
-                                                                uint32_t* __restrict__ list, uint32_t* __restrict__ count) {
-  uint32_t box, c;
-  if (!batch_item(work, box, c)) return;
-  const BoxFrame& f = F[box];
-  if (c >= f.g.ncells) return;
-  amr_mark_item(f.g, kSubGridDensity, f.cell_n, c, box << kWorkBoxShift, list, count, f.words + 0, 8u);
-}
-
+// rebuild_amr of the listed cells (after kb_flip: X.A current, X.B spare): sorted and copied
+// back by one wave each
 __global__ void __launch_bounds__(64) kb_amr_sort(const BoxFrame* __restrict__ F, const uint32_t* __restrict__ list,
                                                   const uint32_t* __restrict__ count, uint32_t par) {
   __shared__ uint32_t keys[kAmrMaxKeys];
@@ -1576,15 +1685,15 @@ void launch_batch_zero_cells(const BoxFrame* F, const uint32_t* work, uint32_t n
 }
 
 void launch_batch_move(BoxFrame* F, const uint32_t* wslots, uint32_t nslots, const uint32_t* wcells, uint32_t ncells,
-                       const uint32_t* boxes, uint32_t nboxes, uint32_t par, hipStream_t st) {
+                       const uint32_t* boxes, uint32_t nboxes, uint32_t* amr_list, uint32_t* amr_count, uint32_t par, hipStream_t st) {
   if (!nboxes) return;
   launch_batch_zero_cells(F, wcells, ncells, st);
   if (nslots) kb_move_flag<<<nslots, kBatchSlotBlock, 0, st>>>(F, wslots, par);
   if (ncells) kb_move_pack<<<ncells, kBatchSlotBlock, 0, st>>>(F, wcells);
   kb_scan_cells<<<nboxes, 1024, 0, st>>>(F, boxes, 0);
   if (nslots) kb_move_scatter<<<nslots, kBatchSlotBlock, 0, st>>>(F, wslots, par);
-  if (ncells) kb_move_incoming<<<ncells, kBatchSlotBlock, 0, st>>>(F, wcells, par);
-  if (ncells) kb_set_inner_cells<<<ncells, kBatchSlotBlock, 0, st>>>(F, wcells);
+  if (nslots) kb_move_incoming<<<nslots, kBatchSlotBlock, 0, st>>>(F, wslots, par);
+  if (ncells) kb_close_cells<<<ncells, kBatchSlotBlock, 0, st>>>(F, wcells, amr_list, amr_count);
   kb_flip<<<(nboxes + 255) / 256, 256, 0, st>>>(F, boxes, nboxes);
 }
 
@@ -1593,7 +1702,6 @@ void launch_batch_ghosts(BoxFrame* F, const uint32_t* wslots, uint32_t nslots, c
                          uint32_t* amr_count, uint32_t par, hipStream_t st) {
   if (!nboxes) return;
   if (ncells) {
-    kb_amr_mark<<<ncells, kBatchSlotBlock, 0, st>>>(F, wcells, amr_list, amr_count);
     kb_amr_sort<<<kAmrGrid, 64, 0, st>>>(F, amr_list, amr_count, par);
     kb_amr_back<<<kAmrGrid, 64, 0, st>>>(F, amr_list, amr_count, par);
   }
