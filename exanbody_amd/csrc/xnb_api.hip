@@ -233,7 +233,7 @@ int scan(xnb_ctx* c, const uint32_t* in, uint32_t n, uint32_t add, uint32_t* out
 
 // words of u32s cleared by a move: its flags, the rebuild_amr count, and those of the list
 // build that follows in a full update (longest list, brick status, brick sizes)
-constexpr uint32_t kMoveWords = 1u << 0, kAmrWords = 1u << 8, kBuildWords = 1u << 2 | 1u << 6 | 0xffu << 16;
+constexpr uint32_t kMoveWords = 1u << 0 | 1u << 10, kAmrWords = 1u << 8, kBuildWords = 1u << 2 | 1u << 6 | 0xffu << 16;
 
 // check false: the out-of-domain flag (u32s[0]) is left for the caller to read (op_ghost_all
 // reads it with the ghost count in one transfer).  update: the move of a full update, which also
@@ -1379,6 +1379,8 @@ int xnb_init(xnb_ctx* c, const xnb_lj_params* p, double rcut, double rcut_inc, i
 
 namespace xnb_impl {
 
+constexpr int64_t kMaxAhead = 32;  // steps launched ahead of a read-back (h_u64 holds their counts)
+
 // The step loop of xnb_run / xnb_run_multimat (mm == nullptr: single-material LJ).
 int run_loop(xnb_ctx* c, xnb_run_params* p, const LJMulti* mm, int ntypes, const double* rcut_pair) {
   int e;
@@ -1412,10 +1414,44 @@ int run_loop(xnb_ctx* c, xnb_run_params* p, const LJMulti* mm, int ntypes, const
   if (p->steps > 0) {
     if ((e = dalloc(c, c->step_counts, (size_t)p->steps))) return e;
     HIPCHK(c, hipMemsetAsync(c->step_counts.p, 0, (size_t)p->steps * sizeof(unsigned long long), c->st));
+    // a run that failed may have left steps halted
+    if (!interval) HIPCHK(c, hipMemsetAsync(c->u32s.p + 10, 0, sizeof(uint32_t), c->st));
   }
   std::vector<char> rebuilt(interval ? (size_t)p->steps : 0, 0);
   bool first_half_done = false;  // step's first half already done by the previous force kernel
-  for (int64_t step = 1; step <= p->steps; step++) {
+  // zero + force of `step` and what closes it
+  auto force = [&](int64_t step, const unsigned long long* guard) -> int {
+    const bool fuse = c->fuse_push && step < p->steps && c->list_kind == 1;
+    // A fused step (EPI_NEXT) stores no forces or energies: the next step overwrites them before
+    // anything reads them (its force kernel sets f = 0 + sum for every inner atom; a rebuild in
+    // between does not carry them, and the first half-step of the next step is done by this
+    // kernel from the force in registers).  The last step of a run is not fused and stores both.
+    NextStep nx{c->rB.p, c->backup.p, dt, dt2, thr2, c->step_counts.p + step, guard, c->u32s.p + 10};
+    tstart(c, XNB_TIMER_FORCE);
+    int e;
+    if (mm) e = launch_force_multimat(c, p->precision, *mm, ntypes, dth, fuse ? &nx : nullptr);
+    else e = launch_force(c, p->precision, false, true, false, p->lj.epsilon, p->lj.sigma, p->rcut, dth, fuse ? &nx : nullptr);
+    tstop(c);
+    if (e) return e;
+    if (fuse) {
+      std::swap(c->rA, c->rB);
+      bind_states(c);
+    }
+    first_half_done = fuse;
+    return XNB_OK;
+  };
+  auto refresh_ghosts = [&]() {
+    tstart(c, XNB_TIMER_GHOST);
+    launch_ghost_update_r(c->g, c->N, c->G, c->A.r, c->ghost_src.p, c->ghost_shift.p, c->st);
+    tstop(c);
+  };
+  // With the displacement trigger, steps are launched ahead of the host's look at their counts
+  // (NextStep::guard), a step that starts with a rebuild and those behind it doing nothing: one
+  // read-back of about 20 us for a group of steps instead of one a step, against some 4 us for
+  // each launch in vain.  The first group after a rebuild reaches to three quarters of the last
+  // interval, the following ones take two steps.
+  int64_t since = 0, last_interval = 4;  // steps since the last rebuild; the interval before it
+  for (int64_t step = 1; step <= p->steps;) {
     unsigned long long* cnt = c->step_counts.p + (step - 1);
     if (!first_half_done) {
       tstart(c, XNB_TIMER_PUSH);
@@ -1426,37 +1462,41 @@ int run_loop(xnb_ctx* c, xnb_run_params* p, const LJMulti* mm, int ntypes, const
     if (interval) {
       trigger = (step % p->rebuild_every) == 0;
     } else {
-      HIPCHK(c, hipMemcpyAsync(c->h_u64, cnt, sizeof(unsigned long long), hipMemcpyDeviceToHost, c->st));
+      // fused steps from `step` on, as many as a group takes; their counts and the next one's
+      int64_t ahead = 0;
+      if (!c->timing && c->fuse_push && c->list_kind == 1 && c->bp.derive) {
+        const int64_t want = std::max<int64_t>(2, last_interval * 3 / 4 - since);
+        ahead = std::max<int64_t>(0, std::min({want, p->steps - step, kMaxAhead}));
+      }
+      for (int64_t q = 0; q < ahead; q++)
+        if ((e = force(step + q, cnt + q))) return e;
+      HIPCHK(c, hipMemcpyAsync(c->h_u64, cnt, (size_t)(ahead + 1) * sizeof(unsigned long long), hipMemcpyDeviceToHost, c->st));
       HIPCHK(c, hipStreamSynchronize(c->st));
-      trigger = c->h_u64[0] > 0;
+      int64_t ran = 0;
+      while (ran < ahead && c->h_u64[ran] == 0) ran++;
+      if ((ahead - ran) & 1) {  // the halted steps wrote nothing: back to the positions of the first of them
+        std::swap(c->rA, c->rB);
+        bind_states(c);
+      }
+      step += ran;
+      since += ran;
+      cnt += ran;
+      trigger = c->h_u64[ran] > 0;
     }
     if (trigger) {
       if ((e = full_update(c, false, mm ? &pc : nullptr))) return e;  // f, ep: overwritten by this step's force kernel
       p->n_rebuilds++;
       if (interval) rebuilt[(size_t)step - 1] = 1;
+      if (since) last_interval = since;
+      since = 0;
     } else if (step == p->steps || c->list_kind != 1 || !c->bp.derive) {
       // ghost_update_r: the force of brick lists places ghosts by their sources, so only the
       // positions a run leaves behind are refreshed (131,072 atoms: 4.7 us of a 40 us step)
-      tstart(c, XNB_TIMER_GHOST);
-      launch_ghost_update_r(c->g, c->N, c->G, c->A.r, c->ghost_src.p, c->ghost_shift.p, c->st);
-      tstop(c);
+      refresh_ghosts();
     }
-    const bool fuse = c->fuse_push && step < p->steps && c->list_kind == 1;
-    // A fused step (EPI_NEXT) stores no forces or energies: the next step overwrites them before
-    // anything reads them (its force kernel sets f = 0 + sum for every inner atom; a rebuild in
-    // between does not carry them, and the first half-step of the next step is done by this
-    // kernel from the force in registers).  The last step of a run is not fused and stores both.
-    NextStep nx{c->rB.p, c->backup.p, dt, dt2, thr2, cnt + 1};
-    tstart(c, XNB_TIMER_FORCE);
-    if (mm) e = launch_force_multimat(c, p->precision, *mm, ntypes, dth, fuse ? &nx : nullptr);
-    else e = launch_force(c, p->precision, false, true, false, p->lj.epsilon, p->lj.sigma, p->rcut, dth, fuse ? &nx : nullptr);
-    tstop(c);
-    if (e) return e;
-    if (fuse) {
-      std::swap(c->rA, c->rB);
-      bind_states(c);
-    }
-    first_half_done = fuse;
+    if ((e = force(step, nullptr))) return e;
+    step++;
+    since++;
   }
   HIPCHK(c, hipGetLastError());
   if (interval && p->steps > 0) {

@@ -1172,10 +1172,20 @@ __device__ __forceinline__ void compute_pair_brick_body(const Geom& g, const Bri
   if (NEXT) wave_group_count_add(over, nx.count, L.wcnt);
 }
 
+// Whole workgroup: the launch is a step that must not run (NextStep::guard).  A workgroup that
+// misses the first one's *halt sees the same *guard.
+__device__ inline bool step_halted(const NextStep& nx) {
+  if (!nx.guard) return false;
+  const bool stop = *nx.guard != 0ull || *nx.halt != 0u;
+  if (stop && blockIdx.x == 0 && threadIdx.x == 0) *nx.halt = 1u;
+  return stop;
+}
+
 template <bool MIXED, bool ACCUM, int EPI, int U>
 __global__ void __launch_bounds__(1024) k_lj_brick(Geom g, BrickParams bp, const double4* __restrict__ r,
                                                    const uint16_t* __restrict__ blist, const uint32_t* __restrict__ bcnt,
                                                    LJConst lj, PState A, double dth, NextStep nx) {
+  if (EPI == EPI_NEXT && step_halted(nx)) return;
   const uint32_t b = brick_of_block<MIXED>(bp);
   if (b >= bp.nbricks) return;  // whole workgroup, before any barrier
   compute_pair_brick_body<LennardJonesForceFunctor<MIXED>, ACCUM, EPI, U>(g, bp, b, r, blist, bcnt,
@@ -1320,6 +1330,7 @@ template <bool MIXED, bool ACCUM, int EPI>
 __global__ void __launch_bounds__(1024) k_lj_quad_brick(Geom g, BrickParams bp, const double4* __restrict__ r,
                                                         const uint16_t* __restrict__ blist, const uint32_t* __restrict__ bcnt, LJConst lj,
                                                         PState A, double dth, NextStep nx) {
+  if (EPI == EPI_NEXT && step_halted(nx)) return;
   const uint32_t b = brick_of_block<MIXED>(bp);
   if (b >= bp.nbricks) return;  // whole workgroup, before any barrier
   lj_quad_brick_body<MIXED, ACCUM, EPI>(g, bp, b, r, blist, bcnt, lj, A, dth, nx);
@@ -1553,6 +1564,7 @@ template <bool MIXED, int NT, bool ACCUM, int EPI>
 __global__ void __launch_bounds__(1024) k_ljmm_brick(Geom g, BrickParams bp, const double4* __restrict__ r,
                                                      const uint16_t* __restrict__ blist, const uint32_t* __restrict__ bcnt, LJMulti mm,
                                                      PState A, double dth, NextStep nx) {
+  if (EPI == EPI_NEXT && step_halted(nx)) return;
   const uint32_t b = brick_of_block<MIXED>(bp);
   if (b >= bp.nbricks) return;  // whole workgroup, before any barrier
   ljmm_brick_body<MIXED, NT, ACCUM, EPI, LJB_UNROLL_B>(g, bp, b, r, blist, bcnt, mm, A, dth, nx);
@@ -1841,7 +1853,7 @@ __device__ __forceinline__ void lj_batch_case(const BoxFrame& f, uint32_t b, uin
   const uint32_t cur = (f.rcur ^ par) & 1u;
   A.r = f.rbuf[cur];
   // the next step's count: local step k = gstep - gstep0 + 1, count of step k + 1 at [k]
-  const NextStep nx{f.rbuf[cur ^ 1u], f.backup, f.dt, f.dt2, f.thr2, f.counts + (gstep - f.gstep0 + 1)};
+  const NextStep nx{f.rbuf[cur ^ 1u], f.backup, f.dt, f.dt2, f.thr2, f.counts + (gstep - f.gstep0 + 1), nullptr, nullptr};
   compute_pair_brick_body<LennardJonesForceFunctor<MIXED>, false, EPI, LJB_UNROLL_B>(
       f.g, f.bp, b, A.r, f.blist, f.bcnt, LennardJonesForceFunctor<MIXED>{f.lj}, f.lj.rc2, A, f.dth, nx);
 }

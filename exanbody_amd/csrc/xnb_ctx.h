@@ -66,7 +66,8 @@ struct xnb_ctx {
 
   // scan / scalar scratch
   DArr<uint32_t> bsum, u32s;            // u32s: [0] err, [1] scan total, [2] max count, [6] brick status, [16..23] brick stats,
-                                        // [7] ghost status, [8] rebuild_amr cell count, [9] largest particle type
+                                        // [7] ghost status, [8] rebuild_amr cell count, [9] largest particle type,
+                                        // [10] steps launched ahead were halted
   DArr<uint32_t> amr_list;              // rebuild_amr: cells to sort
   DArr<unsigned long long> u64s;        // [0] displacement count, [1..2] pair counts
   DArr<unsigned long long> step_counts; // per-step displacement counts of xnb_run

@@ -64,6 +64,10 @@ struct NextStep {
   const uint32_t* backup;
   double dt, dt2, thr2;
   unsigned long long* count;
+  // A step launched before the host knows whether it starts with a rebuild: it is left undone, and
+  // *halt set for the steps launched behind it, when its own displacement count *guard is not 0.
+  const unsigned long long* guard;  // null: the step is known to run
+  uint32_t* halt;
 };
 
 // Extra per-particle FP64 fields a grid may carry beside the fixed ones (a field set with more
