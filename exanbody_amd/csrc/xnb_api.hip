@@ -280,12 +280,6 @@ inline uint32_t grow_cap(uint32_t mx) {
   return (mx + mx / 8 + gran - 1) / gran * gran;
 }
 
-// Boxes of at most this many atoms give every atom four lanes (four atoms' lanes fill two waves
-// per SIMD of the chip; larger boxes have enough waves with one lane an atom, which takes 1.7
-// times fewer instructions).  Force and build launch with one and with four lanes: 6,912 atoms
-// FP64 20.5 and 13.6, 68 and 28 us; 27,431 atoms mixed 15.8 and 15.5, 68 and 38 us; 131,072
-// atoms FP64 36 and 50, 89 and 104 us.
-constexpr uint32_t kQuadAtoms = 32768;
 // Bricks are made smaller until there are this many (three quarters of the CUs): with fewer,
 // idle CUs cost more than the larger staged share of smaller bricks.  60,000-atom slab,
 // force: 112 bricks 70 us, 196 bricks 45 us; 131,072 atoms: 250 bricks 36 us, 500 bricks 41 us.
@@ -316,7 +310,7 @@ void list_shapes(const xnb_ctx* c, bool quads, ShapeList& l) {
     l.add(c->brick_dims, 1u, true);
   }
   if (quads)
-    for (const auto& d : quad) l.add(d, kQuad, &d == &quad[3]);
+    for (const auto& d : quad) l.add(d, kQuad, c->batch_shapes || &d == &quad[3]);
   for (int q = 0; q < 9; q++)
     if ((q != 1 && q != 2) || c->batch_shapes) l.add(wide[q], 1u, c->batch_shapes || q == 8);
 }
@@ -336,9 +330,9 @@ void next_shapes(const xnb_ctx* c, const ShapeList& l, int& at, BrickShapes& sh)
   }
 }
 
-// four lanes an atom: lists of the prefiltered build, for a box run by itself
+// four lanes an atom: lists of the prefiltered build
 bool quad_lists(const xnb_ctx* c, const xnb_chunk_neighbors_config& cfg) {
-  return (c->brick_lanes ? c->brick_lanes == (int)kQuad : c->N <= kQuadAtoms) && !c->batch_shapes && c->nbh_prefilter &&
+  return (c->brick_lanes ? c->brick_lanes == (int)kQuad : (c->batch_shapes ? c->batch_quads : c->N <= kQuadAtoms)) && c->nbh_prefilter &&
          !cfg.half_symmetric && !cfg.skip_ghosts;
 }
 
@@ -478,11 +472,14 @@ int op_nbh_brick(xnb_ctx* c, double nbh_dist, const xnb_chunk_neighbors_config& 
                                      c->nbh_prefilter, c->blist.p, c->bcnt.p, c->u32s.p + 2, c->st);
     tstop(c);
     if (he != hipSuccess) return fail(c, XNB_E_HIP, std::string("brick neighbour build: ") + hipGetErrorString(he));
-    uint32_t w[5];  // u32s[2]: longest list, u32s[6]: brick status
-    if ((e = read_u32(c, c->u32s.p + 2, w, 5))) return e;
+    uint32_t w[5] = {};  // u32s[2]: longest list, u32s[6]: brick status
+    c->build_pending = c->defer_build;
+    if (c->defer_build)
+      HIPCHK(c, hipMemcpyAsync(c->h_u32 + kPendingWords, c->u32s.p + 2, sizeof(w), hipMemcpyDeviceToHost, c->st));
+    else if ((e = read_u32(c, c->u32s.p + 2, w, 5))) return e;
     const uint32_t mx = w[0], bad = w[4];
     if (bad) return fail(c, XNB_E_STATE, "brick sizes changed between statistics and build");
-    c->max_neighbors = mx;
+    if (!c->defer_build) c->max_neighbors = mx;
     if (mx <= bp.cap) {
       c->bp = bp;
       c->nbr_cap = bp.cap;
@@ -497,6 +494,22 @@ int op_nbh_brick(xnb_ctx* c, double nbh_dist, const xnb_chunk_neighbors_config& 
     cap = grow_cap(mx);
   }
   return NOT_APPLICABLE;
+}
+
+int finish_build(xnb_ctx* c, bool* fits) {
+  *fits = true;
+  if (!c->build_pending) return XNB_OK;
+  c->build_pending = false;
+  HIPCHK(c, hipStreamSynchronize(c->st));
+  const uint32_t mx = c->h_u32[kPendingWords], bad = c->h_u32[kPendingWords + 4];
+  if (bad) return fail(c, XNB_E_STATE, "brick sizes changed between statistics and build");
+  c->max_neighbors = mx;
+  if (mx > c->bp.cap) {
+    c->nbr_cap = grow_cap(mx);
+    c->lists_valid = false;
+    *fits = false;
+  }
+  return XNB_OK;
 }
 
 int op_nbh(xnb_ctx* c, double nbh_dist, const xnb_chunk_neighbors_config& cfg, int all_cells, const PairCut* pc) {

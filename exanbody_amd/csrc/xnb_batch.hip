@@ -43,6 +43,7 @@ struct BatchBox {
   int every = 10;         // rebuild every this many steps; 0: when an atom passed max_displ
   bool fresh = true;      // the next step's first half still has to be launched
   uint32_t last_par = 0;  // parity of the box's last step
+  bool quads = false;     // laid out for four lanes an atom (attach)
   uint32_t ghost_span = 0;  // ghost slots covered by its ghost-refresh blocks (>= G)
   int64_t n_rebuilds = 0, n_violations = 0, n_recover = 0;
   std::vector<char> rebuilt;
@@ -56,13 +57,24 @@ struct BatchBox {
 // 3.92e9, 1.15 4.27e9, 1.18 4.21e9, 1.21 3.94e9, 1.35 3.88e9, 1.5 3.45e9; 1.0 recovers
 // thousands of times.
 constexpr double kBrickMargin = 1.15;
+// Boxes attached while the batch holds at most this many unfinished atoms, theirs included, get
+// small bricks built with four lanes an atom (a step's build covers the few boxes that rebuild and
+// takes as long as one lane needs); their force takes four lanes when the step's atoms are at
+// most kQuadAtoms.  24 boxes of 500 to 8,000 atoms (66,000 in all), FP64, 50 steps on the
+// displacement trigger: build 75 to 90 -> 41 us, force 40 -> 24 us, steps 13.3 -> 10.7 ms.  In a
+// large batch small bricks stage more than they gain (64 boxes of 500 to 50,000 atoms, the first
+// 131,072 atoms so: steps 18.5 -> 21.0 ms), so only boxes that are small themselves take them.
+constexpr uint64_t kBatchQuadAtoms = 98304, kBatchQuadBox = 8192;
+// A class of brick launches with fewer workgroups than this joins the next larger one: alone it
+// is another launch in the step's chain (64 boxes: 8 of 2,128 workgroups).
+constexpr uint32_t kClassBricks = 128;
 constexpr double kSlotMargin = 1.3;    // slot capacity head room for ghosts
 
 // One launch of brick work: its table range, workgroup lanes and dynamic LDS.
 struct BrickLaunch {
   int kind = kBatchNbh;  // which batched brick kernel
   size_t o = 0, n = 0;
-  uint32_t T = 64, lds = 0;
+  uint32_t T = 64, lds = 0;  // threads (atoms of a workgroup times lanes), LDS
   bool operator==(const BrickLaunch& b) const { return kind == b.kind && o == b.o && n == b.n && T == b.T && lds == b.lds; }
 };
 
@@ -114,7 +126,7 @@ struct xnb_batch {
   DArr<uint32_t> dclock;  // {par, gstep} of the step being run, then of the previous step
   DArr<uint32_t> amr_list, amr_count;  // rebuild_amr: cells of rebuilding boxes to sort, their number (+3 words)
   uint32_t lds_limit = 65536;
-  BatchKernelInfo kinfo[3] = {};  // per batched brick kernel (kBatchLjFp64, kBatchLjMixed, kBatchNbh)
+  BatchKernelInfo kinfo[kBatchKinds] = {};  // per batched brick kernel
   // steps replayed from captured HIP graphs (XNB_BATCH_GRAPH=0: every step launched eagerly)
   bool use_graph = true;
   // head room of attached boxes (XNB_BATCH_MARGINS="brick,slot" at create; 1,1 leaves none, so
@@ -282,37 +294,78 @@ uint32_t brick_class(uint32_t T, uint32_t lds, uint32_t cu_lds, uint32_t waves_p
   return std::max(1u, std::min({by_lds, by_waves, 4u}));
 }
 
-// Bricks of the listed boxes for the batched kernel `kind` (for the force: the boxes of that
-// precision), one launch per class of boxes whose workgroups fit the same number of times on
+// Bricks of the listed boxes that the batched kernel `kind` serves (kind_of), one launch per class of boxes whose workgroups fit the same number of times on
 // a CU, each sized for its own widest box, so that boxes with small bricks do not run in the
 // lanes and LDS of the largest one.  Results do not depend on the class: a brick's lanes
 // beyond its box's T take no atoms.
-void brick_launches(const xnb_batch* B, Tables& T, int kind, const std::vector<int>& boxes, const std::vector<uint32_t>& tag,
+// build: every listed box by its layout; force: four lanes an atom where the layout allows it and
+// the boxes together are few atoms
+std::vector<int> box_kinds(const xnb_batch* B, const std::vector<int>& boxes, bool build) {
+  uint64_t atoms = 0;
+  for (int i : boxes) atoms += B->box[i].f.N;
+  std::vector<int> k;
+  for (int i : boxes) {
+    const BoxFrame& f = B->box[i].f;
+    const bool quad = f.bp.lanes == kQuad;
+    if (build) k.push_back(quad ? kBatchNbhQuad : kBatchNbh);
+    else if (quad && atoms <= kQuadAtoms) k.push_back(f.mixed ? kBatchLjMixedQuad : kBatchLjFp64Quad);
+    else k.push_back(f.mixed ? kBatchLjMixed : kBatchLjFp64);
+  }
+  return k;
+}
+
+bool is_build(int kind) { return kind == kBatchNbh || kind == kBatchNbhQuad; }
+uint32_t kind_lanes(int kind) { return kind >= kBatchLjFp64Quad ? kQuad : 1u; }
+
+void brick_launches_of(const xnb_batch* B, Tables& T, int kind, const std::vector<int>& kinds, const std::vector<int>& boxes, const std::vector<uint32_t>& tag,
                     std::vector<BrickLaunch>& out) {
   const BatchKernelInfo& ki = B->kinfo[kind];
+  auto lds_of = [&](size_t q) { return brick_lds_bytes(B->box[boxes[q]].f.bp, is_build(kind)); };
+  auto threads_of = [&](size_t q) { return B->box[boxes[q]].f.bp.T * kind_lanes(kind); };
+  std::vector<uint32_t> cls(boxes.size(), 0);  // 0: not of this kind
+  uint32_t wgs[5] = {};
+  for (size_t q = 0; q < boxes.size(); q++) {
+    if (kinds[q] != kind) continue;
+    cls[q] = B->use_classes ? brick_class(threads_of(q), lds_of(q) + ki.static_lds, B->lds_limit, ki.waves_per_cu) : 1u;
+    wgs[cls[q]] += B->box[boxes[q]].f.bp.nbricks;
+  }
+  uint32_t into[5] = {0, 1, 2, 3, 4};
+  for (uint32_t k = 4; k > 1; k--) {
+    uint32_t to = k - 1;
+    while (to > 1 && !wgs[to]) to--;
+    if (wgs[k] >= kClassBricks || !wgs[to]) continue;
+    wgs[to] += wgs[k];
+    wgs[k] = 0;
+    for (uint32_t& x : into)
+      if (x == k) x = to;
+  }
   for (uint32_t k = 1; k <= 4; k++) {
     std::vector<int> sub;
     std::vector<uint32_t> nbr, tg;
     BrickLaunch L;
     L.kind = kind;
     for (size_t q = 0; q < boxes.size(); q++) {
-      const BatchBox& bb = B->box[boxes[q]];
-      if (kind != kBatchNbh && (kind == kBatchLjMixed) != (bb.f.mixed != 0)) continue;
-      const uint32_t lds = brick_lds_bytes(bb.f.bp, kind == kBatchNbh);
-      if (B->use_classes && brick_class(bb.f.bp.T, lds + ki.static_lds, B->lds_limit, ki.waves_per_cu) != k) continue;
+      if (!cls[q] || into[cls[q]] != k) continue;
       sub.push_back(boxes[q]);
-      nbr.push_back(bb.f.bp.nbricks);
+      nbr.push_back(B->box[boxes[q]].f.bp.nbricks);
       tg.push_back(tag[q]);
-      L.T = std::max(L.T, bb.f.bp.T);
-      L.lds = std::max(L.lds, lds);
+      L.T = std::max(L.T, threads_of(q));
+      L.lds = std::max(L.lds, lds_of(q));
     }
     if (!sub.empty()) {
       L.o = T.add(bricks_table(sub, nbr, tg));
       L.n = T.v.size() - L.o;
       out.push_back(L);
     }
-    if (!B->use_classes) break;
   }
+}
+
+// the build's or the force's launches of the listed boxes
+void brick_launches(const xnb_batch* B, Tables& T, bool build, const std::vector<int>& boxes, const std::vector<uint32_t>& tag,
+                    std::vector<BrickLaunch>& out) {
+  const std::vector<int> kinds = box_kinds(B, boxes, build);
+  for (int kind : {kBatchNbh, kBatchNbhQuad, kBatchLjMixed, kBatchLjMixedQuad, kBatchLjFp64, kBatchLjFp64Quad})
+    if (is_build(kind) == build) brick_launches_of(B, T, kind, kinds, boxes, tag, out);
 }
 
 // pinned staging (two buffers) and B->dwork hold at least n words
@@ -389,7 +442,7 @@ hipError_t launch_force_classes(xnb_batch* B, const uint32_t* W, const std::vect
                                 const uint32_t* clock) {
   return launch_split(B, lf.size(), 1, [&](size_t i, hipStream_t s) {
     const BrickLaunch& L = lf[i];
-    return launch_batch_lj(L.kind == kBatchLjMixed, B->dF.p, W + L.o, (uint32_t)L.n, L.T, L.lds, clock, s, set_lds);
+    return launch_batch_lj(L.kind, B->dF.p, W + L.o, (uint32_t)L.n, L.T, L.lds, clock, s, set_lds);
   });
 }
 
@@ -406,7 +459,7 @@ hipError_t launch_step(xnb_batch* B, const uint32_t* W, const StepLayout& L, boo
     launch_batch_ghosts(B->dF.p, W + L.o_rs, (uint32_t)L.n_rs, W + L.o_rc, (uint32_t)L.n_rc, W + L.o_rg, (uint32_t)L.n_rg,
                         W + L.o_list, L.nreb, B->amr_list.p, B->amr_count.p, L.par, B->st);
     const hipError_t he = launch_split(B, L.lb.size(), 0, [&](size_t i, hipStream_t s) {
-      return launch_batch_nbh(B->dF.p, W + L.lb[i].o, (uint32_t)L.lb[i].n, L.lb[i].T, L.lb[i].lds, L.par, s, set_lds);
+      return launch_batch_nbh(L.lb[i].kind, B->dF.p, W + L.lb[i].o, (uint32_t)L.lb[i].n, L.lb[i].T, L.lb[i].lds, L.par, s, set_lds);
     });
     if (he != hipSuccess) return he;
   }
@@ -442,7 +495,7 @@ int capture_step(xnb_batch* B, StepGraph& G, const Tables& T, const StepLayout& 
     G.buf[j].n = B->hwork_cap;
   }
   if ((e = stage_copy(B, T, G.buf[j].p))) return e;
-  for (int kind : {kBatchLjFp64, kBatchLjMixed, kBatchNbh}) {  // attributes set outside the capture
+  for (int kind = 0; kind < kBatchKinds; kind++) {  // attributes set outside the capture
     uint32_t lds = 0;
     for (const auto* v : {&L.lf, &L.lb})
       for (const BrickLaunch& x : *v)
@@ -476,19 +529,21 @@ bool active(const BatchBox& bb) { return bb.used && !bb.finished && !bb.failed; 
 // kernels' static LDS
 uint32_t lds_cap_for(const xnb_batch* B, double frac) {
   uint32_t st_lds = 0;
-  for (int k = 0; k < 3; k++) st_lds = std::max(st_lds, B->kinfo[k].static_lds);
+  for (int k = 0; k < kBatchKinds; k++) st_lds = std::max(st_lds, B->kinfo[k].static_lds);
   return (uint32_t)(frac * B->lds_limit) - std::min<uint32_t>(st_lds + 64u, B->lds_limit / 8);
 }
 
 // chunk_neighbors of a box for the batch: brick head room and the batch's LDS cap per brick
 // workgroup, or the context's own limit when no brick fits the cap (restored afterwards)
-int batch_box_nbh(xnb_batch* B, xnb_ctx* c) {
+int batch_box_nbh(xnb_batch* B, xnb_ctx* c, bool quads, bool defer = false) {
   c->brick_margin = B->brick_margin;
   const uint32_t keep = c->lds_limit;
   xnb_chunk_neighbors_config cfg{1, 0, 0, 0, 0};
   int e = XNB_OK;
   bool done = false;
   c->batch_shapes = true;
+  c->batch_quads = quads;
+  c->defer_build = defer;
   c->derive_ghosts = true;
   if (B->brick_lds_cap < keep) {
     c->lds_limit = B->brick_lds_cap;
@@ -498,6 +553,7 @@ int batch_box_nbh(xnb_batch* B, xnb_ctx* c) {
   }
   if (!done) e = op_nbh(c, c->nbh_dist_lab, cfg, 0);
   c->batch_shapes = false;
+  c->defer_build = false;
   return e;
 }
 
@@ -511,7 +567,7 @@ int recover_box(xnb_batch* B, int i, const xnb_run_params& p) {
   c->brick_margin = B->brick_margin;
   if ((e = ensure_capacity(c, (size_t)std::ceil((c->N + c->G) * B->slot_margin) + 256, c->N))) return e;
   if ((e = op_ghost_all(c, false, false))) return e;  // f and ep of the run's boxes are not carried
-  if ((e = batch_box_nbh(B, c))) return e;
+  if ((e = batch_box_nbh(B, c, bb.quads))) return e;
   if (c->list_kind != 1) return fail(c, XNB_E_STATE, "box no longer fits the brick path");
   if (c->bp.nbricks > kWorkBrickMask + 1) return fail(c, XNB_E_CAPACITY, "box has too many bricks for a batch");
   BHIP(B, hipStreamSynchronize(c->st));
@@ -520,6 +576,28 @@ int recover_box(xnb_batch* B, int i, const xnb_run_params& p) {
   if ((e2 = upload_frame(B, i))) return e2;
   // the overflow the batched rebuild left in the status words no longer holds
   BHIP(B, hipMemsetAsync(B->dwords.p + 4 * (size_t)i, 0, 4 * sizeof(uint32_t), B->st));
+  return XNB_OK;
+}
+
+// Attached boxes' deferred builds, before the batch reads their lists; lists that outgrew their
+// capacity are built again.
+int settle_builds(xnb_batch* B) {
+  for (int i = 0; i < (int)kMaxBatchBoxes; i++) {
+    BatchBox& bb = B->box[i];
+    if (!bb.used || !bb.c->build_pending) continue;
+    bool fits;
+    int e = finish_build(bb.c, &fits);
+    if (!e && fits) continue;
+    if (!e && !(e = batch_box_nbh(B, bb.c, bb.quads))) {
+      BHIP(B, hipStreamSynchronize(bb.c->st));
+      frame_from_ctx(B, i, bb.p);
+      if ((e = upload_frame(B, i))) return e;
+      if (bb.c->list_kind == 1 && bb.c->bp.nbricks <= kWorkBrickMask + 1) continue;
+      bb.c->err = "box no longer fits the brick path";
+    }
+    bb.failed = true;
+    bb.err = std::string("attach: ") + bb.c->err;
+  }
   return XNB_OK;
 }
 
@@ -539,7 +617,7 @@ int xnb_batch_create(xnb_batch** out, int device) {
   int lds = 0;
   if (hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device) == hipSuccess && lds > 0)
     B->lds_limit = (uint32_t)lds;
-  for (int k = 0; k < 3; k++) B->kinfo[k] = batch_kernel_info(k);
+  for (int k = 0; k < kBatchKinds; k++) B->kinfo[k] = batch_kernel_info(k);
   bool ok = hipStreamCreate(&B->st) == hipSuccess && hipStreamCreate(&B->st2) == hipSuccess;
   for (int k = 0; k < 2; k++)
     ok = ok && hipEventCreateWithFlags(&B->fork_ev[k], hipEventDisableTiming) == hipSuccess &&
@@ -646,16 +724,22 @@ int xnb_batch_attach(xnb_batch* B, xnb_ctx* c, const xnb_run_params* p, int* slo
   if (i < 0) return bfail(B, XNB_E_CAPACITY, "batch is full");
   // head room: ghost slots, and bricks / lists rebuilt with margins
   if ((e = ensure_capacity(c, (size_t)std::ceil((c->N + c->G) * B->slot_margin) + 256, (size_t)c->N + c->G))) return e;
-  if ((e = batch_box_nbh(B, c))) return e;
+  uint64_t atoms = c->N;
+  for (const BatchBox& x : B->box)
+    if (x.used && !x.finished) atoms += x.c->N;
+  const bool quads = atoms <= kBatchQuadAtoms && c->N <= kBatchQuadBox;
+  // the build is not waited for (one box's takes some 75 us on a mostly idle chip): the boxes'
+  // builds run beside each other on their own streams until settle_builds
+  if ((e = batch_box_nbh(B, c, quads, true))) return e;
   if (c->list_kind != 1) return bfail(B, XNB_E_STATE, "box geometry is not on the brick path (cell edge < nbh_dist)");
   if (brick_lds_bytes(c->bp, false) > B->lds_limit) return bfail(B, XNB_E_CAPACITY, "box bricks exceed LDS");
   // force-table entries hold the brick index in kWorkEpiShift bits
   if (c->bp.nbricks > kWorkBrickMask + 1) return bfail(B, XNB_E_CAPACITY, "box has too many bricks for a batch");
-  if (hipStreamSynchronize(c->st) != hipSuccess) return bfail(B, XNB_E_HIP, "box stream");
   BatchBox& bb = B->box[i];
   bb = BatchBox{};
   bb.c = c;
   bb.used = true;
+  bb.quads = quads;
   bb.steps = p->steps;
   bb.every = std::max(p->rebuild_every, 0);  // <= 0: displacement trigger, as in xnb_run
   bb.rebuilt.assign((size_t)p->steps, 0);
@@ -681,6 +765,7 @@ int xnb_batch_step(xnb_batch* B, int nsteps, int* n_active) {
   if (!B || nsteps < 0) return XNB_E_ARG;
   BHIP(B, hipSetDevice(B->device));
   int e;
+  if (nsteps && (e = settle_builds(B))) return e;
   for (int s = 0; s < nsteps; s++) {
     std::vector<int> act;
     for (int i = 0; i < (int)kMaxBatchBoxes; i++)
@@ -738,7 +823,7 @@ int xnb_batch_step(xnb_batch* B, int nsteps, int* n_active) {
       L.n_rc = T.v.size() - L.o_rc;
       L.o_rg = T.add(blocks_table(reb, nGh));
       L.n_rg = T.v.size() - L.o_rg;
-      brick_launches(B, T, kBatchNbh, reb, std::vector<uint32_t>(reb.size(), 0u), L.lb);
+      brick_launches(B, T, true, reb, std::vector<uint32_t>(reb.size(), 0u), L.lb);
       L.o_list = T.add(std::vector<uint32_t>(reb.begin(), reb.end()));
       L.o_zero = T.add(std::vector<uint32_t>{0u});
       // the move swaps each rebuilding box's buffer roles on the device; the host mirror follows
@@ -789,7 +874,7 @@ int xnb_batch_step(xnb_batch* B, int nsteps, int* n_active) {
       frc.push_back(i);
       tag.push_back(fuse ? (uint32_t)EPI_NEXT : (uint32_t)EPI_KICK);
     }
-    for (int kind : {kBatchLjMixed, kBatchLjFp64}) brick_launches(B, T, kind, frc, tag, L.lf);
+    brick_launches(B, T, false, frc, tag, L.lf);
     // 3. Launch it, from a captured graph when a step of the same kind (quiet, or rebuilding
     // at fixed intervals) had the same table and layout before.
     const bool plain = fresh.empty() && disp.empty() && !T.v.empty();
@@ -860,7 +945,7 @@ int xnb_batch_step(xnb_batch* B, int nsteps, int* n_active) {
       if (!late.empty()) {
         Tables TL;
         std::vector<BrickLaunch> ll;
-        for (int kind : {kBatchLjMixed, kBatchLjFp64}) brick_launches(B, TL, kind, late, late_tag, ll);
+        brick_launches(B, TL, false, late, late_tag, ll);
         if ((e = upload_tables(B, TL))) return e;
         const hipError_t he = launch_force_classes(B, B->dwork.p, ll, true, B->dclock.p + 2);
         if (he != hipSuccess) return bfail(B, XNB_E_HIP, std::string("batched force after recovery: ") + hipGetErrorString(he));
@@ -926,6 +1011,8 @@ int xnb_batch_autotune(xnb_batch* B, double* lds_frac_out) {
   if (!B) return XNB_E_ARG;
   BHIP(B, hipSetDevice(B->device));
   std::vector<int> boxes;
+  int e;
+  if ((e = settle_builds(B))) return e;
   for (int i = 0; i < (int)kMaxBatchBoxes; i++) {
     const BatchBox& bb = B->box[i];
     if (!bb.used) continue;
@@ -936,7 +1023,6 @@ int xnb_batch_autotune(xnb_batch* B, double* lds_frac_out) {
   BHIP(B, hipStreamSynchronize(B->st));
   for (StepGraph* G : {&B->gq, &B->gr[0], &B->gr[1]}) retire_graph(B, *G);
   destroy_retired(B);
-  int e;
   // every box laid out again under the cap of `frac`
   auto layout = [&](double frac) -> int {
     B->lds_frac = frac;
@@ -946,7 +1032,7 @@ int xnb_batch_autotune(xnb_batch* B, double* lds_frac_out) {
       xnb_ctx* c = bb.c;
       ctx_from_frame(B, i, B->par);
       int e2;
-      if ((e2 = batch_box_nbh(B, c))) return bfail(B, e2, std::string("autotune layout: ") + c->err);
+      if ((e2 = batch_box_nbh(B, c, bb.quads))) return bfail(B, e2, std::string("autotune layout: ") + c->err);
       if (c->list_kind != 1 || brick_lds_bytes(c->bp, false) > B->lds_limit || c->bp.nbricks > kWorkBrickMask + 1)
         return bfail(B, XNB_E_CAPACITY, "autotune layout: a box left the batch's brick path");
       BHIP(B, hipStreamSynchronize(c->st));
@@ -968,9 +1054,8 @@ int xnb_batch_autotune(xnb_batch* B, double* lds_frac_out) {
   auto score = [&](double& ms) -> int {
     Tables T;
     std::vector<BrickLaunch> lb, lf;
-    brick_launches(B, T, kBatchNbh, boxes, std::vector<uint32_t>(boxes.size(), 0u), lb);
-    for (int kind : {kBatchLjMixed, kBatchLjFp64})
-      brick_launches(B, T, kind, boxes, std::vector<uint32_t>(boxes.size(), (uint32_t)EPI_NONE), lf);
+    brick_launches(B, T, true, boxes, std::vector<uint32_t>(boxes.size(), 0u), lb);
+    brick_launches(B, T, false, boxes, std::vector<uint32_t>(boxes.size(), (uint32_t)EPI_NONE), lf);
     const size_t o_list = T.add(std::vector<uint32_t>(boxes.begin(), boxes.end()));
     int e2;
     if ((e2 = upload_tables(B, T))) return e2;
@@ -979,7 +1064,7 @@ int xnb_batch_autotune(xnb_batch* B, double* lds_frac_out) {
     auto build = [&]() {
       launch_batch_zero_words(B->dwords.p, W + o_list, (uint32_t)boxes.size(), B->st);
       return launch_split(B, lb.size(), 0, [&](size_t i, hipStream_t st) {
-        return launch_batch_nbh(B->dF.p, W + lb[i].o, (uint32_t)lb[i].n, lb[i].T, lb[i].lds, par, st, true);
+        return launch_batch_nbh(lb[i].kind, B->dF.p, W + lb[i].o, (uint32_t)lb[i].n, lb[i].T, lb[i].lds, par, st, true);
       });
     };
     constexpr int kReps = 3;
@@ -1029,6 +1114,10 @@ int xnb_batch_detach(xnb_batch* B, int slot, xnb_run_params* p) {
   BHIP(B, hipSetDevice(B->device));
   BHIP(B, hipStreamSynchronize(B->st));
   BatchBox& bb = B->box[slot];
+  if (bb.c->build_pending) {  // detached before any step
+    bool fits;
+    (void)finish_build(bb.c, &fits);
+  }
   ctx_from_frame(B, slot, bb.finished ? bb.last_par : B->par);
   // a box detached before its last step keeps the fused first half of its next step; the
   // one-box loop restarts from a completed step, so only finished boxes are returned as

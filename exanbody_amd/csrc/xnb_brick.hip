@@ -823,14 +823,14 @@ __device__ __forceinline__ void nbh_brick_body(const Geom& g, const BrickParams&
       // every list of the workgroup ends with the sentinel up to a multiple of kQuadBatch of the
       // longest, so the force reads whole batches, with one or four lanes an atom
       if (!A.live) cnt = 0;
-      if (threadIdx.x % LANES == 0) bcnt[(size_t)b * T + t] = cnt;
+      if (threadIdx.x % LANES == 0 && t < T) bcnt[(size_t)b * T + t] = cnt;
       const uint32_t wm = wave_max_b(cnt);
       if ((threadIdx.x & 63u) == 0) L.wsum[threadIdx.x >> 6] = wm;
       __syncthreads();
       uint32_t longest = 0;
       for (uint32_t w = 0; w < (blockDim.x >> 6); w++) longest = max(longest, L.wsum[w]);
       if (threadIdx.x == 0 && longest > 0) atomicMax(max_cnt, longest);
-      const uint32_t end = min((longest + kQuadBatch - 1) / kQuadBatch * kQuadBatch, bp.cap);
+      const uint32_t end = t < T ? min((longest + kQuadBatch - 1) / kQuadBatch * kQuadBatch, bp.cap) : 0u;
       const uint16_t pad = (uint16_t)R;
       for (uint32_t q = min(cnt, bp.cap) + threadIdx.x % LANES; q < end; q += LANES) out[lpos(q, t, T)] = pad;
       return;
@@ -1215,7 +1215,9 @@ __device__ __forceinline__ void lj_quad_brick_body(const Geom& g, const BrickPar
     L.wcnt[1] = 0;
   }
   const uint32_t t = threadIdx.x / kQuad, c = threadIdx.x % kQuad, T = bp.T;
-  const uint32_t n_list = bcnt[(size_t)b * T + t];
+  // a batched launch may be wider than the box's bricks: lanes past T hold no atom and no list
+  const bool held = t < T;
+  const uint32_t n_list = held ? bcnt[(size_t)b * T + t] : 0u;
   const uint32_t lw = lane_word(bp, b, t);
   // batch k of the list is the groups 4 k .. 4 k + 3, the lane's own is 4 k + c; every slab
   // holds whole batches (cap is a multiple of kQuadBatch)
@@ -1223,7 +1225,7 @@ __device__ __forceinline__ void lj_quad_brick_body(const Geom& g, const BrickPar
   uint2 ahead[kAhead];
 #pragma unroll
   for (uint32_t k = 0; k < kAhead; k++)
-    ahead[k] = k * kQuadBatch < bp.cap ? load_list_group(lst + (size_t)(4 * k) * T) : make_uint2(0u, 0u);
+    ahead[k] = held && k * kQuadBatch < bp.cap ? load_list_group(lst + (size_t)(4 * k) * T) : make_uint2(0u, 0u);
   stage_region<false>(g, bp, b, r, L);
   __syncthreads();
   const ForceAtom At = force_atom(bp, b, lw);
@@ -1265,7 +1267,7 @@ __device__ __forceinline__ void lj_quad_brick_body(const Geom& g, const BrickPar
         if (q0 + k * kQuadBatch >= nmax) break;
         const uint2 w = ahead[k];
         const uint32_t nq = q0 + (k + kAhead) * kQuadBatch;
-        if (nq < nmax) ahead[k] = load_list_group(lst + (size_t)(nq >> 2) * T);
+        if (held && nq < nmax) ahead[k] = load_list_group(lst + (size_t)(nq >> 2) * T);
         group(make_uint2(quad_get<0>(w.x), quad_get<0>(w.y)), term);
         group(make_uint2(quad_get<1>(w.x), quad_get<1>(w.y)), term);
         group(make_uint2(quad_get<2>(w.x), quad_get<2>(w.y)), term);
@@ -1282,7 +1284,7 @@ __device__ __forceinline__ void lj_quad_brick_body(const Geom& g, const BrickPar
       sum = 0.0;
 #pragma unroll
       for (uint32_t k = 0; k < kAhead; k++)
-        ahead[k] = k * kQuadBatch < bp.cap ? load_list_group(lst + (size_t)(4 * k) * T) : make_uint2(0u, 0u);
+        ahead[k] = held && k * kQuadBatch < bp.cap ? load_list_group(lst + (size_t)(4 * k) * T) : make_uint2(0u, 0u);
       walk([&](double dx, double dy, double dz, double& e) { return lj_term_fp64_any<ENERGY>(lj, dx, dy, dz, e); });
     }
   }
@@ -1836,6 +1838,7 @@ __device__ inline bool batch_brick(const uint32_t* __restrict__ work, uint32_t& 
   return true;
 }
 
+template <uint32_t LANES>
 __global__ void __launch_bounds__(1024) kb_nbh_brick(const BoxFrame* __restrict__ F, const uint32_t* __restrict__ work, uint32_t par) {
   uint32_t box, b;
   if (!batch_brick(work, box, b)) return;  // whole workgroup
@@ -1844,17 +1847,18 @@ __global__ void __launch_bounds__(1024) kb_nbh_brick(const BoxFrame* __restrict_
   // reach past the slot arrays, so the box is left to the one-box recovery
   if (f.words[0] & 4u) return;
   const double4* r = f.rbuf[(f.rcur ^ par) & 1u];
-  nbh_brick_body<false, false, true>(f.g, f.bpn, b, r, f.cell_off, f.cell_n, f.max2, 0, 0, f.blist, f.bcnt, f.words + 1);
+  nbh_brick_body<false, false, true, LANES>(f.g, f.bpn, b, r, f.cell_off, f.cell_n, f.max2, 0, 0, f.blist, f.bcnt, f.words + 1);
 }
 
-template <bool MIXED, int EPI>
+template <bool MIXED, bool QUAD, int EPI>
 __device__ __forceinline__ void lj_batch_case(const BoxFrame& f, uint32_t b, uint32_t par, uint32_t gstep) {
   PState A = f.ab ? f.B : f.A;
   const uint32_t cur = (f.rcur ^ par) & 1u;
   A.r = f.rbuf[cur];
   // the next step's count: local step k = gstep - gstep0 + 1, count of step k + 1 at [k]
   const NextStep nx{f.rbuf[cur ^ 1u], f.backup, f.dt, f.dt2, f.thr2, f.counts + (gstep - f.gstep0 + 1), nullptr, nullptr};
-  compute_pair_brick_body<LennardJonesForceFunctor<MIXED>, false, EPI, LJB_UNROLL_B>(
+  if constexpr (QUAD) lj_quad_brick_body<MIXED, false, EPI>(f.g, f.bp, b, A.r, f.blist, f.bcnt, f.lj, A, f.dth, nx);
+  else compute_pair_brick_body<LennardJonesForceFunctor<MIXED>, false, EPI, LJB_UNROLL_B>(
       f.g, f.bp, b, A.r, f.blist, f.bcnt, LennardJonesForceFunctor<MIXED>{f.lj}, f.lj.rc2, A, f.dth, nx);
 }
 
@@ -1862,7 +1866,7 @@ __device__ __forceinline__ void lj_batch_case(const BoxFrame& f, uint32_t b, uin
 // so the mixed form runs with its own, smaller register budget); the epilogue is per box
 // (uniform per workgroup).  EPI_KICK closes a box's run; EPI_NEXT fuses its next step;
 // EPI_NONE stores the force and energy only.
-template <bool MIXED>
+template <bool MIXED, bool QUAD>
 __global__ void __launch_bounds__(1024) kb_lj_brick(const BoxFrame* __restrict__ F, const uint32_t* __restrict__ work,
                                                     const uint32_t* __restrict__ clock) {
   uint32_t box, b;
@@ -1876,27 +1880,35 @@ __global__ void __launch_bounds__(1024) kb_lj_brick(const BoxFrame* __restrict__
   // reads the words after the step and redoes it with the one-box operators (or fails it).
   // The words are cleared at attach, before each batched rebuild and after a recovery.
   if (f.words[0] != 0u || f.words[1] > f.bp.cap || f.words[2] != 0u) return;
-  if (epi == EPI_NEXT) lj_batch_case<MIXED, EPI_NEXT>(f, b, par, gstep);
-  else if (epi == EPI_KICK) lj_batch_case<MIXED, EPI_KICK>(f, b, par, gstep);
-  else lj_batch_case<MIXED, EPI_NONE>(f, b, par, gstep);  // force and energy only (the batch autotuner's timings)
+  if (epi == EPI_NEXT) lj_batch_case<MIXED, QUAD, EPI_NEXT>(f, b, par, gstep);
+  else if (epi == EPI_KICK) lj_batch_case<MIXED, QUAD, EPI_KICK>(f, b, par, gstep);
+  else lj_batch_case<MIXED, QUAD, EPI_NONE>(f, b, par, gstep);  // force and energy only (the batch autotuner's timings)
 }
 
-static const void* batch_kernel(int kind) {
+using BatchForce = void (*)(const BoxFrame*, const uint32_t*, const uint32_t*);
+static BatchForce batch_force(int kind) {
   switch (kind) {
-    case kBatchLjFp64: return (const void*)kb_lj_brick<false>;
-    case kBatchLjMixed: return (const void*)kb_lj_brick<true>;
-    default: return (const void*)kb_nbh_brick;
+    case kBatchLjFp64: return kb_lj_brick<false, false>;
+    case kBatchLjMixed: return kb_lj_brick<true, false>;
+    case kBatchLjFp64Quad: return kb_lj_brick<false, true>;
+    default: return kb_lj_brick<true, true>;
   }
 }
+static const void* batch_kernel(int kind) {
+  if (kind == kBatchNbh) return (const void*)kb_nbh_brick<1>;
+  if (kind == kBatchNbhQuad) return (const void*)kb_nbh_brick<kQuad>;
+  return (const void*)batch_force(kind);
+}
 
-hipError_t launch_batch_nbh(const BoxFrame* F, const uint32_t* work, uint32_t nwork, uint32_t T, uint32_t lds, uint32_t par,
-                            hipStream_t st, bool set) {
+hipError_t launch_batch_nbh(int kind, const BoxFrame* F, const uint32_t* work, uint32_t nwork, uint32_t threads, uint32_t lds,
+                            uint32_t par, hipStream_t st, bool set) {
   if (!nwork) return hipSuccess;
   if (set) {
-    hipError_t e = set_lds((const void*)kb_nbh_brick, lds);
+    hipError_t e = batch_set_lds(kind, lds);
     if (e != hipSuccess) return e;
   }
-  kb_nbh_brick<<<nwork, T, lds, st>>>(F, work, par);
+  if (kind == kBatchNbhQuad) kb_nbh_brick<kQuad><<<nwork, threads, lds, st>>>(F, work, par);
+  else kb_nbh_brick<1><<<nwork, threads, lds, st>>>(F, work, par);
   return hipGetLastError();
 }
 
@@ -1917,15 +1929,14 @@ BatchKernelInfo batch_kernel_info(int kind) {
   return info;
 }
 
-hipError_t launch_batch_lj(bool mixed, const BoxFrame* F, const uint32_t* work, uint32_t nwork, uint32_t T, uint32_t lds,
+hipError_t launch_batch_lj(int kind, const BoxFrame* F, const uint32_t* work, uint32_t nwork, uint32_t threads, uint32_t lds,
                            const uint32_t* clock, hipStream_t st, bool set) {
   if (!nwork) return hipSuccess;
   if (set) {
-    hipError_t e = batch_set_lds(mixed ? kBatchLjMixed : kBatchLjFp64, lds);
+    hipError_t e = batch_set_lds(kind, lds);
     if (e != hipSuccess) return e;
   }
-  if (mixed) kb_lj_brick<true><<<nwork, T, lds, st>>>(F, work, clock);
-  else kb_lj_brick<false><<<nwork, T, lds, st>>>(F, work, clock);
+  batch_force(kind)<<<nwork, threads, lds, st>>>(F, work, clock);
   return hipGetLastError();
 }
 

@@ -105,6 +105,10 @@ struct xnb_ctx {
   bool nbh_prefilter = true;        // unfiltered brick builds test in FP32 with an FP64 band (same lists)
   uint32_t lds_limit = 65536;
   bool batch_shapes = false;  // brick shapes offered to batched boxes only
+  // a build launched without waiting for its words (attach): taken as fitting until finish_build
+  // has looked at them (h_u32 + kPendingWords)
+  bool defer_build = false, build_pending = false;
+  bool batch_quads = false;   // with batch_shapes: the shapes of four lanes an atom first
   double brick_margin = 1.0;        // brick T / Rmax head room (batched boxes rebuild without re-choosing)
 
   double last_rcut = 0.;
@@ -165,6 +169,10 @@ int op_nbh(xnb_ctx* c, double nbh_dist, const xnb_chunk_neighbors_config& cfg, i
 // forces false: f and ep neither carried by the move nor copied to ghosts; pc: per type-pair list radii
 int full_update(xnb_ctx* c, bool forces = true, const PairCut* pc = nullptr);
 int ensure_full_lists(xnb_ctx* c);
+constexpr int kPendingWords = 48;
+// the end of a deferred build: waits for it, *fits false when its lists outgrew their capacity
+// (which has grown for the next build)
+int finish_build(xnb_ctx* c, bool* fits);
 int ensure_regions(xnb_ctx* c, bool derive);
 void tstart(xnb_ctx* c, int id);
 void tstop(xnb_ctx* c);

@@ -19,6 +19,12 @@ constexpr uint32_t kXcds = 8;
 constexpr uint32_t kListBatch = 8;
 // Lists of quad bricks (four lanes an atom) are padded per workgroup to a multiple of this many.
 constexpr uint32_t kQuad = 4, kQuadBatch = 16;
+// Boxes of at most this many atoms give every atom four lanes (four atoms' lanes fill two waves
+// per SIMD of the chip; larger boxes have enough waves with one lane an atom, which takes 1.7
+// times fewer instructions).  Force and build launch with one and with four lanes: 6,912 atoms
+// FP64 20.5 and 13.6, 68 and 28 us; 27,431 atoms mixed 15.8 and 15.5, 68 and 38 us; 131,072
+// atoms FP64 36 and 50, 89 and 104 us.
+constexpr uint32_t kQuadAtoms = 32768;
 
 struct BrickParams {
   int Bi, Bj, Bk;     // brick size in cells
@@ -148,17 +154,18 @@ void launch_batch_ghost_update_r(const BoxFrame* F, const uint32_t* work, uint32
 void launch_batch_advance(uint32_t* clock, hipStream_t st);
 void launch_batch_first_half(const BoxFrame* F, const uint32_t* work, uint32_t nwork, uint32_t par, uint32_t gstep, hipStream_t st);
 void launch_batch_trigger(const BoxFrame* F, const uint32_t* boxes, uint32_t n, uint32_t gstep, uint32_t* out, hipStream_t st);
-hipError_t launch_batch_nbh(const BoxFrame* F, const uint32_t* work, uint32_t nwork, uint32_t T, uint32_t lds, uint32_t par,
-                            hipStream_t st, bool set_lds = true);
-// batched brick kernels: the force per precision and the neighbour build
-enum { kBatchLjFp64 = 0, kBatchLjMixed = 1, kBatchNbh = 2 };
+// batched brick kernels: the force per precision and the neighbour build, with one and with four
+// lanes an atom (threads: atoms a workgroup holds times lanes)
+enum { kBatchLjFp64 = 0, kBatchLjMixed = 1, kBatchNbh = 2, kBatchLjFp64Quad = 3, kBatchLjMixedQuad = 4, kBatchNbhQuad = 5, kBatchKinds = 6 };
+hipError_t launch_batch_nbh(int kind, const BoxFrame* F, const uint32_t* work, uint32_t nwork, uint32_t threads, uint32_t lds,
+                            uint32_t par, hipStream_t st, bool set_lds = true);
 struct BatchKernelInfo {
   uint32_t static_lds;    // bytes of static LDS
   uint32_t waves_per_cu;  // waves one CU holds at the kernel's register use
 };
 BatchKernelInfo batch_kernel_info(int kind);
 // set_lds false: the workgroup LDS attribute was already raised to lds (launches under capture)
-hipError_t launch_batch_lj(bool mixed, const BoxFrame* F, const uint32_t* work, uint32_t nwork, uint32_t T, uint32_t lds,
+hipError_t launch_batch_lj(int kind, const BoxFrame* F, const uint32_t* work, uint32_t nwork, uint32_t threads, uint32_t lds,
                            const uint32_t* clock, hipStream_t st, bool set_lds = true);
 hipError_t batch_set_lds(int kind, uint32_t lds);
 constexpr uint32_t kBatchSlotBlock = 256;  // threads per workgroup of the per-slot / per-cell batched kernels
