@@ -1404,112 +1404,131 @@ __device__ __forceinline__ void ljmm_brick_body(const Geom& g, const BrickParams
   }
   const uint2* lst = reinterpret_cast<const uint2*>(blist + (size_t)b * bp.cap * T) + t;
   constexpr int W = U / 4;
-  uint2 wn[W];
-  if (nmax > 0) {
+  // FP64 roots and their range as in lj_batch_fp64: looked at once after the list, which is
+  // walked again with the generic operations if it was left
+  PairRange rng;
+  auto walk = [&](auto generic) {
+    constexpr bool GENERIC = decltype(generic)::value;
+    uint2 wn[W];
+    if (nmax > 0) {
 #pragma unroll
-    for (int w = 0; w < W; w++) wn[w] = load_list_group(lst + (size_t)w * T);
-  }
-  for (uint32_t q0 = 0; q0 < nmax; q0 += U) {
-    uint2 wc[W];
-#pragma unroll
-    for (int w = 0; w < W; w++) wc[w] = wn[w];
-    if (q0 + U < nmax) {
-      const uint2* nxt = lst + (size_t)((q0 + U) >> 2) * T;
-#pragma unroll
-      for (int w = 0; w < W; w++) wn[w] = load_list_group(nxt + (size_t)w * T);
+      for (int w = 0; w < W; w++) wn[w] = load_list_group(lst + (size_t)w * T);
     }
-    uint32_t j[U];
+    for (uint32_t q0 = 0; q0 < nmax; q0 += U) {
+      uint2 wc[W];
 #pragma unroll
-    for (int w = 0; w < W; w++) {
-      j[4 * w + 0] = wc[w].x & 0xffffu;
-      j[4 * w + 1] = wc[w].x >> 16;
-      j[4 * w + 2] = wc[w].y & 0xffffu;
-      j[4 * w + 3] = wc[w].y >> 16;
-    }
-    // pairs in sub-batches of H: one range decision per sub-batch for the FP64 roots.  FP64
-    // takes pairs by two: its per-type tables and sums leave too few registers for more in
-    // flight (timed on the two-species slab: force 3.39 ms at H = 2, 3.44 at 4, 3.54 at 8)
+      for (int w = 0; w < W; w++) wc[w] = wn[w];
+      if (q0 + U < nmax) {
+        const uint2* nxt = lst + (size_t)((q0 + U) >> 2) * T;
 #pragma unroll
-    for (int h = 0; h < U; h += H) {
-      // per pair: displacement, neighbour type, inside its pair's cutoff
-      double dx[H], dy[H], dz[H], d2[H];
-      unsigned tb[H];
-      bool in[H];
-      bool small = false;
-#pragma unroll
-      for (int u = 0; u < H; u++) {
-        dx[u] = L.px[3 * j[h + u]] - ax0;
-        dy[u] = L.py[3 * j[h + u]] - ay0;
-        dz[u] = L.pz[3 * j[h + u]] - az0;
-        tb[u] = min((unsigned)L.pt[j[h + u]], (unsigned)(NT - 1));
-        double prc2 = rc2[0];
-#pragma unroll
-        for (int q = 1; q < NT; q++) prc2 = tb[u] == (unsigned)q ? rc2[q] : prc2;
-        d2[u] = MIXED ? fma(dz[u], dz[u], fma(dy[u], dy[u], dx[u] * dx[u])) : (dx[u] * dx[u] + dy[u] * dy[u]) + dz[u] * dz[u];
-        in[u] = d2[u] <= prc2;
-        small = small || (in[u] && d2[u] < 0x1p-767);
+        for (int w = 0; w < W; w++) wn[w] = load_list_group(nxt + (size_t)w * T);
       }
-      double inv_r[H];  // plain form: 1.0 / sqrt(d2), each correctly rounded (1.0 outside the cutoff)
-      if (!MIXED) {
-        if (__builtin_expect(__any(small), 0)) {
+      uint32_t j[U];
 #pragma unroll
-          for (int u = 0; u < H; u++) inv_r[u] = 1.0 / sqrt(in[u] ? d2[u] : 1.0);
-        } else {
-#pragma unroll
-          for (int u = 0; u < H; u++) inv_r[u] = recip_normal(sqrt_normal(in[u] ? d2[u] : 1.0));
-        }
+      for (int w = 0; w < W; w++) {
+        j[4 * w + 0] = wc[w].x & 0xffffu;
+        j[4 * w + 1] = wc[w].x >> 16;
+        j[4 * w + 2] = wc[w].y & 0xffffu;
+        j[4 * w + 3] = wc[w].y >> 16;
       }
+      // FP64 takes pairs by two, one sub-batch behind the other: 82 registers and two workgroups a
+      // CU, where a root and a reciprocal of their own, a range test a sub-batch and 124 registers
+      // were 14 % slower (force launch, two species: 52,428 atoms 43.2 -> 35.8 us, 393,216 atoms
+      // 219 -> 187 us); by four (100 registers) 36.4 and 189 us.
 #pragma unroll
-      for (int u = 0; u < H; u++) {
-        double psg = sg[0], pe4 = e4[0], pm24 = m24[0];
-        float ps6f = s6f[0], pe4f = e4f[0], pm24f = m24f[0];
+      for (int h = 0; h < U; h += H) {
+        // per pair: displacement, neighbour type, inside its pair's cutoff
+        double dx[H], dy[H], dz[H], d2[H];
+        unsigned tb[H];
+        bool in[H];
 #pragma unroll
-        for (int q = 1; q < NT; q++)
-          if (tb[u] == (unsigned)q) {
-            psg = sg[q];
-            pe4 = e4[q];
-            pm24 = m24[q];
-            ps6f = s6f[q];
-            pe4f = e4f[q];
-            pm24f = m24f[q];
-          }
-        double coef, ce;  // force coefficient (f += coef * d) and pair energy
-        if (MIXED) {
-          const float inv_r2 = in[u] ? __builtin_amdgcn_rcpf((float)d2[u]) : 0.0f;  // 0 outside: coefficient and energy 0
-          float s6;
-          coef = (double)lj_coef_f32(inv_r2, ps6f, pm24f, s6);
-          ce = ENERGY ? (double)lj_energy_f32(s6, pe4f) : 0.0;
-        } else {
-          const double ratio = psg * inv_r[u];
-          const double ratio2 = ratio * ratio;
-          const double ratio6 = ratio2 * ratio2 * ratio2;
-          const double ratio12 = ratio6 * ratio6;
-          double de = (pm24 * (2. * ratio12 - ratio6)) * inv_r[u];
-          de *= inv_r[u];
-          coef = in[u] ? de : 0.0;
-          ce = (ENERGY && in[u]) ? pe4 * (ratio12 - ratio6) : 0.0;
+        for (int u = 0; u < H; u++) {
+          dx[u] = L.px[3 * j[h + u]] - ax0;
+          dy[u] = L.py[3 * j[h + u]] - ay0;
+          dz[u] = L.pz[3 * j[h + u]] - az0;
+          tb[u] = min((unsigned)L.pt[j[h + u]], (unsigned)(NT - 1));
+          double prc2 = rc2[0];
+#pragma unroll
+          for (int q = 1; q < NT; q++) prc2 = tb[u] == (unsigned)q ? rc2[q] : prc2;
+          d2[u] = MIXED ? fma(dz[u], dz[u], fma(dy[u], dy[u], dx[u] * dx[u])) : (dx[u] * dx[u] + dy[u] * dy[u]) + dz[u] * dz[u];
+          in[u] = d2[u] <= prc2;
         }
-        if (MIXED) {
-          // one sum in stream order, f = fma(c, d, f) as in the singlemat mixed form (c and the
-          // energy are +-0 outside the cutoff): the tolerance form needs no per-type grouping
-          gx[0] = fma(coef, dx[u], gx[0]);
-          gy[0] = fma(coef, dy[u], gy[0]);
-          gz[0] = fma(coef, dz[u], gz[0]);
-          if (ENERGY) ge[0] += ce;
-        } else {
+        double inv_r[H];  // plain form: 1.0 / sqrt(d2), each correctly rounded (1.0 outside the cutoff)
+        if (!MIXED) {
 #pragma unroll
-          for (int q = 0; q < NT; q++) {  // f += (de / r) * d per neighbour-type group, the plain form
-            const bool mine = in[u] && tb[u] == (unsigned)q;
-            const double cq = mine ? coef : 0.0;
-            gx[q] += cq * dx[u];
-            gy[q] += cq * dy[u];
-            gz[q] += cq * dz[u];
-            if (ENERGY) ge[q] += mine ? ce : 0.0;
-            any[q] = any[q] || mine;
+          for (int u = 0; u < H; u++) {
+            const double x = in[u] ? d2[u] : 1.0;
+            if (GENERIC) {
+              inv_r[u] = 1.0 / sqrt(x);
+            } else {
+              rng.add(x);
+              inv_r[u] = inv_sqrt_normal(x);
+            }
           }
         }
+#pragma unroll
+        for (int u = 0; u < H; u++) {
+          double psg = sg[0], pe4 = e4[0], pm24 = m24[0];
+          float ps6f = s6f[0], pe4f = e4f[0], pm24f = m24f[0];
+#pragma unroll
+          for (int q = 1; q < NT; q++)
+            if (tb[u] == (unsigned)q) {
+              psg = sg[q];
+              pe4 = e4[q];
+              pm24 = m24[q];
+              ps6f = s6f[q];
+              pe4f = e4f[q];
+              pm24f = m24f[q];
+            }
+          double coef, ce;  // force coefficient (f += coef * d) and pair energy
+          if (MIXED) {
+            const float inv_r2 = in[u] ? __builtin_amdgcn_rcpf((float)d2[u]) : 0.0f;  // 0 outside: coefficient and energy 0
+            float s6;
+            coef = (double)lj_coef_f32(inv_r2, ps6f, pm24f, s6);
+            ce = ENERGY ? (double)lj_energy_f32(s6, pe4f) : 0.0;
+          } else {
+            const double ratio = psg * inv_r[u];
+            const double ratio2 = ratio * ratio;
+            const double ratio6 = ratio2 * ratio2 * ratio2;
+            const double ratio12 = ratio6 * ratio6;
+            double de = (pm24 * fma(2., ratio12, -ratio6)) * inv_r[u];  // doubling is exact: one rounding
+            de *= inv_r[u];
+            coef = in[u] ? de : 0.0;
+            ce = (ENERGY && in[u]) ? pe4 * (ratio12 - ratio6) : 0.0;
+          }
+          if (MIXED) {
+            // one sum in stream order, f = fma(c, d, f) as in the singlemat mixed form (c and the
+            // energy are +-0 outside the cutoff): the tolerance form needs no per-type grouping
+            gx[0] = fma(coef, dx[u], gx[0]);
+            gy[0] = fma(coef, dy[u], gy[0]);
+            gz[0] = fma(coef, dz[u], gz[0]);
+            if (ENERGY) ge[0] += ce;
+          } else {
+#pragma unroll
+            for (int q = 0; q < NT; q++) {  // f += (de / r) * d per neighbour-type group, the plain form
+              const bool mine = in[u] && tb[u] == (unsigned)q;
+              const double cq = mine ? coef : 0.0;
+              gx[q] += cq * dx[u];
+              gy[q] += cq * dy[u];
+              gz[q] += cq * dz[u];
+              if (ENERGY) ge[q] += mine ? ce : 0.0;
+              any[q] = any[q] || mine;
+            }
+          }
+        }
+        // sub-batches stay one behind the other, which bounds the registers
+        if (!MIXED) __builtin_amdgcn_sched_barrier(0);
       }
     }
+  };
+  walk(std::false_type{});
+  if (!MIXED && __builtin_expect(__any(rng.outside()), 0)) {
+#pragma unroll
+    for (int q = 0; q < NT; q++) {
+      gx[q] = gy[q] = gz[q] = ge[q] = 0.0;
+      any[q] = false;
+    }
+    walk(std::true_type{});
   }
   constexpr bool NEXT = EPI == EPI_NEXT;
   bool over = false;
