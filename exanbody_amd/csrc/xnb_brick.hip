@@ -82,11 +82,10 @@ static constexpr int LJB_UNROLL_B = (int)kListBatch;  // list entries per force 
 // the build reads whole candidate chunks of 32 from a row start and needs 32 of them
 static constexpr uint32_t kSentinels = 32;
 static constexpr int32_t kNoDelta = INT32_MIN;  // a region row whose cells' slots do not follow each other
-// region atoms a thread stages per memory round.  A 4x4x2 brick's region holds about 4.2
-// times its own atoms (the workgroup's lanes), so four a round leave a second round trip for
-// the last few; five or six a round measured the same for the mixed force kernel (other
-// workgroups hide the round trip), 2 % faster for the FP64 one (six) and 8 % slower for the
-// prefiltered build (six, more registers).
+// region atoms a thread of the build stages per memory round (the force's rounds: stage_region).
+// A 4x4x2 brick's region holds about 4.2 times its own atoms (the workgroup's lanes), so four a
+// round leave a second round trip for the last few; six were 8 % slower for the prefiltered
+// build (more registers).
 #ifndef XNB_STAGE_ROUND
 #define XNB_STAGE_ROUND 4
 #endif

@@ -243,7 +243,7 @@ __device__ inline void move_pack_bits(const uint32_t* __restrict__ dst, uint32_t
 
 // One thread per cell: packing (move_particles_across_cells.h:186-209).  Written out and searched
 // particle by particle in memory, which cells of more than 128 particles still do, a launch took
-// 36 us for a box of 500 atoms (62 a cell) and 23 us for one of 131,072.
+// 36 us for a box of 500 atoms (62 a cell; with the bits 22) and 23 us for one of 131,072 (8).
 __device__ inline void move_pack_item(Geom g, const uint32_t* __restrict__ cell_off, const uint32_t* __restrict__ cell_n,
                             const uint32_t* __restrict__ cnt_out, const uint32_t* __restrict__ cnt_in,
                             const uint32_t* __restrict__ mv_dst, uint32_t* __restrict__ pk, uint32_t* __restrict__ newloc,
