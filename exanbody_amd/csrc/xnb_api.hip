@@ -754,7 +754,7 @@ int xnb_destroy(xnb_ctx* c) {
                             &c->clen, &c->coff, &c->mv_dst, &c->pk, &c->newloc, &c->in_list, &c->plen, &c->pstart, &c->ghost_src,
                             &c->ghost_shift, &c->backup, &c->nbr, &c->nbr_cnt, &c->bsum, &c->u32s, &c->amr_list})
     dfree(c, *a);
-  dfree(c, c->blist); dfree(c, c->bcnt);
+  dfree(c, c->blist); dfree(c, c->bcnt); dfree(c, c->breg); dfree(c, c->blane);
   dfree(c, c->stream_buf); dfree(c, c->u64s); dfree(c, c->step_counts); dfree(c, c->red_part); dfree(c, c->red_out);
   if (c->h_u32) (void)hipHostFree(c->h_u32);
   if (c->h_u64) (void)hipHostFree(c->h_u64);
