@@ -496,22 +496,6 @@ int op_nbh_brick(xnb_ctx* c, double nbh_dist, const xnb_chunk_neighbors_config& 
   return NOT_APPLICABLE;
 }
 
-int finish_build(xnb_ctx* c, bool* fits) {
-  *fits = true;
-  if (!c->build_pending) return XNB_OK;
-  c->build_pending = false;
-  HIPCHK(c, hipStreamSynchronize(c->st));
-  const uint32_t mx = c->h_u32[kPendingWords], bad = c->h_u32[kPendingWords + 4];
-  if (bad) return fail(c, XNB_E_STATE, "brick sizes changed between statistics and build");
-  c->max_neighbors = mx;
-  if (mx > c->bp.cap) {
-    c->nbr_cap = grow_cap(mx);
-    c->lists_valid = false;
-    *fits = false;
-  }
-  return XNB_OK;
-}
-
 int op_nbh(xnb_ctx* c, double nbh_dist, const xnb_chunk_neighbors_config& cfg, int all_cells, const PairCut* pc) {
   const int lay = (int)std::ceil(nbh_dist / c->g.cs);  // cell_layers (amr_grid_algorithm.h:451)
   if (lay > 15) return fail(c, XNB_E_ARG, "neighbour distance spans more than 15 cells");
@@ -640,11 +624,56 @@ int ensure_regions(xnb_ctx* c, bool derive) {
   return XNB_OK;
 }
 
-int check_ctx(xnb_ctx* c) {
+int batch_lists(xnb_ctx* c, double margin, uint32_t lds_cap, bool quads, bool defer) {
+  const uint32_t keep = c->lds_limit;
+  xnb_chunk_neighbors_config cfg{1, 0, 0, 0, 0};
+  int e = XNB_OK;
+  bool done = false;
+  c->brick_margin = margin;
+  c->batch_lds = lds_cap;
+  c->batch_quads = quads;
+  c->batch_shapes = true;
+  c->defer_build = defer;
+  c->derive_ghosts = true;
+  if (lds_cap < keep) {
+    c->lds_limit = lds_cap;
+    e = op_nbh(c, c->nbh_dist_lab, cfg, 0);
+    c->lds_limit = keep;
+    done = e || c->list_kind == 1;
+  }
+  if (!done) e = op_nbh(c, c->nbh_dist_lab, cfg, 0);
+  c->batch_shapes = false;
+  c->defer_build = false;
+  return e;
+}
+
+int settle_build(xnb_ctx* c) {
+  if (!c->build_pending) return XNB_OK;
+  c->build_pending = false;
+  const bool was_valid = c->lists_valid;
+  c->lists_valid = false;  // until the words are seen
+  HIPCHK(c, hipStreamSynchronize(c->st));
+  const uint32_t mx = c->h_u32[kPendingWords], bad = c->h_u32[kPendingWords + 4];
+  if (bad) return fail(c, XNB_E_STATE, "brick sizes changed between statistics and build");
+  c->max_neighbors = mx;
+  c->lists_valid = was_valid;
+  if (mx <= c->bp.cap) return XNB_OK;
+  c->lists_valid = false;
+  c->nbr_cap = grow_cap(mx);
+  c->build_grown = true;
+  return batch_lists(c, c->brick_margin, c->batch_lds, c->batch_quads, false);
+}
+
+int ctx_device(xnb_ctx* c) {
   if (!c) return XNB_E_ARG;
   hipError_t e = hipSetDevice(c->device);
   if (e != hipSuccess) return fail(c, XNB_E_HIP, hipGetErrorString(e));
   return XNB_OK;
+}
+
+int check_ctx(xnb_ctx* c) {
+  const int e = ctx_device(c);
+  return e ? e : settle_build(c);
 }
 
 }  // namespace xnb_impl
@@ -1352,7 +1381,7 @@ extern "C" {
 
 int xnb_simulation_energies_noalloc(xnb_ctx* c, double* ke_pe) {
   int e;
-  if ((e = check_ctx(c))) return e;  // makes the context's device current
+  if ((e = ctx_device(c))) return e;  // reads no lists: nothing to settle, no wait
   if (!ke_pe) return fail(c, XNB_E_ARG, "null output");
   // the same partial count as xnb_simulation_energies, so the sums are the same bit for bit;
   // the reduction strides over the atoms, so every particle count fits kEnergyParts partials

@@ -533,28 +533,8 @@ uint32_t lds_cap_for(const xnb_batch* B, double frac) {
   return (uint32_t)(frac * B->lds_limit) - std::min<uint32_t>(st_lds + 64u, B->lds_limit / 8);
 }
 
-// chunk_neighbors of a box for the batch: brick head room and the batch's LDS cap per brick
-// workgroup, or the context's own limit when no brick fits the cap (restored afterwards)
 int batch_box_nbh(xnb_batch* B, xnb_ctx* c, bool quads, bool defer = false) {
-  c->brick_margin = B->brick_margin;
-  const uint32_t keep = c->lds_limit;
-  xnb_chunk_neighbors_config cfg{1, 0, 0, 0, 0};
-  int e = XNB_OK;
-  bool done = false;
-  c->batch_shapes = true;
-  c->batch_quads = quads;
-  c->defer_build = defer;
-  c->derive_ghosts = true;
-  if (B->brick_lds_cap < keep) {
-    c->lds_limit = B->brick_lds_cap;
-    e = op_nbh(c, c->nbh_dist_lab, cfg, 0);
-    c->lds_limit = keep;
-    done = e || c->list_kind == 1;
-  }
-  if (!done) e = op_nbh(c, c->nbh_dist_lab, cfg, 0);
-  c->batch_shapes = false;
-  c->defer_build = false;
-  return e;
+  return batch_lists(c, B->brick_margin, B->brick_lds_cap, quads, defer);
 }
 
 // One-box recovery after a batched rebuild overflowed the box's frame sizes: ghosts and
@@ -579,16 +559,17 @@ int recover_box(xnb_batch* B, int i, const xnb_run_params& p) {
   return XNB_OK;
 }
 
-// Attached boxes' deferred builds, before the batch reads their lists; lists that outgrew their
-// capacity are built again.
+// Attached boxes' deferred builds, before the batch reads their lists.  Lists that outgrew their
+// capacity were built again, here or by an operator called since the attach: their frames are
+// laid out anew.
 int settle_builds(xnb_batch* B) {
   for (int i = 0; i < (int)kMaxBatchBoxes; i++) {
     BatchBox& bb = B->box[i];
-    if (!bb.used || !bb.c->build_pending) continue;
-    bool fits;
-    int e = finish_build(bb.c, &fits);
-    if (!e && fits) continue;
-    if (!e && !(e = batch_box_nbh(B, bb.c, bb.quads))) {
+    if (!bb.used || (!bb.c->build_pending && !bb.c->build_grown)) continue;
+    int e = settle_build(bb.c);
+    if (!e && !bb.c->build_grown) continue;
+    bb.c->build_grown = false;
+    if (!e) {
       BHIP(B, hipStreamSynchronize(bb.c->st));
       frame_from_ctx(B, i, bb.p);
       if ((e = upload_frame(B, i))) return e;
@@ -730,6 +711,7 @@ int xnb_batch_attach(xnb_batch* B, xnb_ctx* c, const xnb_run_params* p, int* slo
   const bool quads = atoms <= kBatchQuadAtoms && c->N <= kBatchQuadBox;
   // the build is not waited for (one box's takes some 75 us on a mostly idle chip): the boxes'
   // builds run beside each other on their own streams until settle_builds
+  c->build_grown = false;
   if ((e = batch_box_nbh(B, c, quads, true))) return e;
   if (c->list_kind != 1) return bfail(B, XNB_E_STATE, "box geometry is not on the brick path (cell edge < nbh_dist)");
   if (brick_lds_bytes(c->bp, false) > B->lds_limit) return bfail(B, XNB_E_CAPACITY, "box bricks exceed LDS");
@@ -1114,10 +1096,8 @@ int xnb_batch_detach(xnb_batch* B, int slot, xnb_run_params* p) {
   BHIP(B, hipSetDevice(B->device));
   BHIP(B, hipStreamSynchronize(B->st));
   BatchBox& bb = B->box[slot];
-  if (bb.c->build_pending) {  // detached before any step
-    bool fits;
-    (void)finish_build(bb.c, &fits);
-  }
+  // detached before any step: its lists are marked invalid below, so nobody has to look at them
+  bb.c->build_pending = bb.c->build_grown = false;
   ctx_from_frame(B, slot, bb.finished ? bb.last_par : B->par);
   // a box detached before its last step keeps the fused first half of its next step; the
   // one-box loop restarts from a completed step, so only finished boxes are returned as

@@ -105,10 +105,12 @@ struct xnb_ctx {
   bool nbh_prefilter = true;        // unfiltered brick builds test in FP32 with an FP64 band (same lists)
   uint32_t lds_limit = 65536;
   bool batch_shapes = false;  // brick shapes offered to batched boxes only
-  // a build launched without waiting for its words (attach): taken as fitting until finish_build
+  // a build launched without waiting for its words (attach): taken as fitting until settle_build
   // has looked at them (h_u32 + kPendingWords)
   bool defer_build = false, build_pending = false;
+  bool build_grown = false;   // a deferred build did not fit and was done again (cleared by the batch's look at it)
   bool batch_quads = false;   // with batch_shapes: the shapes of four lanes an atom first
+  uint32_t batch_lds = 65536; // LDS bytes a brick workgroup of a batched box may take
   double brick_margin = 1.0;        // brick T / Rmax head room (batched boxes rebuild without re-choosing)
 
   double last_rcut = 0.;
@@ -160,7 +162,8 @@ int dalloc(xnb_ctx* c, DArr<T>& a, size_t n) {
 void bind_states(xnb_ctx* c);
 void swap_buffers(xnb_ctx* c);
 int ensure_capacity(xnb_ctx* c, size_t ncap, size_t keep);
-int check_ctx(xnb_ctx* c);
+int ctx_device(xnb_ctx* c);  // the context's device is current
+int check_ctx(xnb_ctx* c);   // and its lists are settled
 int scan(xnb_ctx* c, const uint32_t* in, uint32_t n, uint32_t add, uint32_t* out);
 int op_ghost_all(xnb_ctx* c, bool move_check = false, bool forces = true, bool update = false);
 int op_backup(xnb_ctx* c);
@@ -169,10 +172,15 @@ int op_nbh(xnb_ctx* c, double nbh_dist, const xnb_chunk_neighbors_config& cfg, i
 // forces false: f and ep neither carried by the move nor copied to ghosts; pc: per type-pair list radii
 int full_update(xnb_ctx* c, bool forces = true, const PairCut* pc = nullptr);
 int ensure_full_lists(xnb_ctx* c);
+// chunk_neighbors of a batched box: brick head room and the batch's LDS cap per brick workgroup,
+// or the context's own limit when no brick fits the cap; quads: laid out for four lanes an atom;
+// defer: the build is not waited for
+int batch_lists(xnb_ctx* c, double margin, uint32_t lds_cap, bool quads, bool defer);
 constexpr int kPendingWords = 48;
-// the end of a deferred build: waits for it, *fits false when its lists outgrew their capacity
-// (which has grown for the next build)
-int finish_build(xnb_ctx* c, bool* fits);
+// The end of a deferred build, if one is pending: waits for it and looks at its words; lists that
+// outgrew their capacity are built again.  check_ctx does it, so no operator meets lists that
+// nobody has looked at; the batch does it before it reads them.
+int settle_build(xnb_ctx* c);
 int ensure_regions(xnb_ctx* c, bool derive);
 void tstart(xnb_ctx* c, int id);
 void tstop(xnb_ctx* c);
