@@ -611,13 +611,16 @@ int ensure_full_lists(xnb_ctx* c) {
   return op_nbh(c, c->nbh_dist_lab, cfg, 0, nullptr);
 }
 
-// Brick lists' reg words name ghosts the way the caller needs them.
+// Brick lists' reg words name ghosts the way the caller needs them.  The steps of a batch that the
+// box is attached to read the same words on the batch's streams: they end first (the batch has the
+// words its way again before its next step).
 int ensure_regions(xnb_ctx* c, bool derive) {
   c->derive_ghosts = derive;
   if (!c->lists_valid || c->list_kind != 1) return XNB_OK;
   BrickParams bp = c->bp;
   bind_regions(c, bp, derive);
   if (bp.derive == c->bp.derive) return XNB_OK;
+  if (c->attached) HIPCHK(c, hipDeviceSynchronize());
   const hipError_t he = launch_brick_regions(c->g, bp, c->cell_off.p, c->cell_n.p, c->st);
   if (he != hipSuccess) return fail(c, XNB_E_HIP, std::string("brick regions: ") + hipGetErrorString(he));
   c->bp = bp;

@@ -561,12 +561,17 @@ int recover_box(xnb_batch* B, int i, const xnb_run_params& p) {
 
 // Attached boxes' deferred builds, before the batch reads their lists.  Lists that outgrew their
 // capacity were built again, here or by an operator called since the attach: their frames are
-// laid out anew.
+// laid out anew.  A force operator called since also left the box's reg words naming ghosts by
+// slot: they are written again the way the frame reads them.
 int settle_builds(xnb_batch* B) {
   for (int i = 0; i < (int)kMaxBatchBoxes; i++) {
     BatchBox& bb = B->box[i];
-    if (!bb.used || (!bb.c->build_pending && !bb.c->build_grown)) continue;
+    if (!bb.used) continue;
     int e = settle_build(bb.c);
+    if (!e && bb.c->bp.derive != bb.f.bp.derive) {
+      e = ensure_regions(bb.c, bb.f.bp.derive != 0);
+      if (!e) BHIP(B, hipStreamSynchronize(bb.c->st));
+    }
     if (!e && !bb.c->build_grown) continue;
     bb.c->build_grown = false;
     if (!e) {
@@ -734,6 +739,7 @@ int xnb_batch_attach(xnb_batch* B, xnb_ctx* c, const xnb_run_params* p, int* slo
   // the slot's status words: no overflow (a previous box may have left flags)
   BHIP(B, hipMemsetAsync(B->dwords.p + 4 * (size_t)i, 0, 4 * sizeof(uint32_t), B->st));
   bb.p = *p;
+  c->attached = true;
   c->last_rcut = p->rcut;
   frame_from_ctx(B, i, *p);
   if ((e = upload_frame(B, i))) return e;
@@ -1097,7 +1103,7 @@ int xnb_batch_detach(xnb_batch* B, int slot, xnb_run_params* p) {
   BHIP(B, hipStreamSynchronize(B->st));
   BatchBox& bb = B->box[slot];
   // detached before any step: its lists are marked invalid below, so nobody has to look at them
-  bb.c->build_pending = bb.c->build_grown = false;
+  bb.c->build_pending = bb.c->build_grown = bb.c->attached = false;
   ctx_from_frame(B, slot, bb.finished ? bb.last_par : B->par);
   // a box detached before its last step keeps the fused first half of its next step; the
   // one-box loop restarts from a completed step, so only finished boxes are returned as

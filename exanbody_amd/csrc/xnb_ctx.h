@@ -111,6 +111,7 @@ struct xnb_ctx {
   bool build_grown = false;   // a deferred build did not fit and was done again (cleared by the batch's look at it)
   bool batch_quads = false;   // with batch_shapes: the shapes of four lanes an atom first
   uint32_t batch_lds = 65536; // LDS bytes a brick workgroup of a batched box may take
+  bool attached = false;            // to a batch, from the attach to the detach
   double brick_margin = 1.0;        // brick T / Rmax head room (batched boxes rebuild without re-choosing)
 
   double last_rcut = 0.;
