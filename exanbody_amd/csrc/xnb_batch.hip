@@ -566,7 +566,7 @@ int recover_box(xnb_batch* B, int i, const xnb_run_params& p) {
 int settle_builds(xnb_batch* B) {
   for (int i = 0; i < (int)kMaxBatchBoxes; i++) {
     BatchBox& bb = B->box[i];
-    if (!bb.used) continue;
+    if (!active(bb)) continue;  // a finished or failed box's context is left alone until its detach
     int e = settle_build(bb.c);
     if (!e && bb.c->bp.derive != bb.f.bp.derive) {
       e = ensure_regions(bb.c, bb.f.bp.derive != 0);
@@ -712,7 +712,7 @@ int xnb_batch_attach(xnb_batch* B, xnb_ctx* c, const xnb_run_params* p, int* slo
   if ((e = ensure_capacity(c, (size_t)std::ceil((c->N + c->G) * B->slot_margin) + 256, (size_t)c->N + c->G))) return e;
   uint64_t atoms = c->N;
   for (const BatchBox& x : B->box)
-    if (x.used && !x.finished) atoms += x.c->N;
+    if (active(x)) atoms += x.f.N;
   const bool quads = atoms <= kBatchQuadAtoms && c->N <= kBatchQuadBox;
   // the build is not waited for (one box's takes some 75 us on a mostly idle chip): the boxes'
   // builds run beside each other on their own streams until settle_builds
