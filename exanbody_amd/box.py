@@ -283,8 +283,15 @@ class Box:
         self._check(self.L.xnb_copy_probe(self._h, int(nbytes), int(iters), C.byref(g)), "copy_probe")
         return g.value
 
+    def fp64_inv_sqrt(self, x):
+        """1 / sqrt(x) as the FP64 force kernels take it of a squared distance."""
+        x = np.ascontiguousarray(x, np.float64)
+        out = np.empty_like(x)
+        self._check(self.L.xnb_fp64_inv_sqrt(self._h, _ptr(x), x.size, _ptr(out)), "fp64_inv_sqrt")
+        return out
+
     def fp64_core(self, x):
-        """Device sqrt / reciprocal sequences of the FP64 force kernels applied to x."""
+        """Device sqrt of the FP64 force kernels, and a reciprocal on its own, applied to x."""
         x = np.ascontiguousarray(x, np.float64)
         sq, rc = np.empty_like(x), np.empty_like(x)
         self._check(self.L.xnb_fp64_core(self._h, _ptr(x), x.size, _ptr(sq), _ptr(rc)), "fp64_core")

@@ -1778,6 +1778,25 @@ int xnb_fp64_core(xnb_ctx* c, const double* x, size_t n, double* sqrt_out, doubl
   return XNB_OK;
 }
 
+int xnb_fp64_inv_sqrt(xnb_ctx* c, const double* x, size_t n, double* out) {
+  int e;
+  if ((e = check_ctx(c))) return e;
+  if (n == 0) return XNB_OK;
+  if (!x || !out) return fail(c, XNB_E_ARG, "null argument");
+  double* d = nullptr;
+  HIPCHK(c, hipMalloc((void**)&d, 2 * n * sizeof(double)));
+  hipError_t he = hipMemcpyAsync(d, x, n * sizeof(double), hipMemcpyHostToDevice, c->st);
+  if (he == hipSuccess) {
+    launch_fp64_inv_sqrt(d, n, d + n, c->st);
+    he = hipGetLastError();
+  }
+  if (he == hipSuccess) he = hipMemcpyAsync(out, d + n, n * sizeof(double), hipMemcpyDeviceToHost, c->st);
+  if (he == hipSuccess) he = hipStreamSynchronize(c->st);
+  (void)hipFree(d);
+  if (he != hipSuccess) return fail(c, XNB_E_HIP, std::string("fp64 inverse root: ") + hipGetErrorString(he));
+  return XNB_OK;
+}
+
 int xnb_device_bytes(const xnb_ctx* c, size_t* current, size_t* peak) {
   if (!c) return XNB_E_ARG;
   if (current) *current = c->dev_bytes;

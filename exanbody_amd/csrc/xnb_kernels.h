@@ -241,6 +241,7 @@ void launch_stream_fill(const Geom& g, uint32_t n_atoms, const uint32_t* slot_ce
                         const uint32_t* coff, int ntables, int random_access, uint16_t* out, hipStream_t st);
 void launch_copy_probe(const void* src, void* dst, size_t bytes, hipStream_t st);
 void launch_fp64_core(const double* x, size_t n, double* sq, double* rc, hipStream_t st);
+void launch_fp64_inv_sqrt(const double* x, size_t n, double* out, hipStream_t st);
 
 BrickParams brick_params(const Geom& g, int Bi, int Bj, int Bk);
 // LDS layout of the brick kernels (offsets into bp), its bytes; f32_build: the prefiltered

@@ -1228,17 +1228,30 @@ __global__ void __launch_bounds__(256) k_copy_probe(const uint4* __restrict__ sr
   for (size_t q = (size_t)blockIdx.x * 256 + threadIdx.x; q < n; q += (size_t)gridDim.x * 256) dst[q] = src[q];
 }
 
-// device evaluation of the FP64 sqrt / reciprocal sequences of the LJ kernels
+// device evaluation of the FP64 pair loops' root (xnb_fp64_core: with a reciprocal on its own) and
+// of their 1 / sqrt(d2), the generic operations where a list with this d2 is walked again
 __global__ void k_fp64_core(const double* __restrict__ x, size_t n, double* __restrict__ sq, double* __restrict__ rc) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  sq[i] = sqrt_normal(x[i]);
+  double h;
+  sq[i] = sqrt_normal(x[i], h);
   rc[i] = recip_normal(x[i]);
+}
+__global__ void k_fp64_inv_sqrt(const double* __restrict__ x, size_t n, double* __restrict__ out) {
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  PairRange rng;
+  rng.add(x[i]);
+  out[i] = rng.outside() ? 1.0 / sqrt(x[i]) : inv_sqrt_normal(x[i]);
 }
 
 void launch_fp64_core(const double* x, size_t n, double* sq, double* rc, hipStream_t st) {
   if (n == 0) return;
   k_fp64_core<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(x, n, sq, rc);
+}
+void launch_fp64_inv_sqrt(const double* x, size_t n, double* out, hipStream_t st) {
+  if (n == 0) return;
+  k_fp64_inv_sqrt<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(x, n, out);
 }
 
 void launch_copy_probe(const void* src, void* dst, size_t bytes, hipStream_t st) {

@@ -40,20 +40,20 @@ __device__ inline uint32_t wave_max_u32(uint32_t v) {
   return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
 }
 
-// Correctly rounded FP64 square root and reciprocal for normal-range arguments.
+// Correctly rounded FP64 square root and reciprocals for normal-range arguments.
 //
 // sqrt_normal: Goldschmidt iteration from the hardware reciprocal square root estimate
 // (v_rsq_f64), then two fma-corrected Newton steps on the root (P. Markstein, "IA-64 and
-// Elementary Functions", 2000, ch. 9).  recip_normal: two Newton-Raphson steps on the
-// hardware reciprocal estimate (v_rcp_f64) and one fma-corrected quotient step.  For
-// sqrt_normal(x), x in [2^-767, 2^1000], and recip_normal(y), y in [2^-383, 2^383], these
-// are the sequences hipcc emits for sqrt(x) and 1.0 / y without the range scaling and the
-// special-value fix-ups, which are identities there; the results are the IEEE correctly
-// rounded ones (checked against the host's IEEE sqrt and division by the GPU tests).
-__device__ inline double sqrt_normal(double x) {
+// Elementary Functions", 2000, ch. 9), for x in [2^-767, 2^1000]; h becomes 0.5 / sqrt(x) to
+// about 2^-45.  recip_normal, the reciprocal on its own (xnb_fp64_core): two Newton-Raphson steps
+// on the hardware estimate (v_rcp_f64) and one fma-corrected quotient step, for y in
+// [2^-383, 2^383].  The range scaling and special-value fix-ups of the general operations are
+// identities there; the results are the IEEE correctly rounded ones (the GPU tests compare them
+// with the host's over these ranges).
+__device__ inline double sqrt_normal(double x, double& h) {
   const double g = __builtin_amdgcn_rsq(x);
   double s = x * g;
-  double h = g * 0.5;
+  h = g * 0.5;
   const double r = fma(-h, s, 0.5);
   s = fma(s, r, s);
   h = fma(h, r, h);
@@ -73,24 +73,15 @@ __device__ inline double recip_normal(double y) {
   return fma(rem, a, a);
 }
 
-// RN(1 / RN(sqrt(x))) for x in [2^-767, 2^1000].  The root is sqrt_normal's; its iteration
-// leaves h = 0.5 / sqrt(x) to about 2^-45, so the reciprocal starts from 2 h instead of a
-// v_rcp_f64 estimate: one Newton-Raphson step brings it within 1 ulp of 1 / r and the last
-// fma-corrected step rounds it correctly (Markstein, as above) for every r but one whose
-// significand is all ones.  Those roots come from the two largest significands below a power
-// of 4 only; PairRange sends every x whose low word is 0xfffffffe or 0xffffffff (2 in 2^32) to
-// the generic operations.
+// RN(1 / RN(sqrt(x))) for x in [2^-767, 2^1000], what the FP64 pair loops take for 1.0 / r.  The
+// reciprocal starts from the root's own 2 h instead of a v_rcp_f64 estimate: one Newton-Raphson
+// step brings it within 1 ulp of 1 / r and the last fma-corrected step rounds it correctly
+// (Markstein, as above) for every r but one whose significand is all ones.  Those roots come from
+// the two largest significands below a power of 4 only; PairRange sends every x whose low word is
+// 0xfffffffe or 0xffffffff (2 in 2^32) to the generic operations.
 __device__ inline double inv_sqrt_normal(double x) {
-  const double g = __builtin_amdgcn_rsq(x);
-  double s = x * g;
-  double h = g * 0.5;
-  const double r = fma(-h, s, 0.5);
-  s = fma(s, r, s);
-  h = fma(h, r, h);
-  double d = fma(-s, s, x);
-  s = fma(d, h, s);
-  d = fma(-s, s, x);
-  s = fma(d, h, s);
+  double h;
+  const double s = sqrt_normal(x, h);
   double a = h + h;
   double e = fma(-s, a, 1.0);
   a = fma(e, a, a);

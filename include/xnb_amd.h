@@ -229,10 +229,12 @@ int xnb_device_bytes(const xnb_ctx* ctx, size_t* current, size_t* peak);
 /* Device copy of `bytes` (read + write), iters times, timed with HIP events: achieved GB/s
  * counting read and write bytes.  Also the known-size kernel that calibrates HBM counters. */
 int xnb_copy_probe(xnb_ctx* ctx, size_t bytes, int iters, double* gbps);
-/* Diagnostic with no counterpart in the reference: evaluates on the device the FP64 square
- * root and reciprocal sequences the plain-form LJ kernels use for r = sqrt(d2) and 1.0 / r,
- * so tests can check them against IEEE results.  sqrt_out[i] is defined for x[i] in
- * [2^-767, 2^1000], recip_out[i] for x[i] in [2^-383, 2^383]. */
+/* Diagnostics with no counterpart in the reference: evaluate FP64 sequences on the device, so
+ * tests can check them against IEEE results.  xnb_fp64_inv_sqrt: what the plain-form LJ kernels
+ * take for 1.0 / sqrt(d2), defined for x[i] in (0, 2^1000].  xnb_fp64_core: the square root in
+ * it, sqrt_out[i] defined for x[i] in [2^-767, 2^1000], and a reciprocal that stands on its own
+ * (the kernels take theirs from the root), recip_out[i] for x[i] in [2^-383, 2^383]. */
+int xnb_fp64_inv_sqrt(xnb_ctx* ctx, const double* x, size_t n, double* out);
 int xnb_fp64_core(xnb_ctx* ctx, const double* x, size_t n, double* sqrt_out, double* recip_out);
 
 /* ---- autotuning ------------------------------------------------------------------ */
