@@ -1039,7 +1039,7 @@ __device__ __forceinline__ void compute_pair_brick_body(const Geom& g, const Bri
   uint2 wn[W];
 #pragma unroll
   for (int w = 0; w < W; w++) wn[w] = t < T ? load_list_group(lst + (size_t)w * T) : make_uint2(0u, 0u);
-  stage_region<!Tr::Batched>(g, bp, b, r, L);
+  stage_region<PairTypes<Tr>::value>(g, bp, b, r, L);
   __syncthreads();
   const ForceAtom At = force_atom(bp, b, lw);
   const uint32_t n = At.live ? n_list : 0u;
@@ -1766,7 +1766,8 @@ hipError_t launch_lj_brick(int precision, bool accum, int epi, const Geom& g, Br
                            const uint16_t* blist, const uint32_t* bcnt, double eps, double sigma, double rcut,
                            double dth, const NextStep* next, hipStream_t st) {
   const LJConst lj = make_lj_const(eps, sigma, rcut);
-  const uint32_t lds = brick_force_layout(bp, false);
+  using Tr = ComputePairTraits<LennardJonesForceFunctor<false>>;
+  const uint32_t lds = brick_force_layout(bp, PairTypes<Tr>::value);
   const NextStep nx = next ? *next : NextStep{};
   const bool next_epi = epi == EPI_NEXT;
   if (next_epi && (accum || !next)) return hipErrorInvalidValue;
@@ -1819,7 +1820,7 @@ hipError_t launch_ljmm_brick(int precision, int ntypes, int epi, const Geom& g, 
 
 hipError_t launch_gravity_brick(const Geom& g, BrickParams bp, const PState& A, const uint16_t* blist, const uint32_t* bcnt, const GravitationalForceFunctor& gf, double rc2,
                                 hipStream_t st) {
-  const uint32_t lds = brick_force_layout(bp, true);
+  const uint32_t lds = brick_force_layout(bp, PairTypes<ComputePairTraits<GravitationalForceFunctor>>::value);
   hipError_t e = set_lds((const void*)k_compute_pair_brick<GravitationalForceFunctor>, lds);
   if (e != hipSuccess) return e;
   k_compute_pair_brick<GravitationalForceFunctor><<<kXcds * bp.per_xcd, bp.T, lds, st>>>(g, bp, A.r, blist, bcnt, gf,

@@ -364,6 +364,7 @@ struct ComputePairTraits<LennardJonesForceFunctor<MIXED>> {
   static constexpr bool CentralEnergy = true;
   static constexpr bool Batched = true;
   static constexpr bool Checked = !MIXED;
+  static constexpr bool Types = false;
 };
 
 // GravitationalForceFunctor (contribs/pi/gravitational_force.cu:44-82): Newtonian attraction

@@ -42,6 +42,9 @@
  * a wave whose lists held one outside, or any wave when unchecked_parameters() is true, is
  * walked again from zero sums with batch.
  *
+ * Traits that set Types to false say that the functor looks at no particle type (type_a,
+ * cells[..][field::type], NbhBatch::type_of): the traversal then stages none.
+ *
  * The traversals are instantiated inside the library: compute_pair_brick_body (brick lists,
  * exanbody_amd/csrc/xnb_brick.hip) and k_compute_pair_slots (per-slot lists, all cells,
  * exanbody_amd/csrc/xnb_kernels.hip).  A new functor is written beside
@@ -82,6 +85,17 @@ struct PairChecked<T, decltype(void(T::Checked))> {
   static constexpr bool value = T::Checked;
 };
 
+/* ComputePairTraits<F>::Types, true for traits without it: the functor may look at types */
+template <class T, class = void>
+struct PairTypes {
+  static constexpr bool value = true;
+};
+template <class T>
+struct PairTypes<T, decltype(void(T::Types))> {
+  static constexpr bool value = T::Types;
+  static_assert(T::Types || !T::CentralType, "a functor that takes type_a looks at types");
+};
+
 namespace field {
 struct type_t {};
 constexpr type_t type{};
@@ -112,7 +126,7 @@ struct NbhBatch {
   uint32_t off[U];     /* LDS byte address of neighbour u's x (24 j[u]: the staged positions
                           start at LDS address 0, the traversal kernels hold no static LDS) */
   const double* pos;   /* x, y, z of region atom i at pos[3 i], pos[3 i + 1], pos[3 i + 2] */
-  const uint8_t* type; /* type of region atom i at type[i] */
+  const uint8_t* type; /* type of region atom i at type[i] (unless the traits set Types to false) */
   __device__ double4 operator()(int u) const {
     /* read through an LDS-space pointer made from the address, so that forming it is one
        24-bit multiply of the list entry's half-word */
