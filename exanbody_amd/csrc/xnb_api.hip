@@ -1584,13 +1584,14 @@ int xnb_run_multimat(xnb_ctx* c, xnb_run_params* p, int ntypes, const double* ep
 // ---- autotuner: brick shape (cells per workgroup tile) by measurement, cached per class
 namespace {
 struct TuneKey {
-  int di, dj, dk, occ, precision;
+  int di, dj, dk, occ, precision, lanes;
   bool operator<(const TuneKey& o) const {
     if (di != o.di) return di < o.di;
     if (dj != o.dj) return dj < o.dj;
     if (dk != o.dk) return dk < o.dk;
     if (occ != o.occ) return occ < o.occ;
-    return precision < o.precision;
+    if (precision != o.precision) return precision < o.precision;
+    return lanes < o.lanes;
   }
 };
 std::mutex g_tune_mu;
@@ -1608,9 +1609,12 @@ int xnb_autotune(xnb_ctx* c, const xnb_lj_params* p, double rcut, int precision,
     return XNB_OK;
   }
   const Geom& g = c->g;
-  // class: cells per side (large boxes alike), mean atoms per inner cell, precision
+  // class: cells per side (large boxes alike), mean atoms per inner cell, precision, lanes an atom (a
+  // shape timed with four lanes says nothing about the kernel with one)
   const double occ = (double)c->N / ((double)g.Di * g.Dj * g.Dk);
-  const TuneKey key{std::min(g.Di, 16), std::min(g.Dj, 16), std::min(g.Dk, 16), (int)std::lround(occ), precision};
+  xnb_chunk_neighbors_config cfg{1, 0, 0, 0, 0};
+  const TuneKey key{std::min(g.Di, 16),    std::min(g.Dj, 16), std::min(g.Dk, 16),
+                    (int)std::lround(occ), precision,          quad_lists(c, cfg) ? (int)kQuad : 1};
   std::array<int, 3> best{0, 0, 0};
   bool cached = false;
   {
@@ -1622,7 +1626,6 @@ int xnb_autotune(xnb_ctx* c, const xnb_lj_params* p, double rcut, int precision,
     }
   }
   const int saved[3] = {c->brick_dims[0], c->brick_dims[1], c->brick_dims[2]};
-  xnb_chunk_neighbors_config cfg{1, 0, 0, 0, 0};
   if (!cached) {
     static const int cand[][3] = {{4, 4, 2}, {4, 2, 2}, {2, 4, 2}, {4, 4, 1}, {2, 2, 2}, {4, 2, 1}};
     struct Events {  // destroyed on every return path

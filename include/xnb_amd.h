@@ -241,8 +241,8 @@ int xnb_fp64_core(xnb_ctx* ctx, const double* x, size_t n, double* sqrt_out, dou
 /* No counterpart in the reference.  Picks the brick shape (cells per workgroup tile; the tile's
  * atoms are the workgroup's lanes) of an initialised box by timing its LJ force kernel for each
  * candidate shape, and rebuilds its lists with the fastest; results are cached per process by
- * (cells per side up to 16, mean atoms per cell, precision), so boxes of a seen class are not
- * timed again.  Forces and energies are recomputed (bitwise the same: the shape does not enter
+ * (cells per side up to 16, mean atoms per cell, precision, lanes an atom), so boxes of a seen
+ * class are not timed again.  Forces and energies are recomputed (bitwise the same: the shape does not enter
  * the arithmetic).  dims_out (optional) receives the shape, 0s off the brick path. */
 int xnb_autotune(xnb_ctx* ctx, const xnb_lj_params* params, double rcut, int precision, int* dims_out);
 
