@@ -92,9 +92,12 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_scan_apply(const uint32_t* in,
   }
 }
 
-// One workgroup, 8 items a thread and tile: up to kScanOneBlock items take one launch of a few
-// microseconds where the three kernels above take three of 4 us each, one after another.
-static constexpr uint32_t kScanOneBlock = 32768;
+// One workgroup, 8 items a thread and tile, for up to kScanOneBlock items: one launch bound by the
+// latency of a CU's loads, about 0.9 us per 1,000 items, where the three kernels above take 7.4 to
+// 8.5 us whatever the size.  One and three, each scan behind the last (us): 1,000 items 2.7 and
+// 7.4; 4,096 5.4 and 7.7; 5,832 6.8 and 7.8; 8,000 8.6 and 7.8; 16,384 15.9 and 8.5; 32,768 30.0
+// and 8.5.
+static constexpr uint32_t kScanOneBlock = 6144;
 __global__ void __launch_bounds__(1024) k_scan_one_block(const uint32_t* in, uint32_t n, uint32_t add, uint32_t* out,
                                                          uint32_t* total) {
   __shared__ uint32_t wsum[16];
