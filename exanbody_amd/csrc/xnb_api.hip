@@ -451,6 +451,13 @@ void bind_regions(xnb_ctx* c, BrickParams& bp, bool derive) {
   bp.ghost_shift = c->ghost_shift.p;
 }
 
+// chunk_neighbors of a box of at least this many atoms leaves out the words the force reads;
+// ensure_regions writes them for the first force, so a caller that only wants lists does not pay
+// for them.  Lists alone, words in the build and left out (us): 1,000,000 atoms 456 and 431,
+// 1,500,000 613 and 573, 2,048,000 753 and 698, 8,388,608 2,612 and 2,389; lists and one force:
+// 642 and 652, 862 and 871, 1,071 and 1,074, 3,994 and 3,935.
+constexpr uint32_t kWordsLaterAtoms = 1500000;
+
 int op_nbh_brick(xnb_ctx* c, double nbh_dist, const xnb_chunk_neighbors_config& cfg, const PairCut& pc) {
   const double max2 = nbh_dist * nbh_dist;
   int e;
@@ -465,10 +472,13 @@ int op_nbh_brick(xnb_ctx* c, double nbh_dist, const xnb_chunk_neighbors_config& 
     if ((e = dalloc(c, c->breg, brick_reg_words(bp)))) return e;
     if ((e = dalloc(c, c->blane, (size_t)bp.nbricks * bp.T))) return e;
     bind_regions(c, bp, c->derive_ghosts);
+    const bool words = !c->words_later || bp.lanes != 1 || !(cfg.half_symmetric || cfg.skip_ghosts || c->nbh_prefilter);
+    BrickParams bb = bp;
+    if (!words) bb.reg = bb.lane = nullptr;
     if (clear) HIPCHK(c, hipMemsetAsync(c->u32s.p + 2, 0, 5 * sizeof(uint32_t), c->st));
     clear = true;
     tstart(c, XNB_TIMER_NBH);
-    hipError_t he = launch_nbh_brick(c->g, bp, c->A.r, c->cell_off.p, c->cell_n.p, max2, pc, cfg.half_symmetric, cfg.skip_ghosts,
+    hipError_t he = launch_nbh_brick(c->g, bb, c->A.r, c->cell_off.p, c->cell_n.p, max2, pc, cfg.half_symmetric, cfg.skip_ghosts,
                                      c->nbh_prefilter, c->blist.p, c->bcnt.p, c->u32s.p + 2, c->st);
     tstop(c);
     if (he != hipSuccess) return fail(c, XNB_E_HIP, std::string("brick neighbour build: ") + hipGetErrorString(he));
@@ -482,6 +492,7 @@ int op_nbh_brick(xnb_ctx* c, double nbh_dist, const xnb_chunk_neighbors_config& 
     if (!c->defer_build) c->max_neighbors = mx;
     if (mx <= bp.cap) {
       c->bp = bp;
+      c->words_current = words;
       c->nbr_cap = bp.cap;
       c->list_kind = 1;
       c->slot_lists_current = false;
@@ -611,7 +622,7 @@ int ensure_full_lists(xnb_ctx* c) {
   return op_nbh(c, c->nbh_dist_lab, cfg, 0, nullptr);
 }
 
-// Brick lists' reg words name ghosts the way the caller needs them.  The steps of a batch that the
+// Brick lists' words are there and name ghosts the way the caller needs them.  The steps of a batch that the
 // box is attached to read the same words on the batch's streams: they end first (the batch has the
 // words its way again before its next step).
 int ensure_regions(xnb_ctx* c, bool derive) {
@@ -619,11 +630,12 @@ int ensure_regions(xnb_ctx* c, bool derive) {
   if (!c->lists_valid || c->list_kind != 1) return XNB_OK;
   BrickParams bp = c->bp;
   bind_regions(c, bp, derive);
-  if (bp.derive == c->bp.derive) return XNB_OK;
+  if (bp.derive == c->bp.derive && c->words_current) return XNB_OK;
   if (c->attached) HIPCHK(c, hipDeviceSynchronize());
   const hipError_t he = launch_brick_regions(c->g, bp, c->cell_off.p, c->cell_n.p, c->st);
   if (he != hipSuccess) return fail(c, XNB_E_HIP, std::string("brick regions: ") + hipGetErrorString(he));
   c->bp = bp;
+  c->words_current = true;
   return XNB_OK;
 }
 
@@ -1177,7 +1189,10 @@ int xnb_chunk_neighbors(xnb_ctx* c, double nbh_dist_lab, const xnb_chunk_neighbo
   if ((e = check_ctx(c))) return e;
   xnb_chunk_neighbors_config k = cfg ? *cfg : xnb_chunk_neighbors_config{1, 0, 0, 0, 0};
   if (k.dual_particle_offset) k.build_particle_offset = 1;  // chunk_neighbors_config.h:76-80
-  return op_nbh(c, nbh_dist_lab, k, all_cells);
+  c->words_later = c->N >= kWordsLaterAtoms;
+  e = op_nbh(c, nbh_dist_lab, k, all_cells);
+  c->words_later = false;
+  return e;
 }
 
 int xnb_chunk_neighbors_stream(xnb_ctx* c, uint16_t* out, size_t cap, uint64_t* cell_offsets, size_t* total,

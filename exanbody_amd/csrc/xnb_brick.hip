@@ -495,7 +495,8 @@ __device__ inline BrickLds force_lds(const BrickParams& bp, char* lds) {
   return L;
 }
 
-// reg words of every brick again, for lists that stay (ghosts by slot or by source)
+// reg and lane words of every brick, for lists that stay: the ghosts named the other way (by slot
+// or by source), or lists built without the words
 __global__ void __launch_bounds__(1024) k_brick_regions(Geom g, BrickParams bp, const uint32_t* __restrict__ cell_off,
                                                         const uint32_t* __restrict__ cell_n) {
   extern __shared__ __align__(16) char lds[];
@@ -514,6 +515,8 @@ __global__ void __launch_bounds__(1024) k_brick_regions(Geom g, BrickParams bp, 
     const uint32_t c = upper_index(L.rpref, (uint32_t)bp.nrc, idx);
     reg[idx] = region_word(bp, L.roff[c] + (idx - L.rpref[c]));
   }
+  const LaneAtom A = lane_atom(bp, L, threadIdx.x);
+  bp.lane[(size_t)b * bp.T + threadIdx.x] = A.live ? A.ia | A.bc << 16 : NONE;  // T threads
 }
 
 // ------------------------------------------------------------------ statistics
@@ -581,7 +584,8 @@ __global__ void __launch_bounds__(256) k_brick_stats(Geom g, BrickShapes sh, con
 // pair's radius while the mask is expanded.
 // LANES 4 (prefiltered builds of small boxes): four lanes share an atom.  Each tests its quarter
 // of a row's candidates; their kept counts give each lane the place of its entries in the list.
-template <bool FILTER, bool PAIRWISE = false, bool PREF = false, uint32_t LANES = 1>
+// WORDS false: the brick's words are left out (bp.reg null).
+template <bool FILTER, bool PAIRWISE = false, bool PREF = false, uint32_t LANES = 1, bool WORDS = true>
 __device__ __forceinline__ void nbh_brick_body(const Geom& g, const BrickParams& bp, uint32_t b, const double4* __restrict__ r,
                                                const uint32_t* __restrict__ cell_off, const uint32_t* __restrict__ cell_n,
                                                double max2, int half_symmetric, int skip_ghosts, uint16_t* __restrict__ blist,
@@ -593,11 +597,12 @@ __device__ __forceinline__ void nbh_brick_body(const Geom& g, const BrickParams&
   const BrickLds L = brick_lds(bp, lds);
   const BrickPos P = brick_pos(g, bp, b);
   if (!brick_setup(g, bp, P, L, r, cell_off, cell_n, PREF ? (PAIRWISE ? kPosF32N : kPosF32) : kPosF64,
-                   bp.reg + (size_t)b * (bp.Rmax + 1u)))
+                   WORDS ? bp.reg + (size_t)b * (bp.Rmax + 1u) : nullptr))
     return;
   const uint32_t t = threadIdx.x / LANES, T = bp.T;
   const LaneAtom A = lane_atom(bp, L, t);
-  if (threadIdx.x % LANES == 0 && t < T) __builtin_nontemporal_store(A.live ? A.ia | A.bc << 16 : NONE, bp.lane + (size_t)b * T + t);
+  if (WORDS && threadIdx.x % LANES == 0 && t < T)
+    __builtin_nontemporal_store(A.live ? A.ia | A.bc << 16 : NONE, bp.lane + (size_t)b * T + t);
   uint16_t* out = blist + (size_t)b * bp.cap * T;
   // every lane, live or not, tests against its own LDS atom when past the candidate cell's
   // end (A.ia = 0 for lanes without an atom), so d2 == 0 rejects those candidates
@@ -974,14 +979,14 @@ __device__ __forceinline__ void nbh_brick_body(const Geom& g, const BrickParams&
   for (uint32_t q = min(cnt, bp.cap); q < pad_end; q++) out[lpos(q, t, T)] = sentinel;
 }
 
-template <bool FILTER, bool PAIRWISE, bool PREF = false, uint32_t LANES = 1>
+template <bool FILTER, bool PAIRWISE, bool PREF = false, uint32_t LANES = 1, bool WORDS = true>
 __global__ void __launch_bounds__(1024) k_nbh_brick_mask(Geom g, BrickParams bp, const double4* __restrict__ r,
                                                          const uint32_t* __restrict__ cell_off, const uint32_t* __restrict__ cell_n,
                                                          double max2, int half_symmetric, int skip_ghosts, uint16_t* __restrict__ blist,
                                                          uint32_t* __restrict__ bcnt, uint32_t* __restrict__ max_cnt, PairCut pc) {
   const uint32_t b = brick_of_block<true>(bp);
   if (b >= bp.nbricks) return;  // whole workgroup, before any barrier
-  nbh_brick_body<FILTER, PAIRWISE, PREF, LANES>(g, bp, b, r, cell_off, cell_n, max2, half_symmetric, skip_ghosts, blist, bcnt, max_cnt, &pc);
+  nbh_brick_body<FILTER, PAIRWISE, PREF, LANES, WORDS>(g, bp, b, r, cell_off, cell_n, max2, half_symmetric, skip_ghosts, blist, bcnt, max_cnt, &pc);
 }
 
 // ------------------------------------------------------------------ pair traversal
@@ -1714,12 +1719,14 @@ hipError_t launch_nbh_brick(const Geom& g, BrickParams bp, const double4* r, con
   const uint32_t lds = brick_layout(bp);
   hipError_t e;
   if (bp.lanes != 1 && (half_symmetric || skip_ghosts || !prefilter)) return hipErrorInvalidValue;
+  const bool words = bp.reg != nullptr;
+  if (!words && (bp.lanes != 1 || pc.nt > 0 || !(half_symmetric || skip_ghosts || prefilter))) return hipErrorInvalidValue;
   if (half_symmetric || skip_ghosts) {
     if (pc.nt > 0) return hipErrorInvalidValue;
-    e = set_lds((const void*)k_nbh_brick_mask<true, false>, lds);
+    auto* const fn = words ? k_nbh_brick_mask<true, false> : k_nbh_brick_mask<true, false, false, 1, false>;
+    e = set_lds((const void*)fn, lds);
     if (e != hipSuccess) return e;
-    k_nbh_brick_mask<true, false><<<kXcds * bp.per_xcd, bp.T, lds, st>>>(g, bp, r, cell_off, cell_n, max2, half_symmetric, skip_ghosts,
-                                                                        blist, bcnt, max_cnt, pc);
+    fn<<<kXcds * bp.per_xcd, bp.T, lds, st>>>(g, bp, r, cell_off, cell_n, max2, half_symmetric, skip_ghosts, blist, bcnt, max_cnt, pc);
   } else if (pc.nt > 0 && prefilter) {
     BrickParams bq = bp;
     const uint32_t lds_b = brick_layout(bq, true, true);
@@ -1735,7 +1742,9 @@ hipError_t launch_nbh_brick(const Geom& g, BrickParams bp, const double4* r, con
   } else if (prefilter) {
     BrickParams bq = bp;  // the same bricks and lists, the prefilter's smaller LDS layout
     const uint32_t lds_b = brick_layout(bq, true);
-    auto* const fn = bq.lanes == kQuad ? k_nbh_brick_mask<false, false, true, kQuad> : k_nbh_brick_mask<false, false, true>;
+    auto* const fn = bq.lanes == kQuad ? k_nbh_brick_mask<false, false, true, kQuad>
+                     : words           ? k_nbh_brick_mask<false, false, true>
+                                       : k_nbh_brick_mask<false, false, true, 1, false>;
     e = set_lds((const void*)fn, lds_b);
     if (e != hipSuccess) return e;
     fn<<<kXcds * bq.per_xcd, bq.T * bq.lanes, lds_b, st>>>(g, bq, r, cell_off, cell_n, max2, 0, 0, blist, bcnt, max_cnt, pc);

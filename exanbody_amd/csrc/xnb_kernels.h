@@ -41,7 +41,8 @@ struct BrickParams {
   uint32_t off_rcnt, off_rpref, off_roff, off_bpref, off_pos, off_type;  // LDS byte offsets
   uint32_t off_rdel, off_crow;  // staging tables: per region row, per 64 region atoms
   uint32_t off_wsum;            // 32 scan words, then the 2 wave-group counter words
-  // the region as the force kernels read it, written by the build (see region_word)
+  // the region as the force kernels read it, written by the build (see region_word); null: a build
+  // that leaves them out
   uint32_t* reg;                // (Rmax + 1) words per brick
   uint32_t* lane;               // T words per brick
   uint32_t derive;              // 1: ghosts by source slot and shift, 0: by their own slot
@@ -249,7 +250,7 @@ BrickParams brick_params(const Geom& g, int Bi, int Bj, int Bk);
 uint32_t brick_layout(BrickParams& bp, bool f32_build = false, bool f32_types = false);
 uint32_t brick_force_layout(BrickParams& bp, bool types);  // of the force kernels
 size_t brick_reg_words(const BrickParams& bp);
-// bp.reg again for bp.derive (the lists and lane words stay)
+// bp.reg for bp.derive and bp.lane, for lists that stay
 hipError_t launch_brick_regions(const Geom& g, BrickParams bp, const uint32_t* cell_off, const uint32_t* cell_n, hipStream_t st);
 uint32_t brick_list_granule();
 // brick shapes whose occupancy is looked at together; out: 2 words a shape, 0 on entry
