@@ -57,14 +57,24 @@ struct BatchBox {
 // 3.92e9, 1.15 4.27e9, 1.18 4.21e9, 1.21 3.94e9, 1.35 3.88e9, 1.5 3.45e9; 1.0 recovers
 // thousands of times.
 constexpr double kBrickMargin = 1.15;
-// Boxes attached while the batch holds at most this many unfinished atoms, theirs included, get
-// small bricks built with four lanes an atom (a step's build covers the few boxes that rebuild and
-// takes as long as one lane needs); their force takes four lanes when the step's atoms are at
-// most kQuadAtoms.  24 boxes of 500 to 8,000 atoms (66,000 in all), FP64, 50 steps on the
-// displacement trigger: build 75 to 90 -> 41 us, force 40 -> 24 us, steps 13.3 -> 10.7 ms.  In a
-// large batch small bricks stage more than they gain (64 boxes of 500 to 50,000 atoms, the first
-// 131,072 atoms so: steps 18.5 -> 21.0 ms), so only boxes that are small themselves take them.
-constexpr uint64_t kBatchQuadAtoms = 98304, kBatchQuadBox = 8192;
+// Small boxes get small bricks built with four lanes an atom (a step's build covers the few boxes
+// that rebuild and takes as long as one lane needs); their force takes four lanes when the step's
+// atoms are at most kQuadAtoms.  24 boxes of 500 to 8,000 atoms (66,000 in all), FP64, 50 steps on
+// the displacement trigger: build 75 to 90 -> 41 us, force 40 -> 24 us, steps 13.3 -> 10.7 ms.
+//
+// Which boxes: at most kBatchQuadBox atoms, attached while the batch holds at most kBatchQuadAtoms
+// unfinished atoms, theirs included; and, on the displacement trigger, every box of at most
+// kBatchQuadSmall: there some box rebuilds in almost every step, so the build decides.  100 steps
+// on the trigger with one and with four lanes for all boxes, FP64 (mixed), ms: 48 boxes of 4,000
+// atoms 28.2 and 23.1 (25.6 and 21.4), 192 of 4,000 46.9 and 44.1 (38.9 and 37.6), 200 of 1,000
+// 28.7 and 25.1, 12 of 8,000 21.6 and 19.4, 32 of 8,000 28.3 and 28.7, 64 of 8,000 35.5 and 41.5.  A
+// batch that is part one, part the other launches more kernels a rebuild and lies above both (48
+// of 4,000, 24 of them with four lanes: 28.9; 32 of 8,000, 12 of them: 30.3; 64 of 8,000, 49 of
+// them: 42.6, 12 of them: 38.5).  With a fixed interval all boxes rebuild together and the force
+// counts more: 100 steps rebuilt every 10, 32 of 1,000 5.9 and 4.6, 8 of 4,000 5.2 and 4.0, 24 of
+// 4,000 8.0 and 6.3, 16 of 6,000 7.4 and 6.5; where a 2x2x2 brick does not fit four lanes it loses,
+// 32 of 2,000 6.0 and 7.0, 19 of 5,000 5.7 and 7.9, as do 12 of 8,000, 7.6 and 8.4.
+constexpr uint64_t kBatchQuadAtoms = 98304, kBatchQuadBox = 8192, kBatchQuadSmall = 4096;
 // A class of brick launches with fewer workgroups than this joins the next larger one: alone it
 // is another launch in the step's chain (64 boxes: 8 of 2,128 workgroups).
 constexpr uint32_t kClassBricks = 128;
@@ -713,7 +723,7 @@ int xnb_batch_attach(xnb_batch* B, xnb_ctx* c, const xnb_run_params* p, int* slo
   uint64_t atoms = c->N;
   for (const BatchBox& x : B->box)
     if (active(x)) atoms += x.f.N;
-  const bool quads = atoms <= kBatchQuadAtoms && c->N <= kBatchQuadBox;
+  const bool quads = (c->N <= kBatchQuadBox && atoms <= kBatchQuadAtoms) || (c->N <= kBatchQuadSmall && p->rebuild_every <= 0);
   // the build is not waited for (one box's takes some 75 us on a mostly idle chip): the boxes'
   // builds run beside each other on their own streams until settle_builds
   c->build_grown = false;

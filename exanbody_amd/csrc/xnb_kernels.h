@@ -21,9 +21,12 @@ constexpr uint32_t kListBatch = 8;
 constexpr uint32_t kQuad = 4, kQuadBatch = 16;
 // Boxes of at most this many atoms give every atom four lanes (four atoms' lanes fill two waves
 // per SIMD of the chip; larger boxes have enough waves with one lane an atom, which takes 1.7
-// times fewer instructions).  Force and build launch with one and with four lanes: 6,912 atoms
-// FP64 20.5 and 13.6, 68 and 28 us; 27,431 atoms mixed 15.8 and 15.5, 68 and 38 us; 131,072
-// atoms FP64 36 and 50, 89 and 104 us.
+// times fewer instructions).  200 steps rebuilt every 10, with one and with four lanes, FP64
+// (mixed), ms: 12,000 atoms 6.74 and 4.80 (5.99 and 4.53), 20,000 7.09 and 5.07 (6.19 and 4.57),
+// 24,000 6.87 and 6.35 (5.96 and 5.63), 28,000 7.02 and 6.83 (6.17 and 6.10), 32,000 6.71 and 6.40
+// (5.90 and 5.68), 36,000 6.99 and 6.66 (6.15 and 5.88), 44,000 8.34 and 9.93 (6.80 and 8.90),
+// 64,000 8.91 and 10.46 (7.31 and 9.39).  From 24,000 on the build gains (75 -> 46 us) and the force
+// alone is level (FP64 20.5 and 22.0, mixed 16.2 and 18.0 us).
 constexpr uint32_t kQuadAtoms = 32768;
 
 struct BrickParams {
