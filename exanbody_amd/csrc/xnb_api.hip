@@ -445,7 +445,7 @@ int choose_bricks(xnb_ctx* c, uint32_t cap, bool quads, BrickParams& out) {
 void bind_regions(xnb_ctx* c, BrickParams& bp, bool derive) {
   bp.reg = c->breg.p;
   bp.lane = c->blane.p;
-  bp.derive = derive && c->N < kDeriveSlots ? 1u : 0u;
+  bp.derive = derive && c->N < c->derive_slots ? 1u : 0u;
   bp.n_inner = c->N;
   bp.ghost_src = c->ghost_src.p;
   bp.ghost_shift = c->ghost_shift.p;
@@ -772,6 +772,8 @@ int xnb_create(xnb_ctx** out, const xnb_domain* d, int device) {
     if (v[0] == '0' && v[1] == 0) c->use_bricks = false;
     else std::sscanf(v, "%d,%d,%d,%d", &c->brick_dims[0], &c->brick_dims[1], &c->brick_dims[2], &c->brick_lanes);
   }
+  if (const char* v = std::getenv("XNB_DERIVE_SLOTS"))  // fewer inner slots than this name ghosts by their sources
+    c->derive_slots = (uint32_t)std::min<unsigned long>(std::strtoul(v, nullptr, 10), kDeriveSlots);
   if (const char* v = std::getenv("XNB_FUSE_PUSH")) c->fuse_push = v[0] != '0';
   if (const char* v = std::getenv("XNB_NBH_PREFILTER")) c->nbh_prefilter = v[0] != '0';
   HIPCHK(c, hipMemsetAsync(c->cell_n.p, 0, c->cell_n.n * sizeof(uint32_t), c->st));

@@ -100,6 +100,7 @@ struct xnb_ctx {
   // ghosts in the brick lists' reg words by source and shift (the run loops and batches, whose
   // ghosts always follow their sources) or by slot (operators, which read the ghosts as they are)
   bool derive_ghosts = false;
+  uint32_t derive_slots = kDeriveSlots;
   bool words_later = false, words_current = true;  // the next build leaves the words out; the lists' words are there
   bool slot_lists_current = false;  // nbr/nbr_cnt mirror the brick lists
   bool fuse_push = true;            // force kernel performs the next step's first half (brick lists)
