@@ -12,8 +12,8 @@
 #include <atomic>
 #include <condition_variable>
 #include <cstring>
+#include <exception>
 #include <mutex>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -69,6 +69,7 @@ struct Block {
           p = (char*)h;
           return;
         }
+        (void)hipGetLastError();  // dealt with here: a later launch's check must not find it
         if (P.n_blocks == 0) return;
       }
       if (!wait) return;
@@ -143,7 +144,7 @@ int read_chunks(xnb_ctx* c, size_t n, size_t per, size_t bytes, const Launch& la
       th[started] = std::thread(work, false);
       started++;
     }
-  } catch (const std::system_error&) {  // fewer threads: the chunks go to those there are
+  } catch (const std::exception&) {  // no thread, or no memory for one: the chunks go to those there are
   }
   work(true);
   for (int q = 0; q < started; q++) th[q].join();
