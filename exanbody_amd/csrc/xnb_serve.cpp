@@ -126,32 +126,40 @@ extern "C" {
 // capacity growth step): two copies of the particle state, backup, scratch and the ghost
 // scheme, ~500 B per slot.  Brick lists: 4 B per neighbour within the list radius (u16
 // entries in both directions, lane and wave padding, the brick head room).  Cells: the
-// per-cell tables, ~64 B per cell with the ghost layers.  Plus a fixed 16 MiB for the scalar
-// buffers, reduction partials and launch tables.  Checked against counted allocations from
-// 300 to 200k atoms, densities 0.6 to 1.6 and list radii 2.8 to 4.4 (measured peaks 0.65-0.8
-// of this from 30k atoms on).
-static size_t job_bytes(double slots, double atoms, double neighbours, double cells) {
-  const double b = slots * 500.0 + atoms * 4.0 * std::max(neighbours, 0.0) + cells * 64.0;
+// per-cell tables, ~64 B per cell with the ghost layers.  A fixed 16 MiB for the scalar
+// buffers, reduction partials and launch tables, which also holds the staging words of the first
+// 32,768 atoms.  Staging words of the others: 4 B for every atom of a brick's region, 4.5 times
+// the brick's own atoms with thin cells (bricks of 4x4x2 cells) up to 27 times (one cell) as the
+// cells fill and the bricks shrink to fit LDS, times the brick head room and the fullest brick's
+// lead (together 1.5), and 4 B a lane.  Checked against counted allocations from 300 to 4M
+// atoms, densities 0.6 to 1.6 and list radii 2.8 to 4.4, up to about 80 atoms a cell (measured
+// peaks 0.58-0.97 of this from 30k atoms on; fuller cells, whose bricks no longer fit the batch's
+// LDS, take up to 1.7 times as much).
+static size_t job_bytes(double slots, double atoms, double neighbours, double cells, double per_cell) {
+  const double words = 6.0 * std::min(27.0, 4.5 + std::max(per_cell, 0.0) / 3.0) + 16.0;
+  const double b =
+      slots * 500.0 + atoms * 4.0 * std::max(neighbours, 0.0) + cells * 64.0 + std::max(0.0, atoms - 32768.0) * words;
   return (size_t)b + ((size_t)16 << 20);
 }
 
-size_t xnb_job_bytes(size_t n) { return job_bytes(1.4 * (double)n, (double)n, 110.0, (double)n); }
+size_t xnb_job_bytes(size_t n) { return job_bytes(1.4 * (double)n, (double)n, 110.0, (double)n, 27.0); }
 
 size_t xnb_job_bytes_for(const xnb_job* J) {
   if (!J) return 0;
   const xnb_domain& d = J->domain;
   const double rl = J->run.rcut + J->run.rcut_inc;
   const double gl = d.cell_size > 0 ? std::max(1.0, std::ceil(rl / d.cell_size)) : 1.0;
-  double vol = 1.0, ghost = 1.0, cells = 1.0;
+  double vol = 1.0, ghost = 1.0, cells = 1.0, inner = 1.0;
   for (int a = 0; a < 3; a++) {
     const double D = std::max<double>(1.0, (double)d.grid_dims[a]);
     vol *= d.bounds_max[a] - d.bounds_min[a];
     cells *= D + 2.0 * gl;
+    inner *= D;
     if (d.periodic[a]) ghost *= (D + 2.0 * gl) / D;
   }
   const double n = (double)J->n;
   const double nb = vol > 0 ? n / vol * (4.0 / 3.0) * M_PI * rl * rl * rl : 0.0;
-  return job_bytes(n * ghost, n, nb, cells);
+  return job_bytes(n * ghost, n, nb, cells, n / inner);
 }
 
 int xnb_serve_run(const xnb_job* jobs, int njobs, const xnb_serve_config* cfg, xnb_job_result* results,
