@@ -269,7 +269,11 @@ typedef struct xnb_batch xnb_batch;
 int xnb_batch_create(xnb_batch** out, int device);
 int xnb_batch_destroy(xnb_batch* batch);
 const char* xnb_batch_error(const xnb_batch* batch);
-/* Attach an initialised box for p->steps steps; *slot identifies it in the batch. */
+/* Attach an initialised box for p->steps steps; *slot identifies it in the batch.  The box's
+ * lists are built for the batch without waiting; whoever uses them next (the batch's next step,
+ * a call on the context) waits and builds them again if they outgrew their capacity, and an
+ * error there fails the box (xnb_batch_box_status) or that call.  The context must live until
+ * its box has finished. */
 int xnb_batch_attach(xnb_batch* batch, xnb_ctx* box, const xnb_run_params* p, int* slot);
 /* Advance every unfinished box by up to nsteps steps; *n_active = unfinished boxes left. */
 int xnb_batch_step(xnb_batch* batch, int nsteps, int* n_active);
@@ -279,8 +283,9 @@ int xnb_batch_box_status(xnb_batch* batch, int slot, int64_t* done, int* state);
  * one-box operators (which re-size its arrays). */
 int xnb_batch_box_recoveries(xnb_batch* batch, int slot, int64_t* n);
 /* Steps replayed from a captured HIP graph and graphs captured so far.  A step with no box
- * starting or rebuilt on displacement is one launch sequence (rebuilds at fixed intervals,
- * ghost refresh, force, clock); quiet steps and rebuild steps each replay their own graph once
+ * starting or rebuilt on displacement is one launch sequence (rebuilds at fixed intervals, the
+ * force, which places ghosts by their sources, the ghost refresh of boxes at their last step,
+ * clock); quiet steps and rebuild steps each replay their own graph once
  * the same sequence has come twice.  XNB_BATCH_GRAPH=0 in the environment at
  * xnb_batch_create launches every step eagerly. */
 int xnb_batch_graph_stats(xnb_batch* batch, int64_t* graph_steps, int64_t* captures);
