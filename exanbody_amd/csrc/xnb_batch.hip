@@ -586,6 +586,7 @@ int settle_builds(xnb_batch* B) {
     bb.c->build_grown = false;
     if (!e) {
       BHIP(B, hipStreamSynchronize(bb.c->st));
+      BHIP(B, hipStreamSynchronize(B->st));  // attach's copy of the frame has left the staging entry
       frame_from_ctx(B, i, bb.p);
       if ((e = upload_frame(B, i))) return e;
       if (bb.c->list_kind == 1 && bb.c->bp.nbricks <= kWorkBrickMask + 1) continue;
